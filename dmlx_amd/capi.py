@@ -368,14 +368,20 @@ def gather_qmm(x, qw, rhs_indices, ws, lhs_indices=None, sorted_indices=False):
     return out
 
 
-def _c_ints(code, values):
-    """host integers as a C array ("I" u32, "i" i32): one pass in C, value by value only for what that refuses (floats, or
-    integers to be taken modulo 2^32)"""
+def _c_ints(code, values, n):
+    """n host integers as a C array ("I" u32, "i" i32): zeros behind a shorter list, IndexError for a longer one. One pass in
+    C, value by value only for what that refuses (floats, or integers to be taken modulo 2^32)"""
+    if isinstance(values, (bytes, bytearray)) or not hasattr(values, "__len__"):
+        values = list(values)
     try:
-        return array(code, list(values) if isinstance(values, (bytes, bytearray)) else values)
+        a = array(code, values)
     except (TypeError, OverflowError):
         to = C.c_uint32 if code == "I" else C.c_int32
-        return array(code, [to(int(v)).value for v in values])
+        a = array(code, [to(int(v)).value for v in values])
+    if len(a) > n:
+        raise IndexError(f"{len(a)} values where {n} belong")
+    a.extend([0] * (n - len(a)))
+    return a
 
 
 def batch_build(tokens, seq_lens, base_pos, ws, want_mask=True):
@@ -386,7 +392,7 @@ def batch_build(tokens, seq_lens, base_pos, ws, want_mask=True):
     d_pos = torch.empty(T, dtype=torch.int32, device=dev)
     d_req = torch.empty(T, dtype=torch.int32, device=dev)
     d_mask = torch.empty((T, T), dtype=torch.float32, device=dev) if want_mask else None
-    h_tok, h_len, h_base = _c_ints("I", tokens), _c_ints("i", seq_lens), _c_ints("i", base_pos)
+    h_tok, h_len, h_base = _c_ints("I", tokens, max(T, 1)), _c_ints("i", seq_lens, max(n, 1)), _c_ints("i", base_pos, max(n, 1))
     check(lib().dmoe_batch_build(_ptr(d_tok), _ptr(d_pos), _ptr(d_mask), _ptr(d_req), *(C.c_void_p(a.buffer_info()[0]) for a in (h_tok, h_len, h_base)),
                                  n, T, ws.h, _stream()))
     return d_tok, d_pos, d_mask, d_req

@@ -64,3 +64,17 @@ def test_remap_builders_reference_vectors(orc, golden):
     assert cnt == 51
     remap = capi.build_remap(mask)
     assert [remap[e] for e in np.flatnonzero(mask)] == list(range(51))
+
+
+@pytest.mark.parametrize("make", [list, tuple, iter, np.array, lambda v: [float(x) for x in v], lambda v: iter([float(x) for x in v])])
+def test_host_lists_have_the_length_the_library_reads(make):
+    """The library reads n entries of every list it is given: a shorter one is zeros from there on, a longer one is refused,
+    whatever kind of sequence it came as."""
+    for code in ("i", "I"):
+        assert capi._c_ints(code, make([5, 6, 7]), 3).tolist() == [5, 6, 7]
+        short = capi._c_ints(code, make([5]), 3)
+        assert short.tolist() == [5, 0, 0] and short.buffer_info()[1] == 3
+        with pytest.raises(IndexError):
+            capi._c_ints(code, make([5, 6, 7, 8]), 3)
+    assert capi._c_ints("I", [-1, 2 ** 32 + 3], 2).tolist() == [2 ** 32 - 1, 3]
+    assert capi._c_ints("I", bytes([4, 9]), 2).tolist() == [4, 9]

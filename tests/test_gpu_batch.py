@@ -69,6 +69,14 @@ def test_batch_build_rejects_inconsistent_requests(dmoe, ws):
         dmoe.batch_build([1, 2, 3], [4, -1], [0, 0], ws)
 
 
+def test_batch_build_base_positions_shorter_and_longer_than_the_requests(dmoe, ws):
+    """A missing base position is 0; one too many is refused."""
+    _, pos, _, _ = dmoe.batch_build([1, 2, 3], [2, 1], [5], ws)
+    assert pos.tolist() == [5, 6, 0]
+    with pytest.raises(IndexError):
+        dmoe.batch_build([1, 2, 3], [2, 1], [5, 0, 7], ws)
+
+
 @pytest.mark.parametrize("lens", [[1] * 255, [256], [257], [1] * 600, [0, 255, 0, 0, 1, 0, 256, 0], [513, 0, 1, 510], [2047, 1, 1, 1], [3]])
 def test_batch_build_block_edges(dmoe, orc, ws, lens):
     """Requests that start, end and fall empty at the edges of the 256-token blocks, and masks whose rows start on every
