@@ -182,11 +182,13 @@ __global__ void combine_kernel(uint16_t *__restrict__ out, const uint16_t *__res
 constexpr int kSkinnyAvgRows = 16;
 // Workgroups of the weight-streaming kernel up to which a launch leaves the chip half empty (one per compute unit, where two
 // fit). It is then bound by each workgroup's own chain of memory round trips, not by bandwidth: tiles are cut to one row
-// block (no restaging of the activations on the way; an expert's second tile finds the weights in L2), and in decode steps
-// of at most kPairMinRows sorted rows each tile's reduction is split over two workgroups (GemmArgs::ksplit). 8 experts
-// top-2, hidden 1024, ffn 2048, 4-bit: 16 / 32 tokens 33.4 / 41.4 -> 27.6 / 30.4 us per step; hidden 4096, 16 tokens 50.7 ->
-// 40.5 us. At twice as many workgroups it is a loss: 60 tokens with the shared expert, MXFP4, hidden 4096: 70 -> 93 us.
+// block (no restaging of the activations on the way; an expert's second tile finds the weights in L2; the sums, and so the
+// bits, are the same). 8 experts top-2, hidden 1024, ffn 2048, 4-bit: 16 / 32 tokens 39.9 / 42.1 -> 32.3 / 34.3 us per step;
+// hidden 4096: 32 tokens 62.2 -> 53.3 us; one projection [8, 1408, 2048] on 64 rows, 4-bit / MXFP4: 24.5 / 21.9 -> 19.1 / 17.7.
 constexpr int kSkinnyFewGroups = 256;
+// Sorted rows up to which each tile's reduction is also split over two workgroups (GemmArgs::ksplit). The split adds two
+// halves where the other kernels sum left to right, so it stays with single tokens: a token's bits above this line do not
+// depend on the batch it is in. (Up to 64 rows it would save 2 us of 32 on the small layer and 10 of 50 at hidden 4096.)
 constexpr int kSplitTileM = 8;
 #ifndef DMOE_PAIR_MIN_ROWS
 #define DMOE_PAIR_MIN_ROWS 64
@@ -225,7 +227,7 @@ struct FwdLayout {
     size_t h, y, sh_h, sh_y, total;
     int max_tiles, tile_m;
     bool small;
-    bool ksplit; // a handful of tiles of at most 8 rows: the weight-streaming kernel splits each tile's reduction in two
+    bool ksplit; // at most kSplitTileM sorted rows: the weight-streaming kernel splits each tile's reduction in two
     bool fold; // the shared expert rides in the routed launches: T more sorted rows behind the T*K routed ones
 };
 
@@ -253,7 +255,7 @@ static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean)
         const size_t strips = (size_t)std::max(ceil_div(L->F, 128), ceil_div(L->D, 256));
         const size_t tiles = (size_t)pack_max_tiles(n, L->E, kSplitTileM) + (f.fold ? (size_t)ceil_div(T, kSplitTileM) : 0);
         const bool few = !lean && tiles * strips <= (size_t)kSkinnyFewGroups;
-        f.ksplit = (rows <= (size_t)kSplitTileM || (few && rows <= (size_t)kPairMinRows)) &&
+        f.ksplit = rows <= (size_t)kSplitTileM &&
                    qgemm_skinny_ksplit_ok(L->gate.view) && qgemm_skinny_ksplit_ok(L->up.view) && qgemm_skinny_ksplit_ok(L->down.view) &&
                    (!f.fold || (qgemm_skinny_ksplit_ok(L->sgate.view) && qgemm_skinny_ksplit_ok(L->sup.view) &&
                                 qgemm_skinny_ksplit_ok(L->sdown.view)));
