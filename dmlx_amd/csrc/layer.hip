@@ -201,25 +201,27 @@ static bool use_small_path(size_t rows, int n_experts, const QView &b) {
     return qgemm_skinny_supports(b) && few_rows(rows, n_experts);
 }
 
-// A layer's own limit: affine formats leave the weight-streaming kernel earlier where the matrix-core launches fill the chip
-// (strips of 128 gate / up columns over all experts). us per layer_forward, 256 experts top-6, weight-streaming | prefill
+// A layer's own limit: 8-bit affine layers leave the weight-streaming kernel earlier where the matrix-core launches fill the
+// chip (strips of 128 gate / up columns over all experts). us per layer_forward, 256 experts top-6, weight-streaming | prefill
 // path:
-//  - shapes whose reduction does not cut into spans get tiles of 8 rows only, and an expert is streamed once per 8 rows.
-//    4-bit, 10.5 / 12 / 14 / 15.5 rows per expert: hidden 3072, ffn 1408: 605 / 649 / 722 / 799 | 515 / 523 / 545 / 538;
-//    hidden 1536, ffn 2048: 531 / 572 / 636 / 673 | 397 / 399 / 405 / 412. 8-bit, 8.5 / 12 / 15.5
-//    rows, hidden 4096, ffn 1408: 1193 / 1506 / 1826 | 897 / 898 / 885;
-//  - the 8-bit kernel also wins with tiles of 32 rows once there are 4096 strips: hidden 4096, ffn 2048, 350 / 509 / 620
-//    tokens 788 / 953 / 1052 | 764 / 841 / 886; hidden 2048 even 627 / 628 / 644 | 606 / 608 / 620, Zipf-skewed 334 / 370 /
-//    469 | 252 / 269 / 311. With half the strips (128 experts) it loses: 578 / 580 / 590 | 627 / 627 / 614.
-// 4-bit tiles of 32 rows stay: even routing loses 3 to 6 % at hidden 2048, for 2 % on a biased and 25 % on a skewed routing.
+//  - shapes whose reduction does not cut into spans get tiles of 8 rows only, and an expert is streamed once per 8 rows:
+//    8.5 / 12 / 15.5 rows per expert, hidden 4096, ffn 1408: 1193 / 1506 / 1826 | 897 / 898 / 885;
+//  - with tiles of 32 rows it still wins once there are 4096 strips: hidden 4096, ffn 2048, 350 / 509 / 620 tokens 788 / 953 /
+//    1052 | 764 / 841 / 886; hidden 2048 even 627 / 628 / 644 | 606 / 608 / 620, Zipf-skewed 334 / 370 / 469 | 252 / 269 /
+//    311. With half the strips (128 experts) it loses: 578 / 580 / 590 | 627 / 627 / 614.
+// Both paths multiply the same bf16 weights of an 8-bit layer in the same order: the bits do not change at the line. A 4-bit
+// layer (groups of 64 and more) stays to the general limit although its 8-row tiles lose there as well (hidden 3072, ffn 1408,
+// 12 rows per expert: 649 | 523): the weight-streaming kernel applies its scales in f32, the prefill path rounds each weight
+// to bf16 first, and a step of this size is not to have less precision than a smaller one.
 static bool layer_small_path(const Layer *L, size_t rows) {
-    const QView &gate = L->gate.view, &down = L->down.view;
+    const QView &gate = L->gate.view, &up = L->up.view, &down = L->down.view;
     if (!use_small_path(rows, L->E, gate) || !qgemm_skinny_supports(down)) return false;
-    if (gate.mode != DMOE_QUANT_AFFINE || !qgemm_wide_supports(gate) || !qgemm_wide_supports(L->up.view) || !qgemm_wide_supports(down)) return true;
+    const auto affine8 = [](const QView &b) { return b.mode == DMOE_QUANT_AFFINE && b.bits == 8 && qgemm_wide_supports(b); };
+    if (!affine8(gate) || !affine8(up) || !affine8(down)) return true;
     const int strips = L->E * ceil_div(L->F, 128);
     const bool short_tiles = std::min(qgemm_skinny_tile_m(gate), qgemm_skinny_tile_m(down)) <= kSplitTileM;
-    if (!(short_tiles && strips >= 2560) && !(gate.bits == 8 && strips >= 4096)) return true;
-    return rows <= (size_t)(gate.bits == 4 ? 10 : 8) * (size_t)L->E;
+    if (strips < (short_tiles ? 2560 : 4096)) return true;
+    return rows <= (size_t)8 * (size_t)L->E;
 }
 
 struct FwdLayout {
