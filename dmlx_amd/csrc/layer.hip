@@ -233,10 +233,13 @@ struct FwdLayout {
     bool fold; // the shared expert rides in the routed launches: T more sorted rows behind the T*K routed ones
 };
 
-// May the shared expert ride in the matrix-core launches of a prefill as dense tiles? Not in those of the fallback kernel.
+// May the shared expert ride in the matrix-core launches of a prefill as dense tiles? Not in those of the fallback kernel, and
+// not up to kSharedSkinnyRows tokens: shared_forward streams so few rows through the weight-streaming kernel, which does not
+// round 4-bit affine weights to bf16 as the matrix-core kernels do.
 // On the side stream it queued behind the small tiles' launch and ran after everything else: [1531 tokens, 256 experts
 // top-6, MXFP4] 797 -> 755 us per step, 4000 tokens 4-bit affine 1653 -> 1636, 2080 tokens 8-bit 1310 -> 1295 (same box).
-static bool fold_prefill(const Layer *L) {
+static bool fold_prefill(const Layer *L, int T) {
+    if (T <= kSharedSkinnyRows) return false;
     if (L->gate.view.mode == DMOE_QUANT_NONE) return true;
     return qgemm_wide_supports(L->gate.view) && qgemm_wide_supports(L->down.view);
 }
@@ -249,7 +252,7 @@ static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean)
     // one tile list serves both GEMMs: the smaller of their tile sizes
     f.tile_m = f.small ? std::min(qgemm_skinny_tile_m(L->gate.view), qgemm_skinny_tile_m(L->down.view))
                        : std::min(qgemm_mfma_tile_m(L->gate.view), qgemm_mfma_tile_m(L->down.view));
-    f.fold = with_shared && L->shared_folded && (f.small || (!lean && fold_prefill(L)));
+    f.fold = with_shared && L->shared_folded && (f.small || (!lean && fold_prefill(L, T)));
     const size_t rows = n + (f.fold ? (size_t)T : 0); // sorted rows of the GEMMs
     f.ksplit = false;
     if (f.small) {
