@@ -101,6 +101,26 @@ def test_static_entry_point_accepts_batches_up_to_the_array(dmoe, ws):
     layer.close()
 
 
+def test_static_entry_point_bits_near_the_limit(dmoe, ws):
+    """[8 experts top-3, hidden 512, ffn 256, shared expert]: 2695 tokens fit the 16 MiB only with the shared expert apart,
+    while a workspace takes it into the routed launches. Its last 128-row tile has 7 rows: the same kernel, the same bytes."""
+    D, F, E, K, T = 512, 256, 8, 3, 2695
+    g = torch.Generator(device="cuda").manual_seed(12)
+
+    def stack(n, rows, cols):
+        w, s, b = quantize.quantize_affine(torch.randn((n, rows, cols), generator=g, device="cuda") * 0.05, 64, 4)
+        return dmoe.QWeight(w, s, b, rows, cols, dmoe.QUANT_AFFINE, 4, 64)
+
+    layer = dmoe.Layer(D, F, K, stack(E, F, D), stack(E, F, D), stack(E, D, F), shared=(stack(1, F, D), stack(1, F, D), stack(1, D, F)))
+    x = torch.randn((T, D), generator=g, device="cuda").to(torch.bfloat16)
+    scores = torch.rand((T, E), generator=g, device="cuda")
+    got = layer.layer_forward(x, scores, None, None, True, 1.0, None)
+    want = layer.layer_forward(x, scores, None, None, True, 1.0, ws)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    layer.close()
+
+
 @pytest.mark.parametrize("config,scale,T", [(1, 0.5, 48), (4, 0.125, 200)])
 def test_static_entry_point_under_graph_capture(dmoe, ws, config, scale, T):
     """The callers this entry point is for include code under HIP graph capture: one static forward is captured
