@@ -252,7 +252,9 @@ static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean)
     // one tile list serves both GEMMs: the smaller of their tile sizes
     f.tile_m = f.small ? std::min(qgemm_skinny_tile_m(L->gate.view), qgemm_skinny_tile_m(L->down.view))
                        : std::min(qgemm_mfma_tile_m(L->gate.view), qgemm_mfma_tile_m(L->down.view));
-    f.fold = with_shared && L->shared_folded && (f.small || (!lean && fold_prefill(L, T)));
+    // (a prefill's dense tiles must leave the list within the grid limit of the paired launch, which the routed tiles alone meet)
+    const size_t prefill_tiles = n / (size_t)f.tile_m + (size_t)L->E + (size_t)ceil_div(T, f.tile_m);
+    f.fold = with_shared && L->shared_folded && (f.small || (!lean && fold_prefill(L, T) && 2 * prefill_tiles <= 65535));
     const size_t rows = n + (f.fold ? (size_t)T : 0); // sorted rows of the GEMMs
     f.ksplit = false;
     if (f.small) {
