@@ -266,6 +266,7 @@ int launch_qgemm_skinny_pair(const GemmArgs &gu, const GemmArgs &dn, hipStream_t
 int launch_qgemm_mfma(const GemmArgs &g, hipStream_t st); // picks the wide kernel when the format allows it
 int launch_qgemm_wide(const GemmArgs &g, hipStream_t st);
 // prefill sizes on MLX-layout weights whose scale rows are whole 16-byte blocks: everything through rings of LDS slots
+constexpr int kRingMaxTiles = 65528; // its grid is rounded up to whole eights
 bool qgemm_ring_supports(const QView &b);
 int launch_qgemm_ring(const GemmArgs &g, hipStream_t st);
 bool qgemm_skinny_supports(const QView &b);

@@ -363,7 +363,7 @@ struct MfmaLaunch {
 
 int launch_qgemm_mfma(const GemmArgs &g, hipStream_t st) {
     if (qgemm_wide_supports(g.b0)) return launch_qgemm_wide(g, st);
-    if (qgemm_ring_supports(g.b0) && (!g.gate_up || qgemm_ring_supports(g.b1))) return launch_qgemm_ring(g, st);
+    if (qgemm_ring_supports(g.b0) && (!g.gate_up || qgemm_ring_supports(g.b1)) && g.max_tiles <= kRingMaxTiles) return launch_qgemm_ring(g, st);
     DMOE_REQUIRE(g.tile_m > 0 && g.tile_m <= kMfmaTileM && g.tile_m % 32 == 0, "MFMA GEMM: bad tile size %d", g.tile_m);
     DMOE_REQUIRE(qgemm_mfma_supports(g.b0) && !g.b0.packed, "MFMA GEMM: unsupported weight shape (rows=%d cols=%d)",
                  g.b0.rows, g.b0.cols);

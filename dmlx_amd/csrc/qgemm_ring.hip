@@ -474,7 +474,7 @@ int launch_qgemm_ring(const GemmArgs &g, hipStream_t st) {
     DMOE_REQUIRE(qgemm_ring_supports(g.b0) && (!g.gate_up || qgemm_ring_supports(g.b1)),
                  "ring GEMM: unsupported weight format or shape (rows=%d cols=%d)", g.b0.rows, g.b0.cols);
     DMOE_REQUIRE(g.tile_m > 0 && std::min(g.tile_m, g.max_rows) <= kMfmaTileM, "ring GEMM: bad tile size %d", g.tile_m);
-    DMOE_REQUIRE(g.max_tiles >= 0 && g.max_tiles <= 65528, "ring GEMM: %d tiles exceed the grid limit", g.max_tiles);
+    DMOE_REQUIRE(g.max_tiles >= 0 && g.max_tiles <= kRingMaxTiles, "ring GEMM: %d tiles exceed the grid limit", g.max_tiles);
     DMOE_REQUIRE(g.a && g.out && g.ldo > 0 && g.ldo % 4 == 0 && ((uintptr_t)g.out % 8) == 0 && ((uintptr_t)g.a % 16) == 0,
                  "ring GEMM: bad output / activation pointer or pitch");
     if (g.gate_up)
