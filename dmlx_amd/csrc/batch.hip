@@ -5,8 +5,8 @@
 //
 // At the sizes of a serving step (a few thousand tokens) the call is bound by the host's way to the device, not by the
 // kernels (3 + 7 us at 2080 tokens). So the host lists take no copy of their own: they are laid out in a slot of pinned
-// memory, and the first kernel reads them there, over the bus, while it writes the per-token arrays. Nothing waits: a slot
-// is used again two calls later, behind an event that has passed by then. (Three copies from pageable memory and a
+// memory, and the first kernel reads them there, over the bus, while it writes the per-token arrays. A slot is used again
+// two calls later, behind an event: only a caller that is two calls ahead of the device waits for it. (Three copies from pageable memory and a
 // synchronisation before: 2080 tokens 150 us per call, of which the lists' conversion in the caller's language is not this
 // file's.)
 #include <string.h>
@@ -16,6 +16,7 @@
 namespace dmoe {
 
 constexpr int kBatchBlock = 256; // tokens per workgroup of the first kernel
+constexpr size_t kStagingTokens = 8192; // batches of up to so many tokens never allocate (128 KiB of pinned memory per slot)
 
 // Slot layout (32-bit words): first[n_blocks] = index of the non-empty request that holds the first token of each block of
 // tokens; then, per non-empty request, offset[m], base position[m], request index[m]; then tokens[T] if wanted.
@@ -72,20 +73,31 @@ __global__ __launch_bounds__(256) void batch_mask_kernel(float *__restrict__ mas
     else if (i - head < T - tail) row[tail + i - head] = value(tail + i - head);
 }
 
+static int staging_grow(StagingSlot &s, size_t words) {
+    if (s.host) DMOE_HIP(hipHostFree(s.host));
+    s.host = nullptr;
+    s.words = 0;
+    DMOE_HIP(hipHostMalloc((void **)&s.host, words * sizeof(uint32_t), hipHostMallocDefault));
+    s.words = words;
+    return DMOE_OK;
+}
+
+// Slots and events are made with the workspace, so that no call up to the size below allocates: 4 T + T / 256 words hold a
+// batch of T tokens however it is cut into requests.
+int staging_create(Workspace *w) {
+    for (StagingSlot &s : w->staging) {
+        DMOE_HIP(hipEventCreateWithFlags(&s.read, hipEventDisableTiming));
+        DMOE_TRY(staging_grow(s, 4 * kStagingTokens + kStagingTokens / kBatchBlock));
+    }
+    return DMOE_OK;
+}
+
 // the next slot of the workspace's pinned staging memory, at least `words` long and no longer read by an earlier call
 static int staging_slot(Workspace *w, size_t words, StagingSlot **out) {
     StagingSlot &s = w->staging[w->staging_next];
     w->staging_next = (w->staging_next + 1) % kStagingSlots;
-    if (!s.read) DMOE_HIP(hipEventCreateWithFlags(&s.read, hipEventDisableTiming));
-    else DMOE_HIP(hipEventSynchronize(s.read)); // passed long ago unless the caller is kStagingSlots calls ahead of the device
-    if (s.words < words) {
-        if (s.host) DMOE_HIP(hipHostFree(s.host));
-        s.host = nullptr;
-        s.words = 0;
-        const size_t want = words + words / 4 + 1024;
-        DMOE_HIP(hipHostMalloc((void **)&s.host, want * sizeof(uint32_t), hipHostMallocDefault));
-        s.words = want;
-    }
+    DMOE_HIP(hipEventSynchronize(s.read)); // passed long ago unless the caller is kStagingSlots calls ahead of the device
+    if (s.words < words) DMOE_TRY(staging_grow(s, words + words / 4));
     *out = &s;
     return DMOE_OK;
 }

@@ -104,6 +104,7 @@ int workspace_reserve(dmoe_workspace ws, size_t bytes, Workspace **out);
 void weight_cache_clear(Workspace *w);
 int weight_cache_invalidate(Workspace *w, const dmoe_qweight *qw);  // one stack's copy, or every copy (qw == null)
 int weight_cache_stats(Workspace *w, size_t *out_bytes, int *out_stacks);
+int staging_create(Workspace *w); // the slots of dmoe_batch_build, at workspace creation (batch.hip)
 void staging_clear(Workspace *w); // waits for and frees the pinned staging slots (batch.hip)
 // the current device's workspace over the static device scratch (layer.hip); resolves its address on first use
 int static_workspace(Workspace **out);

@@ -215,17 +215,16 @@ int dmoe_workspace_create(dmoe_workspace *out, size_t initial_bytes) {
         return hip_fail(e, "hipMalloc(workspace flags)");
     }
     out->ctx = w;
-    if (initial_bytes) {
-        Workspace *tmp;
-        int rc = workspace_reserve(*out, initial_bytes, &tmp);
-        if (rc != DMOE_OK) {
-            (void)hipFree(w->flags);
-            delete w;
-            out->ctx = nullptr;
-            return rc;
-        }
+    int rc = staging_create(w);
+    Workspace *tmp;
+    if (rc == DMOE_OK && initial_bytes) rc = workspace_reserve(*out, initial_bytes, &tmp);
+    if (rc != DMOE_OK) {
+        staging_clear(w);
+        (void)hipFree(w->flags);
+        delete w;
+        out->ctx = nullptr;
     }
-    return DMOE_OK;
+    return rc;
 }
 
 int dmoe_workspace_set_stage_timing(dmoe_workspace ws, int enabled) {

@@ -448,7 +448,10 @@ int dmoe_block_post(uint16_t *d_out, const uint16_t *d_ffn_out, const uint16_t *
  *                                  column <= row, -inf elsewhere (:140-177); 16-byte aligned, T <= 65535
  *   d_out_request_of_token u32 [T] request index of every token (no counterpart in the reference; the
  *                                  per-request view of a packed batch)
- * Host inputs are read before the call returns. T = sum of h_seq_lens; T == 0 is the empty batch. */
+ * Host inputs are read before the call returns. T = sum of h_seq_lens; T == 0 is the empty batch. The lists travel through
+ * two pinned slots of the workspace: a call waits only if the device has not yet run the call two before it, and only
+ * lists of more than 8192 tokens can make it allocate (host memory, once per slot and size). Not under stream capture
+ * (DMOE_ERR_INVALID): a replay would read lists of later calls. */
 int dmoe_batch_build(uint32_t *d_out_tokens, int32_t *d_out_positions, float *d_out_mask,
                      uint32_t *d_out_request_of_token, const uint32_t *h_tokens, const int32_t *h_seq_lens,
                      const int32_t *h_base_pos, int n_requests, int T, dmoe_workspace ws, dmoe_stream s);

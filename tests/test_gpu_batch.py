@@ -1,5 +1,7 @@
 """GPU parity of the device-side batch builder against the oracle's restatement of batch_builder.build:
 tokens, positions and the block-diagonal causal mask bit for bit."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -115,3 +117,28 @@ def test_batch_build_under_capture_is_refused(dmoe, ws):
             dmoe.batch_build([1, 2, 3], [2, 1], [0, 0], ws)
     tok, pos, _, _ = dmoe.batch_build([1, 2, 3], [2, 1], [0, 7], ws)
     assert tok.tolist() == [1, 2, 3] and pos.tolist() == [0, 1, 7]
+
+
+def test_batch_build_on_a_new_workspace_beside_a_capture(dmoe, ws):
+    """The first calls on a workspace allocate nothing, its two slots are made with it. Seen while another stream is being
+    captured: an allocation would be refused there and would invalidate the capture."""
+    T, x, side = 8192, torch.zeros(4, device="cuda"), torch.cuda.Stream()
+    outs = [(torch.empty(T, dtype=torch.int32, device="cuda"), torch.empty(T, dtype=torch.int32, device="cuda")) for _ in range(2)]
+    lists = [((C.c_uint32 * T)(*range(i, T + i)), (C.c_int32 * 2)(T - 1, 1), (C.c_int32 * 2)(i, 7)) for i in range(2)]
+    new = dmoe.Workspace(1 << 20)
+    torch.cuda.synchronize()
+    graph, rc = torch.cuda.CUDAGraph(), []
+    with torch.cuda.graph(graph):
+        x.add_(1)
+        for (tok, pos), (h_tok, h_len, h_base) in zip(outs, lists):
+            rc.append(dmoe.lib().dmoe_batch_build(dmoe._ptr(tok), dmoe._ptr(pos), None, None, h_tok, h_len, h_base, 2, T, new.h,
+                                                  dmoe._Handle(side.cuda_stream)))
+        x.add_(1)
+    assert rc == [0, 0]
+    graph.replay()
+    torch.cuda.synchronize()
+    assert x.tolist() == [2.0] * 4
+    for i, (tok, pos) in enumerate(outs):
+        assert torch.equal(tok.cpu(), torch.arange(i, T + i, dtype=torch.int32))
+        assert torch.equal(pos.cpu(), torch.cat([torch.arange(i, T - 1 + i), torch.tensor([7])]).int())
+    new.close()
