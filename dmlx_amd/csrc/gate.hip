@@ -30,17 +30,30 @@ constexpr int kGateTokens = 8;  // tokens per wavefront
 constexpr int kGateTokensFew = 2; // ... for batches of at most kGateFewTokens tokens: four times the wavefronts, each a quarter as long
 constexpr int kGateFewTokens = 256;
 constexpr int kGateWaves = 4;
+constexpr int kGateTeam = 8;    // wavefronts that share a tile of gate_logits_team_kernel
 
 // Which kernel forms the sums (the bits are the same). gate.forward at 4096 hidden, us, vector kernel | team kernel below:
 // 256 experts 260 / 400 / 509 / 800 / 1531 / 2080 tokens 26 / 31 / 32 / 43 / 69 / 107 | 30 / 30 / 31 / 32 / 52 / 75;
 // 64 experts 509 / 800 / 1531 / 8192 tokens 28 / 37 / 61 / 294 | 29 / 29 / 29 / 59; 8 experts 26 / 35 / 58 / 291 | 29 / 29 /
 // 29 / 36. The team kernel's time does not depend on the tokens until its tiles fill the chip, the vector kernel's does
-// (and a little on the experts): they meet at 400 tokens with 256 experts and between 560 and 590 with 8.
-static bool gate_team_pays(int T, int E) { return (size_t)T * (size_t)(512 + (E < 256 ? E : 256)) >= (size_t)400 * 768; }
+// (and a little on the experts): they meet at 400 tokens with 256 experts and between 560 and 590 with 8. Below 4096 hidden
+// they meet earlier (the line stays), above it later: 7168 hidden, 256 experts 400 / 450 tokens 47 / 55 | 50 / 50.
+// Reductions of fewer segments than the team has wavefronts leave wavefronts idle: from 640 tiles on the kernel of whole
+// reductions passes it (512 hidden, 256 experts 4096 tokens 25 us against 23, 128 hidden 21 against 15), and with a single
+// segment the vector kernel does from two tiles per compute unit on (128 hidden, 2080 tokens, 520 tiles 17 us against 15;
+// 256 / 512 hidden 18 / 20 against 22 / 31).
+static bool gate_team_pays(int T, int D, int E, size_t tiles) {
+    const int line = 400 + std::max(D - 4096, 0) / 64; // tokens, 256 experts
+    if ((size_t)T * (size_t)(512 + std::min(E, 256)) < (size_t)line * 768) return false;
+    return D > kGateSeg || tiles <= 256;
+}
 // The kernel of whole reductions per wavefront runs at the same rate without the team's hand-over, but in steps of 1024 or
-// 2048 tiles: 1024 / 1536 / 2048 tiles (256 experts) 103 / 178 / 181 | 101 / 147 / 194 us. It takes the batches whose last
-// step is at least 15/16 full.
-static bool gate_whole_pays(size_t tiles) { return tiles * 16 >= (tiles + 2047) / 2048 * 2048 * 15; }
+// 2048 tiles: 1024 / 1536 / 2048 tiles (256 experts) 103 / 178 / 181 | 101 / 147 / 194 us. It takes the batches that fill its
+// steps of 2048 tiles to at least 15/16 overall, and short reductions (see above) from 640 tiles on.
+static bool gate_whole_pays(int D, size_t tiles) {
+    if (D <= (kGateTeam - 1) * kGateSeg) return tiles >= 640;
+    return tiles * 16 >= (tiles + 2047) / 2048 * 2048 * 15;
+}
 
 struct Gate {
     int device = 0;
@@ -303,7 +316,6 @@ __global__ __launch_bounds__(kGateWaves * 64) void gate_logits_mfma_kernel(float
 // changes nothing. Team size: 8 wavefronts and two LDS buffers (64 KiB) leave room for two workgroups per compute unit.
 // Workgroup order: an XCD gets whole token blocks with all their expert tiles, so activations enter one L2 only (the
 // router's weights, 2 MiB at 256 experts, stay in all of them).
-constexpr int kGateTeam = 8;
 __global__ __launch_bounds__(kGateTeam * 64, 4) void gate_logits_team_kernel(float *__restrict__ logits,
                                                                              const uint16_t *__restrict__ x,
                                                                              const uint4 *__restrict__ wgp, int T, int D, int E) {
@@ -668,8 +680,8 @@ int dmoe_gate_forward(uint32_t *d_out_indices, float *d_out_weights, float *d_ou
     // 32-token x 32-expert tiles: the matrix-core kernels (whole sums); of the one without hand-over two tiles per wavefront
     // once there are more than two wavefronts per SIMD
     const size_t mfma_tiles = (size_t)ceil_div(T, 32) * ceil_div(G->E, 32);
-    const bool mfma = gate_whole_pays(mfma_tiles);
-    const bool team = !mfma && gate_team_pays(T, G->E);
+    const bool mfma = gate_whole_pays(G->D, mfma_tiles);
+    const bool team = !mfma && gate_team_pays(T, G->D, G->E, mfma_tiles);
     const int mfma_nb = mfma_tiles > 2048 ? 2 : 1;
     const bool split = groups > 1 && !mfma && !team;
     const int n_out_seg = split ? n_seg : 1;

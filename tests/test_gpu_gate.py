@@ -56,7 +56,14 @@ def test_gate_forward_bit_exact(dmoe, orc, ws, func, T, D, E, K, with_bias, with
     (400, 1160, 256, 6),     # the fewest tokens the team kernel takes; two rounds of segments, the second partial, its last segment short
     (604, 128, 8, 2),        # one segment: seven of the eight wavefronts idle, three quarters of the tile past E
     (777, 2048, 33, 4),      # two full rounds, a second expert block of one expert
-    (2049, 72, 250, 5),      # a short segment only, a token block of one token
+    (2049, 72, 250, 5),      # a short segment only, more than one tile per compute unit: the vector kernel
+    (993, 72, 250, 5),       # the same on 256 tiles: the team kernel, a token block of one token
+    (2529, 200, 256, 6),     # two segments on 640 tiles: the kernel of whole reductions
+    (2528, 200, 256, 6),     # the team
+    (2529, 896, 250, 6),     # seven segments on 640 tiles
+    (2529, 904, 250, 6),     # eight segments: the team
+    (447, 7168, 256, 6),     # one token below the line of long reductions
+    (448, 7168, 256, 6),
     (590, 3080, 8, 2),       # one token below the line: the vector kernel
     (12500, 392, 300, 6),    # two full steps of the kernel with two expert blocks per wavefront
 ])
