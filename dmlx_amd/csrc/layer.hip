@@ -240,8 +240,10 @@ struct FwdLayout {
 // top-6, MXFP4] 797 -> 755 us per step, 4000 tokens 4-bit affine 1653 -> 1636, 2080 tokens 8-bit 1310 -> 1295 (same box).
 static bool fold_prefill(const Layer *L, int T) {
     if (T <= kSharedSkinnyRows) return false;
-    if (L->gate.view.mode == DMOE_QUANT_NONE) return true;
-    return qgemm_wide_supports(L->gate.view) && qgemm_wide_supports(L->down.view);
+    if (L->gate.view.mode != DMOE_QUANT_NONE) return qgemm_wide_supports(L->gate.view) && qgemm_wide_supports(L->down.view);
+    // unquantized: run_gemm's choice for the routed rows (few of them per expert, on rows too long for the weight-streaming
+    // kernel, take the fallback; hidden 12288, 64 experts top-2, 65 / 400 tokens 520 / 639 us apart, 696 / 903 in its launches)
+    return !few_rows((size_t)T * L->K, L->E) && qgemm_wide_bf16_supports(L->gate.view) && qgemm_wide_bf16_supports(L->down.view);
 }
 
 static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean) {
