@@ -204,11 +204,15 @@ static bool use_small_path(size_t rows, int n_experts, const QView &b) {
 // A layer's own limit: 8-bit affine layers leave the weight-streaming kernel earlier where the matrix-core launches fill the
 // chip (strips of 128 gate / up columns over all experts). us per layer_forward, 256 experts top-6, weight-streaming | prefill
 // path:
-//  - shapes whose reduction does not cut into spans get tiles of 8 rows only, and an expert is streamed once per 8 rows:
-//    8.5 / 12 / 15.5 rows per expert, hidden 4096, ffn 1408: 1193 / 1506 / 1826 | 897 / 898 / 885;
-//  - with tiles of 32 rows it still wins once there are 4096 strips: hidden 4096, ffn 2048, 350 / 509 / 620 tokens 788 / 953 /
-//    1052 | 764 / 841 / 886; hidden 2048 even 627 / 628 / 644 | 606 / 608 / 620, Zipf-skewed 334 / 370 / 469 | 252 / 269 /
-//    311. With half the strips (128 experts) it loses: 578 / 580 / 590 | 627 / 627 / 614.
+//  - shapes whose reduction does not cut into spans get tiles of 8 rows only, and an expert is streamed once per 8 rows: from
+//    8 rows per expert and 2560 strips on. 8.5 / 12 / 15.5 rows, hidden 4096, ffn 1408: 1193 / 1506 / 1826 | 897 / 898 / 885;
+//    8.2 / 16 rows at 2560 strips: ffn 1280 777 / 1223 | 571 / 598, 512 experts with ffn 640 600 / 899 | 412 / 445;
+//  - tiles of 16 rows from 4096 strips on: hidden 1536, ffn 2048 549 / 753 | 460 / 490, 512 experts with ffn 1024 496 / 670 |
+//    471 / 506;
+//  - tiles of 32 rows from 12 rows per expert on, ffn of 2048 and more: 12 / 16 rows, hidden 4096, ffn 2048 1175 / 1267 | 1179 /
+//    1168, Zipf-skewed 664 / 803 | 529 / 595; hidden 2048, ffn 3072 924 / 947 | 902 / 897; hidden 1024, ffn 2048 445 / 486 | 343
+//    / 332. At 8 rows per expert some of them still lose (hidden 2048, ffn 3072: 815 | 880), and so do narrower experts up to
+//    13 (512 of them, ffn 1024: 549 / 605 | 604 / 617) and fewer strips (128 experts, ffn 2048: 578 | 627).
 // Both paths multiply the same bf16 weights of an 8-bit layer in the same order: the bits do not change at the line. A 4-bit
 // layer (groups of 64 and more) stays to the general limit although its 8-row tiles lose there as well (hidden 3072, ffn 1408,
 // 12 rows per expert: 649 | 523): the weight-streaming kernel applies its scales in f32, the prefill path rounds each weight
@@ -218,10 +222,9 @@ static bool layer_small_path(const Layer *L, size_t rows) {
     if (!use_small_path(rows, L->E, gate) || !qgemm_skinny_supports(down)) return false;
     const auto affine8 = [](const QView &b) { return b.mode == DMOE_QUANT_AFFINE && b.bits == 8 && qgemm_wide_supports(b); };
     if (!affine8(gate) || !affine8(up) || !affine8(down)) return true;
-    const int strips = L->E * ceil_div(L->F, 128);
-    const bool short_tiles = std::min(qgemm_skinny_tile_m(gate), qgemm_skinny_tile_m(down)) <= kSplitTileM;
-    if (strips < (short_tiles ? 2560 : 4096)) return true;
-    return rows <= (size_t)8 * (size_t)L->E;
+    const int strips = L->E * ceil_div(L->F, 128), tile = std::min(qgemm_skinny_tile_m(gate), qgemm_skinny_tile_m(down));
+    if (strips < (tile <= 8 ? 2560 : 4096) || (tile == 32 && L->F < 2048)) return true;
+    return rows <= (size_t)(tile <= 16 ? 8 : 12) * (size_t)L->E;
 }
 
 struct FwdLayout {
