@@ -236,17 +236,49 @@ struct FwdLayout {
     bool fold; // the shared expert rides in the routed launches: T more sorted rows behind the T*K routed ones
 };
 
-// May the shared expert ride in the matrix-core launches of a prefill as dense tiles? Not in those of the fallback kernel, and
+// Prefill-sized calls: the matrix-core kernel takes the tiles above `small_rows` rows, and the weight-streaming kernel
+// the rest of the same list right behind it (a tile of a few rows is bound by reading its expert's weights, and the
+// large-tile kernel spends a whole pass of its LDS pipeline on it). small_rows = 0: everything on the matrix-core kernel.
+constexpr int kPrefillSmallRows = 8;
+static int prefill_small_rows(const QView &b0, const QView &b1) {
+    if (!qgemm_skinny_supports(b0) || !qgemm_skinny_supports(b1)) return 0;
+    // measured: pays with the kernel of the packed 4-bit formats (8k-token ragged prefill: gate/up 1.757 -> 1.715 ms, down
+    // unchanged), not with the 8-bit kernel (2080-token mixed batch: +1 %)
+    if (!qgemm_wide_supports(b0) || !qgemm_wide_supports(b1)) return 0;
+    const auto four_bit = [](const QView &b) { return b.mode == DMOE_QUANT_MXFP4 || (b.mode == DMOE_QUANT_AFFINE && b.bits == 4); };
+    if (!four_bit(b0) || !four_bit(b1)) return 0;
+    // threshold measured on the same prefill: 8 rows 2.62 ms, 16 rows 2.63, 32 rows 2.64, 4 rows 2.67, no split 2.70
+    return std::min(kPrefillSmallRows, std::min(qgemm_skinny_tile_m(b0), qgemm_skinny_tile_m(b1)));
+}
+
+// May the shared expert ride in the matrix-core launches of a prefill as dense tiles? Not in those of the fallback kernels, and
 // not up to kSharedSkinnyRows tokens: shared_forward streams so few rows through the weight-streaming kernel, which does not
-// round 4-bit affine weights to bf16 as the matrix-core kernels do.
-// On the side stream it queued behind the small tiles' launch and ran after everything else: [1531 tokens, 256 experts
-// top-6, MXFP4] 797 -> 755 us per step, 4000 tokens 4-bit affine 1653 -> 1636, 2080 tokens 8-bit 1310 -> 1295 (same box).
+// round 4-bit affine weights to bf16 as the matrix-core kernels do. Where it may (the bits are the same), us per step apart | in
+// the routed launches, or their ratio:
+//  - with a launch for the small tiles, the shared expert on the side stream queued behind that and ran after everything else.
+//    256 experts top-6, MXFP4, 1531 tokens 797 | 755; 64 experts top-6, 4-bit, hidden 2048, ffn 1408, 230 / 1200
+//    tokens 0.70 / 0.86, 8 experts top-2, hidden 4096, 66 / 500 / 1200 tokens 0.62 / 0.68 / 0.88. With many rows per expert
+//    few experts have a small tile and the dense tiles only lengthen the launches: 8 experts top-2, 1450 tokens (362 rows per
+//    expert) 1.09, 3000 tokens 1.07, 32 experts top-4, 1531 tokens (191 rows) 1.03;
+//  - without one (8-bit, unquantized), while everything is one round of workgroups, one per compute unit, it saves two launches
+//    beside the others: 8 experts top-2, hidden 4096, 66 / 500 tokens 0.77 / 0.75 (8-bit), 0.69 / 0.75 (bf16). With more, what
+//    the dense tiles add can be a second round: 8 experts top-4, 8-bit, 380 / 760 tokens 1.08 / 1.09. Over many rounds it
+//    pays for bf16 weights, 0.91 to 0.96 from 1024 workgroups on; 8-bit layers are level.
 static bool fold_prefill(const Layer *L, int T) {
     if (T <= kSharedSkinnyRows) return false;
-    if (L->gate.view.mode != DMOE_QUANT_NONE) return qgemm_wide_supports(L->gate.view) && qgemm_wide_supports(L->down.view);
-    // unquantized: run_gemm's choice for the routed rows (few of them per expert, on rows too long for the weight-streaming
-    // kernel, take the fallback; hidden 12288, 64 experts top-2, 65 / 400 tokens 520 / 639 us apart, 696 / 903 in its launches)
-    return !few_rows((size_t)T * L->K, L->E) && qgemm_wide_bf16_supports(L->gate.view) && qgemm_wide_bf16_supports(L->down.view);
+    const QView &gate = L->gate.view, &down = L->down.view;
+    const size_t n = (size_t)T * L->K, E = (size_t)L->E;
+    const bool bf16 = gate.mode == DMOE_QUANT_NONE;
+    // (unquantized: run_gemm's choice for the routed rows; few of them per expert, on rows too long for the weight-streaming
+    // kernel, take the fallback: hidden 12288, 64 experts top-2, 65 / 400 tokens 520 / 639 | 696 / 903)
+    if (bf16 ? few_rows(n, L->E) || !qgemm_wide_bf16_supports(gate) || !qgemm_wide_bf16_supports(down)
+             : !qgemm_wide_supports(gate) || !qgemm_wide_supports(down))
+        return false;
+    if (prefill_small_rows(gate, down) > 0) return n < (T < 1500 ? 320 : 176) * E;
+    // workgroups of the larger launch, if the routing is even
+    const size_t strips = (size_t)std::max(ceil_div(L->F, 128), ceil_div(L->D, 256));
+    const size_t routed = (n < E ? n : E * ((n + E * kMfmaTileM - 1) / (E * kMfmaTileM))) * strips;
+    return routed + (size_t)ceil_div(T, kMfmaTileM) * strips <= 256 || (bf16 && routed >= 1024);
 }
 
 static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean) {
@@ -310,20 +342,6 @@ static FwdLayout forward_layout(const Layer *L, int T, bool with_shared = true, 
     return f;
 }
 
-// Prefill-sized calls: the matrix-core kernel takes the tiles above `small_rows` rows, and the weight-streaming kernel
-// the rest of the same list right behind it (a tile of a few rows is bound by reading its expert's weights, and the
-// large-tile kernel spends a whole pass of its LDS pipeline on it). small_rows = 0: everything on the matrix-core kernel.
-constexpr int kPrefillSmallRows = 8;
-static int prefill_small_rows(const QView &b0, const QView &b1) {
-    if (!qgemm_skinny_supports(b0) || !qgemm_skinny_supports(b1)) return 0;
-    // measured: pays with the kernel of the packed 4-bit formats (8k-token ragged prefill: gate/up 1.757 -> 1.715 ms, down
-    // unchanged), not with the 8-bit kernel (2080-token mixed batch: +1 %)
-    if (!qgemm_wide_supports(b0) || !qgemm_wide_supports(b1)) return 0;
-    const auto four_bit = [](const QView &b) { return b.mode == DMOE_QUANT_MXFP4 || (b.mode == DMOE_QUANT_AFFINE && b.bits == 4); };
-    if (!four_bit(b0) || !four_bit(b1)) return 0;
-    // threshold measured on the same prefill: 8 rows 2.62 ms, 16 rows 2.63, 32 rows 2.64, 4 rows 2.67, no split 2.70
-    return std::min(kPrefillSmallRows, std::min(qgemm_skinny_tile_m(b0), qgemm_skinny_tile_m(b1)));
-}
 // `few` = few rows per expert (only read for unquantized weights; the quantized formats have `small`)
 static int run_gemm(const GemmArgs &g, bool small, hipStream_t st, int small_rows = 0, bool few = false) {
     if (g.b0.mode == DMOE_QUANT_NONE) {

@@ -102,9 +102,9 @@ def test_static_entry_point_accepts_batches_up_to_the_array(dmoe, ws):
 
 
 def test_static_entry_point_bits_near_the_limit(dmoe, ws):
-    """[8 experts top-3, hidden 512, ffn 256, shared expert]: 2695 tokens fit the 16 MiB only with the shared expert apart,
-    while a workspace takes it into the routed launches. Its last 128-row tile has 7 rows: the same kernel, the same bytes."""
-    D, F, E, K, T = 512, 256, 8, 3, 2695
+    """[64 experts top-3, hidden 512, ffn 256, shared expert]: 2694 tokens fit the 16 MiB only with the shared expert apart,
+    while a workspace takes it into the routed launches. Its last 128-row tile has 6 rows: the same kernel, the same bytes."""
+    D, F, E, K, T = 512, 256, 64, 3, 2694
     g = torch.Generator(device="cuda").manual_seed(12)
 
     def stack(n, rows, cols):
