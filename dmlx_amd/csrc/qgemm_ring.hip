@@ -1,5 +1,6 @@
-// Grouped quantized GEMM, ring path: prefill-sized calls on weights in the MLX layout (the caller's own arrays), every
-// quantized format, tiles of up to 128 rows of one expert segment.
+// Grouped quantized GEMM, ring path: prefill-sized calls on weights in the MLX layout, every quantized format, tiles of up to
+// 128 rows of one expert segment. That is dmoe_gather_qmm on the caller's own arrays, and the gate / up launch of a layer whose
+// ffn is no multiple of 32 (such stacks are not re-ordered; their down projection is then an unquantized one).
 //
 // What bounds such a call on these arrays is how the weights are fetched. Operand-layout loads (qgemm_mfma.hip) take 32
 // bytes out of each of 64 rows, and one 2-byte scale and bias per row and step: every 128-byte line is touched four times
@@ -54,14 +55,13 @@ struct RingGeom {
     static constexpr int MBLK = !META ? 0 : BIAS ? 2048 : 1024; // a block of scale (and bias) entries, per wavefront
     static constexpr int fit() {
         const int left = (int)kRingLdsBytes - kRingWaves * 2 * MBLK;
-        const int r = left / (ACT + kRingWaves * WB);
-        return r > 6 ? 6 : r;
+        return left / (ACT + kRingWaves * WB); // 8-bit: 3 slots at MT = 1, else 2; FP8: 4, 3, 2, 2
     }
     static constexpr int RW = PAIRS ? (MT == 1 ? 3 : 2) : fit();            // weight slots
     static constexpr int RA = PAIRS ? (MT <= 2 ? 4 : 2) : fit();            // activation slots
     static constexpr int W_OFF = RA * ACT, M_OFF = W_OFF + kRingWaves * RW * WB;
     static constexpr int TOTAL = M_OFF + kRingWaves * 2 * MBLK;
-    static_assert(RA >= 2 && RW >= 2 && TOTAL <= (int)kRingLdsBytes, "the ring does not fit");
+    static_assert(RA >= 2 && RA <= 4 && RW >= 2 && TOTAL <= (int)kRingLdsBytes, "the ring does not fit, or holds more groups than the waits below tell apart");
     static constexpr int NW = 4;                                // weight requests of a slot
 };
 
@@ -305,8 +305,6 @@ __device__ __forceinline__ void ring_tile(const GemmArgs &g, const Tile &t, uint
                         } else {
                             const int young = n_steps - 2 - s; // groups behind s + 1 that exist
                             if (young >= RA - 2) __builtin_amdgcn_s_waitcnt(ring_wait_both((RA - 2) * NOPS));
-                            else if (RA > 5 && young >= 3) __builtin_amdgcn_s_waitcnt(ring_wait_both(3 * NOPS));
-                            else if (RA > 4 && young >= 2) __builtin_amdgcn_s_waitcnt(ring_wait_both(2 * NOPS));
                             else if (RA > 3 && young >= 1) __builtin_amdgcn_s_waitcnt(ring_wait_both(NOPS));
                             else __builtin_amdgcn_s_waitcnt(ring_wait_both(0));
                         }
