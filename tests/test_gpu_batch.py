@@ -93,9 +93,14 @@ def test_batch_build_block_edges(dmoe, orc, ws, lens):
 
 
 def test_batch_build_calls_in_flight_do_not_share_lists(dmoe, orc, ws):
-    """Calls of growing and shrinking size enqueued without a wait between them: each reads its own lists."""
+    """Calls of equal, growing and shrinking size enqueued behind some tens of milliseconds of other work: each reads its own
+    lists, although none of their kernels has run when the later calls are made."""
     cases, got = [], []
-    for i, n in enumerate((700, 40, 3000, 3000, 9, 5000, 300)):
+    busy = torch.ones((8192, 8192), dtype=torch.bfloat16, device="cuda")
+    dmoe.batch_build([1], [1], [0], ws)
+    for _ in range(40):
+        busy @ busy
+    for i, n in enumerate((700, 700, 700, 700, 40, 3000, 3000, 9, 9000, 300)):
         lens = [n // 2, 0, n - n // 2 - 1, 1]
         cases.append((lens, *_requests(100 + i, lens)))
     for lens, toks, base in cases:
