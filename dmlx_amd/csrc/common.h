@@ -220,7 +220,6 @@ size_t qweight_w_bytes(const dmoe_qweight *q);
 size_t qweight_s_bytes(const dmoe_qweight *q);
 size_t qweight_b_bytes(const dmoe_qweight *q);
 
-constexpr int kAllRows = 0x7fffffff;
 struct GemmArgs {
     QView b0, b1;                 // b1 = up projection when gate_up
     bool gate_up = false;         // out[p, f] = swiglu(x.b0[f], x.b1[f]) instead of x.b0[n]
@@ -238,9 +237,8 @@ struct GemmArgs {
     int dense_rows = 0;
     float swiglu_limit = 0.0f;
     // a launch serves the tiles with min_rows <= nrows <= max_rows of the list (prefill: the matrix-core kernels take the
-    // large tiles, the weight-streaming kernel the small ones). Tiles flagged kTileDense go to the former at any size: which
-    // kernel computes the shared expert's last rows, and so their bits, does not depend on whether it rides in the list.
-    int min_rows = 0, max_rows = kAllRows;
+    // large tiles, the weight-streaming kernel the small ones)
+    int min_rows = 0, max_rows = 0x7fffffff;
     // weight-streaming kernel, launches of a handful of tiles: the reduction of a tile split over two groups of
     // wavefronts (see qgemm_skinny_ksplit_ok: packed layout, tiles of at most 8 rows)
     int ksplit = 0;

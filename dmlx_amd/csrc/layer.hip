@@ -253,7 +253,9 @@ static int prefill_small_rows(const QView &b0, const QView &b1) {
 
 // May the shared expert ride in the matrix-core launches of a prefill as dense tiles? Not in those of the fallback kernels, and
 // not up to kSharedSkinnyRows tokens: shared_forward streams so few rows through the weight-streaming kernel, which does not
-// round 4-bit affine weights to bf16 as the matrix-core kernels do. Where it may (the bits are the same), us per step apart | in
+// round 4-bit affine weights to bf16 as the matrix-core kernels do. For the same reason not with a last tile of so few rows that
+// it would count as a small one: the bits must not depend on whether the shared expert rides along (a mark on such tiles,
+// tested by the kernels, cost small decode steps 0.2 to 0.9 us of 33). Where it may (the bits are the same), us per step apart | in
 // the routed launches, or their ratio:
 //  - with a launch for the small tiles, the shared expert on the side stream queued behind that and ran after everything else.
 //    256 experts top-6, MXFP4, 1531 tokens 797 | 755; 64 experts top-6, 4-bit, hidden 2048, ffn 1408, 230 / 1200
@@ -274,7 +276,8 @@ static bool fold_prefill(const Layer *L, int T) {
     if (bf16 ? few_rows(n, L->E) || !qgemm_wide_bf16_supports(gate) || !qgemm_wide_bf16_supports(down)
              : !qgemm_wide_supports(gate) || !qgemm_wide_supports(down))
         return false;
-    if (prefill_small_rows(gate, down) > 0) return n < (T < 1500 ? 320 : 176) * E;
+    const int small_rows = prefill_small_rows(gate, down), last = (T - 1) % kMfmaTileM + 1;
+    if (small_rows > 0) return last > small_rows && n < (T < 1500 ? 320 : 176) * E;
     // workgroups of the larger launch, if the routing is even
     const size_t strips = (size_t)std::max(ceil_div(L->F, 128), ceil_div(L->D, 256));
     const size_t routed = (n < E ? n : E * ((n + E * kMfmaTileM - 1) / (E * kMfmaTileM))) * strips;

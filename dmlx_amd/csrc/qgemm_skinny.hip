@@ -621,8 +621,7 @@ __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(Gem
         const uint32_t n_tiles = *g.n_tiles; // both loads are issued before either is needed
         t = g.tiles[slot];                   // the list has room for every launched slot
         if (slot >= n_tiles) return;
-        // a list shared with the matrix-core kernel: that takes the larger tiles, and the folded shared expert's whatever their size
-        if ((int)t.nrows > g.max_rows || ((t.flags & kTileDense) && g.max_rows != kAllRows)) return;
+        if ((int)t.nrows > g.max_rows) return; // a list built for the matrix-core kernels: those take the larger tiles
     } else {
         t.expert = 0;
         t.flags = 0;

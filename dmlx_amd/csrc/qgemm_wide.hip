@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kWideWaves * 64, 2) void qgemm_wide_kernel(GemmArgs
         const uint32_t n_tiles = *g.n_tiles;
         t = g.tiles[slot < (uint32_t)g.max_tiles ? slot : 0u];
         if (slot >= n_tiles) return;
-        if ((int)t.nrows < g.min_rows && !(t.flags & kTileDense)) return; // left to the weight-streaming kernel
+        if ((int)t.nrows < g.min_rows) return; // left to the weight-streaming kernel
     } else {
         t.expert = 0;
         t.flags = 0;
