@@ -23,8 +23,8 @@ struct Layer {
     int D = 0, F = 0, K = 0, E = 0, Fs = 0;
     QOwned gate, up, down, sgate, sup, sdown;
     bool has_shared = false;
-    // the shared expert's packed weights also sit behind the routed experts' as matrix E of the same buffers: at
-    // decode sizes it then rides in the routed launches as an always-on expert (no side stream, no fork / join)
+    // the shared expert's packed weights also sit behind the routed experts' as matrix E of the same buffers: it can then ride
+    // in the routed launches as an always-on expert (no side stream, no fork / join): FwdLayout::fold
     bool shared_folded = false;
     float swiglu_limit = 0.0f, shared_swiglu_limit = 0.0f;
     bool score_before_down = false;
