@@ -26,9 +26,10 @@ namespace dmoe {
 
 // E8M0 shared exponent -> 2^(s-127); 255 is NaN
 __device__ __forceinline__ float e8m0_to_f32(uint32_t s) {
-    if (s == 255u) return __uint_as_float(0x7fc00000u);
-    if (s == 0u) return __uint_as_float(0x00400000u); // 2^-127, an f32 subnormal
-    return __uint_as_float(s << 23);
+    uint32_t bits = s << 23;
+    bits = s == 0u ? 0x00400000u : bits; // 2^-127, an f32 subnormal
+    bits = s == 255u ? 0x7fc00000u : bits;
+    return __uint_as_float(bits);
 }
 
 // E2M1 code (sign in bit 3) -> f32: 0, .5, 1, 1.5, 2, 3, 4, 6

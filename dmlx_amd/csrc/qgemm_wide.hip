@@ -18,14 +18,23 @@
 //    the second, so the MFMA operand reads (32 rows at the same reduction offset) run at the full 256 bytes per
 //    cycle (position piece ^ (r & 7) made rows r and r + 8 collide: 155 bytes per cycle measured). The swizzle
 //    costs nothing because each lane picks its global source address freely.
-//  * Four LDS buffers of one reduction step each (4 x 16 KiB): while step s computes, the loads of step s+2
-//    are in flight. The compiler does not know about these loads (they are issued from inline assembly), so
-//    their completion is tracked by hand: VMEM operations return in order, hence "at most MT operations
-//    outstanding" three quarters into step s implies that everything issued before this step's own MT loads
-//    -- in particular the loads of step s+1 -- has landed. One s_barrier per step then publishes the buffer.
-//  * The same in-order rule means a deep register ring of weight loads buys nothing (any wait for a staging request
-//    also waits for every older weight load), so the weights of only two steps are in flight, which is what
-//    keeps the wavefront under 256 registers.
+//  * A ring of LDS buffers of one reduction step each: while step s computes, the loads of the next steps are in flight.
+//    The compiler does not know about these loads (they are issued from inline assembly), so their completion is
+//    tracked by hand: VMEM operations return in order, hence "at most N operations outstanding" three quarters into
+//    step s, with N = what has been issued since the loads of step s + 1, implies that these have landed. One s_barrier
+//    per step then publishes the buffer.
+//  * The same in-order rule ties the two streams together: a wait for a weight chunk also waits for every older staging
+//    request and the other way round, so that only looking ahead further with BOTH helps. Tiles of at most 64 rows have
+//    the room (64 or 96 accumulator registers less, LDS buffers of 4 or 8 KiB instead of 16) and need it: a step of theirs
+//    is 8 or 16 matrix instructions long, a memory round trip as long as several steps, and their expert's weights come
+//    from HBM (such a tile is nearly always its expert's only one), so their weight loads carry the streaming hint, too.
+//    Eight buffers (six blocks ahead), eight (4-bit) or four (8-bit) steps of weights. Tiles of more rows keep two steps
+//    of weights and four buffers, which is what stays under 256 registers. 256 experts, one projection [2048, 4096], with
+//    32 / 64 rows each, four buffers and two steps for all tiles -> this: 4-bit affine 312 / 354 -> 264 / 332 us, MXFP4
+//    234 / 279 -> 210 / 276, 8-bit 431 / 451 -> 385 / 425, bf16 773 / 778 -> 708 / 727.
+//  * Rows past the end of a tile are zeros in LDS and never requested: the chip is power-limited here, and multiplying
+//    zeros costs less of it than multiplying copies of a row (33 rows per expert: MXFP4 263 -> 251 us, 4-bit affine 324 ->
+//    311, 65 and 97 rows 1 to 3 %).
 //  * Activation fragments are single-buffered (except for tiles of at most 64 rows): the fragment of row tile mt
 //    is reloaded for the next MFMA group right after its last use in this one, 2*MT-1 units before it is needed
 //    again.
@@ -41,14 +50,35 @@
 namespace dmoe {
 
 constexpr int kWideWaves = 4;
-constexpr int kWideRing = 4;                              // LDS activation buffers = steps per unrolled trip
-constexpr int kWideWRing = 2;                             // weight steps held in registers (see the header)
-constexpr int kWideBufBytes = kMfmaWideTileM * 128;       // one reduction step (64 bf16) of every row of the tile
-constexpr size_t kWideLdsBytes = (size_t)kWideRing * kWideBufBytes;
+constexpr size_t kWideLdsBytes = 65536;   // two workgroups per compute unit
+
+// Pipeline depths of a tile of MT row blocks of 32.
+template <typename Fmt, int MT>
+struct WidePipe {
+    static constexpr int kSlots = MT <= 2 ? 8 : 4;  // LDS activation buffers = steps per unrolled trip
+    static constexpr int kAhead = kSlots - 2;       // blocks of activations in flight ahead of the one being computed
+    // the loop runs whole trips (surplus steps multiply zeros), or ends behind the last step
+    // (leaving in mid-trip costs the larger tiles the registers they do not have)
+    static constexpr bool kWholeTrips = MT > 2;
+    static constexpr bool kStream = MT <= 2; // weight loads with the streaming hint
+    // steps of weights held in registers
+    static constexpr int kWeights = Fmt::kVals == 32 ? (MT <= 2 ? 8 : 2) : Fmt::kVals == 16 ? (MT <= 2 ? 4 : 2) : (MT == 1 ? 4 : MT == 2 ? 2 : 1);
+};
 
 // s_waitcnt immediates (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14])
 constexpr int wait_vmcnt(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int wait_vmcnt_lgkm0(int n) { return 0x0070 | (n & 15) | ((n >> 4) << 14); }
+// the same for a count that is a constant only once the loops around it are unrolled
+__device__ __forceinline__ void wait_vmcnt_at_most(int n) {
+#define DMOE_WAIT(N) case N: __builtin_amdgcn_s_waitcnt(wait_vmcnt(N)); break;
+#define DMOE_WAIT8(N) DMOE_WAIT(N) DMOE_WAIT(N + 1) DMOE_WAIT(N + 2) DMOE_WAIT(N + 3) DMOE_WAIT(N + 4) DMOE_WAIT(N + 5) DMOE_WAIT(N + 6) DMOE_WAIT(N + 7)
+    switch (n) {
+        DMOE_WAIT8(0) DMOE_WAIT8(8) DMOE_WAIT8(16) DMOE_WAIT8(24) DMOE_WAIT8(32) DMOE_WAIT8(40) DMOE_WAIT8(48) DMOE_WAIT8(56)
+    default: __builtin_amdgcn_s_waitcnt(wait_vmcnt(63)); // the counter's largest value
+    }
+#undef DMOE_WAIT8
+#undef DMOE_WAIT
+}
 constexpr int kWaitLgkm0 = 0xc07f;
 
 template <typename Fmt, bool GATE_UP, int MT>
@@ -63,15 +93,16 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
     constexpr int NJC = NJ / CH;          // MFMA groups per chunk step
     constexpr int NUC = NJC * MT * NT;    // units (MFMAs) per chunk step
     constexpr int NPC = NT * (KV / 2);    // packed pairs to decode per chunk step
-    // chunk steps held in registers (twice as many for tiles of at most 64 rows moved the 8-bit mixed batch by nothing)
-    // (unquantized weights: four chunk steps per step, so one step's worth keeps the ring at the 8-bit formats' size)
-    constexpr int WRC = CH == 4 ? CH : kWideWRing * CH;
-    static_assert(kWideRing % kWideWRing == 0 && (kWideRing * CH) % WRC == 0, "ring slots must line up across trips");
+    using P = WidePipe<Fmt, MT>;
+    constexpr int SLOTS = P::kSlots, AHEAD = P::kAhead, WR = P::kWeights, WRC = WR * CH; // (WRC: chunk steps held in registers)
+    constexpr bool WHOLE = P::kWholeTrips;
+    constexpr int BUF = MT * 4096; // one LDS slot: one reduction step (64 bf16) of every row of the tile
+    static_assert(SLOTS % WR == 0 && (SLOTS * CH) % 2 == 0, "ring slots must line up across trips");
+    static_assert(SLOTS * BUF <= (int)kWideLdsBytes && SLOTS == AHEAD + 2, "a slot is refilled two barriers after its last read");
     const int tid = (int)threadIdx.x, lane = tid & 63, ln = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cols = g.b0.cols, n_out = g.b0.rows;
     const int n_steps = cols / KSTEP, n_csteps = n_steps * CH;
-    const int n_trips = (n_steps + kWideRing - 1) / kWideRing;
     const size_t e = t.expert;
 
     // ---- this wavefront's weight rows (gate_up: tile 0 = gate, tile 1 = up rows of the same 32 columns) ----
@@ -93,38 +124,59 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             const QView &b = (GATE_UP && nt == 1) ? g.b1 : g.b0;
-            ring_raw[slot_][nt] = cs[nt].load_chunk(cstep);
+            ring_raw[slot_][nt] = P::kStream ? cs[nt].load_chunk_stream(cstep) : cs[nt].load_chunk(cstep);
             cs[nt].load_meta(b, cstep, ring_sb[slot_][nt]);
         }
     };
-#pragma unroll
-    for (int j = 0; j < WRC; ++j) load_b(j < n_csteps ? j : n_csteps - 1, j);
 
     // ---- activation staging -------------------------------------------------------------------------------
     // operation i of this wavefront moves rows (wave + 4 i) * 8 .. + 7; lane = (row r8 of the eight, position c),
-    // and fetches piece c ^ ((row >> 1) & 7) of its row. Rows past the segment end alias the tile's first row (never
-    // stored).
+    // and fetches piece c ^ ((row >> 1) & 7) of its row. Rows past the segment end: see last_on.
     const int r8 = lane >> 3, c = lane & 7;
     const uint8_t *a_src[MT];
+    uint32_t a_row[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const int r = (wave + 4 * i) * 8 + r8;
-        const uint32_t pr = t.row0 + (uint32_t)(r < (int)t.nrows ? r : 0);
-        const size_t src = g.a_rows ? g.a_rows[pr] : pr;
+        a_row[i] = t.row0 + (uint32_t)(r < (int)t.nrows ? r : 0);
+    }
+    if (g.a_rows) { // (requested ahead of the weights: loads return in order)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) a_row[i] = g.a_rows[a_row[i]];
+    }
+#pragma unroll
+    for (int j = 0; j < WRC; ++j) load_b(j < n_csteps ? j : n_csteps - 1, j);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int r = (wave + 4 * i) * 8 + r8;
+        const size_t src = a_row[i];
         a_src[i] = (const uint8_t *)(g.a + src * (size_t)cols) + ((c ^ (((r >> 1) & 7))) * 16);
+    }
+    // Only the last operation can hold rows past the segment end. Their lanes request nothing, and their places in the
+    // buffers are zeroed here, once. (A wavefront whose last operation has no row at all still requests one lane's piece,
+    // of the tile's first row, so that every operation counts as one in the waits below.)
+    const bool last_on = (wave + 4 * (MT - 1)) * 8 + r8 < (int)t.nrows;
+    const uint64_t last_lanes = __ballot(last_on), last_mask = last_lanes ? last_lanes : 1ull;
+    if (!last_on) {
+#pragma unroll
+        for (int b = 0; b < SLOTS; ++b) *(uint4 *)(lds + b * BUF + (wave + 4 * (MT - 1)) * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
     }
     const uint32_t lds_addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     auto stage_op = [&](int blk, int buf, int i) {
         const uint8_t *gp = a_src[i] + (size_t)blk * 128;
-        const uint32_t la = lds_addr + (uint32_t)(buf * kWideBufBytes + (wave + 4 * i) * 1024); // uniform
+        const uint32_t la = lds_addr + (uint32_t)(buf * BUF + (wave + 4 * i) * 1024); // uniform
         // (a wait state between the write of M0 and the request that reads it; nothing else in this kernel uses M0)
-        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(gp), "s"(la) : "memory");
+        if (i < MT - 1)
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(gp), "s"(la) : "memory");
+        else
+            asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dwordx4 %0, off\n\ts_mov_b64 exec, -1"
+                         : : "v"(gp), "s"(la), "s"(last_mask) : "memory"); // (control flow is uniform: every lane is on)
     };
-    // surplus steps of the last trip (n_steps not a multiple of the ring) must multiply zeros
+    // surplus steps of the last trip (WHOLE, n_steps not a multiple of the trip) must multiply zeros
+    const int n_whole = (n_steps + SLOTS - 1) / SLOTS * SLOTS;
     auto zero_block = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-            *(uint4 *)(lds + buf * kWideBufBytes + (wave + 4 * i) * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+        for (int i = 0; i < MT; ++i) *(uint4 *)(lds + buf * BUF + (wave + 4 * i) * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
         __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
     };
 
@@ -140,10 +192,6 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
     // activation fragment of each row tile for the current MFMA group; small tiles have registers to spare and too
     // few units per group to hide an LDS round trip, so they keep a second set and fetch a whole group ahead
     constexpr int XB = MT <= 2 ? 2 : 1;
-    // blocks in flight ahead of the one being computed. A short step (small tile) does not cover a memory round
-    // trip, so small tiles run three blocks ahead; that reuses the buffer read during the previous step, which is
-    // only safe because those tiles also wait for their own LDS reads before each barrier (see below).
-    constexpr int AHEAD = MT <= 2 ? 3 : 2;
     bf16x8_t xf[XB][MT];
     // fragment (mt, j) of a step: row mt * 32 + ln, the piece that holds this lane's eight reduction elements of MFMA
     // group j (chunk step c = j / NJC of the step, elements (2 c + h) * KV + 8 (j % NJC) onwards), stored at
@@ -155,7 +203,7 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
         x_rd[j] = lds + (ln >> 3) * 1024 + (ln & 7) * 128 + ((piece ^ ((ln >> 1) & 7)) * 16);
     }
     auto read_x = [&](int buf, int j, int mt) {
-        uint4 q = *(const uint4 *)(x_rd[j] + buf * kWideBufBytes + mt * 4096);
+        uint4 q = *(const uint4 *)(x_rd[j] + buf * BUF + mt * 4096);
         xf[j % XB][mt] = __builtin_bit_cast(bf16x8_t, q);
     };
 
@@ -165,11 +213,12 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
         if (b < n_steps) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) stage_op(b, b, i);
-        } else {
+        } else if (WHOLE) {
             zero_block(b);
         }
     }
-    __builtin_amdgcn_s_waitcnt(wait_vmcnt(0));
+    if (n_steps >= AHEAD) __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0((AHEAD - 1) * MT)); // block 0, and the zeros
+    else __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0(0));
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -178,23 +227,23 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) read_x(0, 0, mt);
 
-    // The loop always runs whole trips of kWideRing steps: surplus steps multiply zeroed activations with weights
-    // clamped onto the last valid step. Step j of a trip computes from buffer j, requests block s + AHEAD into buffer
-    // (j + AHEAD) % 4 during its first three MFMA groups, and at the start of the fourth waits for block s + 1 and
-    // synchronises, so that the first fragments of the next step can be fetched during that last group.
+    // Step j of a trip computes from slot j, requests block s + AHEAD into slot (j + AHEAD) % SLOTS during its first three
+    // MFMA groups, and at the start of the fourth waits for block s + 1 and synchronises, so that the first fragments of
+    // the next step can be fetched during that last group.
+    bool more = true;
 #pragma unroll 1
-    for (int trip = 0; trip < n_trips; ++trip) {
-        const int s0 = trip * kWideRing;
+    for (int s0 = 0; more; s0 += SLOTS) {
 #pragma unroll
-        for (int j = 0; j < kWideRing; ++j) {
+        for (int j = 0; j < SLOTS; ++j) {
             const int s = s0 + j;
-            const int buf_next = (j + 1) % kWideRing;
+            const int buf_next = (j + 1) % SLOTS;
             const bool stage = s + AHEAD < n_steps; // uniform
 #pragma unroll
             for (int c = 0; c < CH; ++c) {
                 const int ci = j * CH + c; // chunk step within the trip
                 const int cs_ahead = s * CH + c + WRC < n_csteps ? s * CH + c + WRC : n_csteps - 1;
                 load_b(cs_ahead, ci % WRC); // this slot was decoded one chunk step ago
+                asm volatile("" ::: "memory"); // every load stays one of its own: they are counted below
                 const int slot_next = (ci + 1) % WRC, which = ci & 1;
                 Meta meta_next[NT];
 #pragma unroll
@@ -205,21 +254,17 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
                 for (int jc = 0; jc < NJC; ++jc) {
                     const int jj = c * NJC + jc; // MFMA group within the step
                     if (jj == NJ - 1) {
-                        // block s + 1 must have landed; the AHEAD - 1 younger requests of MT operations each may still
-                        // fly (fewer near the end of the reduction, when nothing is requested any more), and so may
-                        // the weight chunks that the later chunk steps of this step have requested since (LATE, at
-                        // least one load per weight tile each)
-                        constexpr int LATE = (CH - 1) * NT;
-                        if (AHEAD == 2) {
-                            if (stage) __builtin_amdgcn_s_waitcnt(wait_vmcnt(MT + LATE));
-                            else __builtin_amdgcn_s_waitcnt(wait_vmcnt(LATE));
-                        } else {
-                            // also drain this wavefront's LDS reads: the next step's requests overwrite the buffer
-                            // that the reads issued during the previous MFMA group came from
-                            if (stage) __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0(2 * MT + LATE));
-                            else if (s + AHEAD - 1 < n_steps) __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0(MT + LATE));
-                            else __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0(LATE));
-                        }
+                        // Block s + 1 must have landed. Younger than its requests are those of the AHEAD - 1 blocks
+                        // behind it (near the end of the reduction there are fewer: none is counted on) and the loads
+                        // of the weight chunks (and their scales) of the steps since then: AHEAD - 1 steps' worth, in the
+                        // first trip only those requested inside the loop.
+                        constexpr int LOADS = CH * NT * (Fmt::kMetaEntryBytes ? 2 : 1), REQS = (AHEAD - 1) * MT;
+                        const int later = (AHEAD - 1) * LOADS, first = j + 1 < AHEAD - 1 ? (j + 1) * LOADS : later;
+                        const bool in_first = first < later && s0 == 0;
+                        if (stage && !in_first) wait_vmcnt_at_most(REQS + later);
+                        else if (stage) wait_vmcnt_at_most(REQS + first);
+                        else if (!in_first) wait_vmcnt_at_most(later);
+                        else wait_vmcnt_at_most(first);
                         asm volatile("" ::: "memory");
                         __builtin_amdgcn_s_barrier();
                         asm volatile("" ::: "memory");
@@ -242,7 +287,7 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
                                 else read_x(buf_next, 0, mt);
                             }
                             if (u % 6 == 0 && u / 6 < MT) { // the staging requests all fall into the first three groups
-                                if (stage) stage_op(s + AHEAD, (j + AHEAD) % kWideRing, u / 6);
+                                if (stage) stage_op(s + AHEAD, (j + AHEAD) % SLOTS, u / 6);
                             }
 #pragma unroll
                             for (int p = uc * NPC / NUC; p < (uc + 1) * NPC / NUC; ++p) {
@@ -256,7 +301,13 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
                     }
                 }
             }
-            if (!stage && s + AHEAD < n_trips * kWideRing) zero_block((j + AHEAD) % kWideRing); // a surplus step: zeros
+            if (WHOLE) {
+                if (!stage && s + AHEAD < n_whole) zero_block((j + AHEAD) % SLOTS); // a surplus step: zeros
+                if (j == SLOTS - 1) more = s + 1 < n_whole;
+            } else if (s + 1 >= n_steps) { // uniform
+                more = false;
+                break;
+            }
         }
     }
 
