@@ -405,6 +405,7 @@ static int routed_forward(const Layer *L, Workspace *w, const FwdLayout &f, cons
     gu.ldo = L->F;
     gu.tiles = po.tiles;
     gu.n_tiles = po.n_tiles;
+    gu.n_live = po.n_live;
     gu.max_tiles = f.max_tiles;
     gu.tile_m = f.tile_m;
     gu.ksplit = f.ksplit ? 1 : 0;
@@ -423,6 +424,7 @@ static int routed_forward(const Layer *L, Workspace *w, const FwdLayout &f, cons
     dn.out_rows = po.order; // unsort while storing (deepseek_v4.zig:809)
     dn.tiles = po.tiles;
     dn.n_tiles = po.n_tiles;
+    dn.n_live = po.n_live;
     dn.max_tiles = f.max_tiles;
     dn.tile_m = f.tile_m;
     dn.ksplit = f.ksplit ? 1 : 0;
@@ -883,7 +885,7 @@ static int gather_qmm_view(uint16_t *d_out, const uint16_t *d_x, const QView &v,
     const int max_tiles = pack_max_tiles((size_t)R, v.n_mats, tile_m);
     Bump b;
     size_t o_order = b.take((size_t)R * 4), o_arows = b.take((size_t)R * 4);
-    size_t o_tiles = b.take((size_t)max_tiles * sizeof(Tile)), o_nt = b.take(4);
+    size_t o_tiles = b.take((size_t)max_tiles * sizeof(Tile)), o_nt = b.take(4), o_nl = b.take(4);
     size_t o_scr = b.take(pack_scratch_bytes((size_t)R, v.n_mats));
     Workspace *w = nullptr;
     DMOE_TRY(workspace_reserve(ws, b.off, &w));
@@ -891,6 +893,7 @@ static int gather_qmm_view(uint16_t *d_out, const uint16_t *d_x, const QView &v,
     po.order = at<uint32_t>(w, o_order);
     po.tiles = at<Tile>(w, o_tiles);
     po.n_tiles = at<uint32_t>(w, o_nt);
+    po.n_live = at<uint32_t>(w, o_nl);
     po.bad_ids = w->flags + 1;
     DMOE_TRY(launch_pack(po, d_rhs_indices, (size_t)R, 1, v.n_mats, tile_m, at<void>(w, o_scr), st));
     const uint32_t *a_rows = po.order;
@@ -910,6 +913,7 @@ static int gather_qmm_view(uint16_t *d_out, const uint16_t *d_x, const QView &v,
     g.out_rows = po.order;
     g.tiles = po.tiles;
     g.n_tiles = po.n_tiles;
+    g.n_live = po.n_live;
     g.max_tiles = max_tiles;
     g.tile_m = tile_m;
     return run_gemm(g, small, st, small ? 0 : prefill_small_rows(v, v), few_rows((size_t)R, v.n_mats));

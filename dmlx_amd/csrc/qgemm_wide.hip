@@ -318,10 +318,22 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
     wide_epilogue<Fmt, GATE_UP, MT>(g, t, lds + wave * (kWideLdsBytes / kWideWaves), acc, col_base);
 }
 
+// Consecutive tiles whose workgroups for one column strip start back to back on one XCD. Unquantized weights: a tile of 128
+// rows does 128 flops per byte of weights, so experts of several tiles are bound by fetching their weights through the L2s
+// again for every tile (256 rows per expert: 0.83 PFLOP/s x 1 byte / 128 flops = 6.5 TB/s). With runs of four the second to
+// fourth workgroup of a strip find the weights in their L2: one projection [256, 2048, 4096], 256 / 512 rows per expert 1321 /
+// 2533 -> 1139 / 1978 us; a step of 8192 tokens, Zipf-skewed, 3379 -> 3076 us. Not where most experts have one tile (128 rows
+// each: 831 -> 844 us), and not the last tiles of a list that make no whole group: four of them would go to one XCD pair. The
+// quantized formats stay at one: 2080 tokens on 8-bit experts +1.5 %, 8192 tokens on 4-bit ones +5 %.
+template <typename Fmt>
+__host__ __device__ constexpr uint32_t wide_run() {
+    return Fmt::kVals == 8 ? 4u : 1u;
+}
+
 template <typename Fmt, bool GATE_UP>
 __global__ __launch_bounds__(kWideWaves * 64, 2) void qgemm_wide_kernel(GemmArgs g) {
-    extern __shared__ __attribute__((aligned(1024))) uint8_t wide_lds[]; // [kWideRing][128 rows][128 bytes], swizzled
-    Tile t;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t wide_lds[]; // [slots][rows of the tile][128 bytes], swizzled
+    constexpr uint32_t RUN = wide_run<Fmt>();
     // Workgroups go to the eight XCDs round-robin in launch order; gridDim.y is a multiple of 8, which makes the maps
     // below permutations of the grid. XCD x = (tile class x / 2, strip half x % 2): it takes every fourth tile of the
     // list and one half of the tile's column strips, a tile's strips back to back. A tile's activations then enter two
@@ -332,20 +344,32 @@ __global__ __launch_bounds__(kWideWaves * 64, 2) void qgemm_wide_kernel(GemmArgs
     // 2..16 consecutive tiles with ALL their strips, so that the tiles of an expert could share its weights through
     // that L2, measured 0.5 % to 15 % slower the longer the run: an expert's weights do not fit one L2.)
     const uint32_t nx = gridDim.x, b = blockIdx.y * nx + blockIdx.x, k = b >> 3, xcd = b & 7u;
-    uint32_t slot;
+    uint32_t slot, n_slots, run = 1;
+    if (g.tiles) {
+        n_slots = *g.n_tiles;
+        if (RUN > 1 && g.n_live) run = 8u * n_slots >= 9u * *g.n_live ? RUN : 1u;
+    } else {
+        n_slots = (uint32_t)((g.dense_rows + g.tile_m - 1) / g.tile_m);
+        run = RUN;
+    }
     int strip;
     if (nx % 2u == 0u) {
-        const uint32_t half = nx / 2u;
-        slot = 4u * (k / half) + (xcd >> 1);
-        strip = (int)((xcd & 1u) * half + k % half);
+        const uint32_t half = nx / 2u, group = k / (RUN * half), r = k % (RUN * half); // a group: 4 * RUN tiles (fewer at the grid's end)
+        if (run > 1u && (group + 1u) * 4u * RUN <= n_slots) {
+            slot = 4u * RUN * group + RUN * (xcd >> 1) + r % RUN;
+            strip = (int)((xcd & 1u) * half + r / RUN);
+        } else {
+            slot = 4u * (RUN * group + r / half) + (xcd >> 1);
+            strip = (int)((xcd & 1u) * half + r % half);
+        }
     } else {
         slot = (k / nx) * 8u + xcd;
         strip = (int)(k % nx);
     }
+    Tile t;
     if (g.tiles) {
-        const uint32_t n_tiles = *g.n_tiles;
         t = g.tiles[slot < (uint32_t)g.max_tiles ? slot : 0u];
-        if (slot >= n_tiles) return;
+        if (slot >= n_slots) return;
         if ((int)t.nrows < g.min_rows) return; // left to the weight-streaming kernel
     } else {
         t.expert = 0;
