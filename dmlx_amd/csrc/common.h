@@ -233,6 +233,7 @@ struct GemmArgs {
     const Tile *tiles = nullptr;  // nullable: dense mode (one segment, expert 0, `dense_rows` rows)
     const uint32_t *n_tiles = nullptr;
     const uint32_t *n_live = nullptr; // nullable: experts with rows, for the wide kernel's choice of a tile map
+    int stream_weights = 0;           // wide kernel, set by its launcher: see kWideStreamBytes
     int max_tiles = 0;
     int tile_m = 0;               // rows per tile the tile list (or the dense split) was built with
     int dense_rows = 0;

@@ -110,7 +110,10 @@ __global__ void dequant_fused_kernel(uint16_t *__restrict__ out, QView q, int ma
     const uint8_t *srow = q.scales + (size_t)mat * q.s_mat + (size_t)row * q.s_row;
     const uint8_t *brow = q.biases ? q.biases + (size_t)mat * q.s_mat + (size_t)row * q.s_row : nullptr;
     uint4 raw = *(const uint4 *)(wrow + (size_t)c * 16);
-    const Meta m = Fmt::pair_meta(Fmt::load_meta(q, srow, brow, k0));
+    uint32_t sb[2];
+    Fmt::load_meta_raw(q, srow, brow, k0, sb);
+    if (Fmt::kMetaEntryBytes == 2) sb[0] |= sb[1] << 16; // the word of the packed layout
+    const Meta m = Fmt::pair_meta(Fmt::meta_from_packed(sb));
     uint32_t pairs[Fmt::kVals / 2], st[Fmt::kPairState] = {};
     Fmt::pair_state(st);
 #pragma unroll

@@ -26,10 +26,9 @@ namespace dmoe {
 
 // E8M0 shared exponent -> 2^(s-127); 255 is NaN
 __device__ __forceinline__ float e8m0_to_f32(uint32_t s) {
-    uint32_t bits = s << 23;
-    bits = s == 0u ? 0x00400000u : bits; // 2^-127, an f32 subnormal
-    bits = s == 255u ? 0x7fc00000u : bits;
-    return __uint_as_float(bits);
+    if (s == 255u) return __uint_as_float(0x7fc00000u);
+    if (s == 0u) return __uint_as_float(0x00400000u); // 2^-127, an f32 subnormal
+    return __uint_as_float(s << 23);
 }
 
 // E2M1 code (sign in bit 3) -> f32: 0, .5, 1, 1.5, 2, 3, 4, 6
@@ -237,7 +236,14 @@ struct FmtMxfp4 {
         m.b = 0.0f;
         return m;
     }
-    __device__ static __forceinline__ Meta meta_from_packed(const uint32_t *sb) { return meta_from_raw(sb); }
+    // for the packed conversions only, which take the exponent field of their scale operand as an E8M0 exponent, 0 and 255
+    // included (compared with e8m0_to_f32 for all 256 exponents)
+    __device__ static __forceinline__ Meta meta_from_packed(const uint32_t *sb) {
+        Meta m;
+        m.s = __uint_as_float(sb[0] << 23);
+        m.b = 0.0f;
+        return m;
+    }
     __device__ static __forceinline__ Meta load_meta(const QView &q, const uint8_t *row_s, const uint8_t *row_b,
                                                      int k0) {
         uint32_t sb[2];
