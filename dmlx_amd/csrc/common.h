@@ -232,8 +232,6 @@ struct GemmArgs {
     const uint32_t *row_scale_idx = nullptr; // nullable: row_scale index of sorted row p (else p)
     const Tile *tiles = nullptr;  // nullable: dense mode (one segment, expert 0, `dense_rows` rows)
     const uint32_t *n_tiles = nullptr;
-    const uint32_t *n_live = nullptr; // nullable: experts with rows, for the wide kernel's choice of a tile map
-    int stream_weights = 0;           // wide kernel, set by its launcher: see kWideStreamBytes
     int max_tiles = 0;
     int tile_m = 0;               // rows per tile the tile list (or the dense split) was built with
     int dense_rows = 0;
@@ -254,6 +252,8 @@ struct GemmArgs {
     uint32_t *wait_expired = nullptr;
     float swiglu_limit_dense = 0.0f;    // the limit for tiles flagged kTileDense
     uint32_t row_scale_rows = 0xffffffffu; // row_scale applies to sorted rows below this
+    const uint32_t *n_live = nullptr; // nullable: experts with rows, for the wide kernel's choice of a tile map
+    int stream_weights = 0;           // wide kernel, set by its launcher: see kWideStreamBytes
 };
 // tile_m the kernels were built for
 constexpr int kSkinnyTileM = 32;          // most rows a skinny tile can hold (see qgemm_skinny_tile_m)

@@ -65,7 +65,10 @@ struct SkinnyStage {
 };
 
 // One tile, start to finish. RJT = 1: tiles of one row block (4 accumulators per lane, no restaging); RJT = 4: larger
-// tiles (16 accumulators; a tile of two row blocks computes four, the surplus rows are never stored). The kernel
+// tiles (16 accumulators). RJT = 2, factored form only, where a lane scales every accumulator at every step (the others leave
+// that to the matrix instruction, and compute four row blocks for a tile of two): 8 accumulators for tiles of 9 to 16 rows. The
+// vector ALU then has 48 instead of 64 operations per step, where the weight stream leaves it 96 issue slots (9 / 12 / 16 rows
+// per expert, [256, 2048, 4096] 4-bit: 237 / 240 / 251 -> 227 / 232 / 239 us; a step of 509 tokens, its launch 790 -> 776). The kernel
 // calls one or the other right after fetching the tile, so the two share nothing but the arguments and each keeps
 // its own register allocation.
 // `gate_up` (workgroup-uniform) is the role of the launch: gate and up projections with SwiGLU (their rows on
@@ -227,7 +230,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     // stored. The matrix instruction always covers 32 rows; what grows with the tile is the number of accumulators
     // a lane scales and keeps (4 per row block), behind wave-uniform branches.
     const int nrows = __builtin_amdgcn_readfirstlane((int)t.nrows);
-    const int rj = RJT == 1 ? 1 : nrows <= 2 * kSkinnyRowBlock ? 2 : 4; // row blocks = spans of the reduction
+    const int rj = RJT <= 2 ? RJT : nrows <= 2 * kSkinnyRowBlock ? 2 : 4; // row blocks = spans of the reduction
     const int rp = rj * kSkinnyRowBlock;             // rows the LDS layout is made for
     const int span_steps = n_steps / rj;             // the launcher only builds larger tiles when this divides
     const int span_bytes = span_steps * KSTEP * 2;   // bytes of one row in one span
@@ -636,6 +639,8 @@ __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(Gem
     }
     if (__builtin_amdgcn_readfirstlane((int)t.nrows) <= kSkinnyRowBlock)
         skinny_tile<Fmt, FACTORED, PACKED, 1, MBLK>(g, t, skinny_lds, g.gate_up, sync, slot);
+    else if (FACTORED && __builtin_amdgcn_readfirstlane((int)t.nrows) <= 2 * kSkinnyRowBlock)
+        skinny_tile<Fmt, FACTORED, PACKED, FACTORED ? 2 : 4, MBLK>(g, t, skinny_lds, g.gate_up, sync, slot);
     else
         skinny_tile<Fmt, FACTORED, PACKED, kSkinnyTileM / kSkinnyRowBlock, MBLK>(g, t, skinny_lds, g.gate_up, sync, slot);
 }
