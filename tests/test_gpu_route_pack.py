@@ -144,7 +144,10 @@ def test_gate_route_bit_exact(dmoe, orc, T, E, K, masked):
                                    # experts, nearly every row on the same few experts); and sizes just above it
                                    (1, 6, 256), (2, 8, 1024), (16, 1, 16), (5, 3, 3), (3, 5, 40), (2, 6, 256),
                                    (10, 6, 256), (64, 1, 16), (8, 8, 1024), (9, 7, 3), (17, 1, 40),
-                                   (171, 6, 256), (2080, 6, 256), (8192, 6, 256), (5000, 3, 1000), (300, 1, 1)])
+                                   (171, 6, 256), (2080, 6, 256), (8192, 6, 256), (5000, 3, 1000), (300, 1, 1),
+                                   # one launch of 2 to 4 groups per wavefront, and the first size above it
+                                   (1025, 1, 8), (1024, 2, 1), (2049, 1, 1024), (3000, 1, 3), (1024, 3, 256), (683, 6, 256),
+                                   (682, 6, 51), (2048, 2, 1024), (4097, 1, 256)])
 def test_pack_bit_exact(dmoe, orc, ws, T, K, E):
     rng = np.random.default_rng(T * 7 + K + E)
     if T >= 2000:  # skewed: a few heavy experts, many empty ones
