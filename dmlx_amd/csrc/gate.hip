@@ -459,8 +459,12 @@ __device__ __forceinline__ float det_softplusf(float x) {
 // round trip through memory; `scores` is written only when the caller wants them. Lane l owns experts l, l + 64, ...
 // (EPL of them). Softmax: the sum is taken as one partial per lane (its experts in increasing order), folded by
 // halves (lane i += lane i + 32, 16, .. 1).
+// SPLIT (a few hundred tokens at most; the matmul kernel stored every segment's sum): one workgroup per token, whose
+// wavefronts each add up and score 64 experts, one per lane; the first one goes on with all of them. (One wavefront alone
+// had 32 sums of four experts to fetch in two memory round trips and four times the scoring: one token 8.3 -> 5.0 us, 64 tokens
+// 14.4 -> 8.4, 300 tokens 9.9 -> 6.7.)
 template <int EPL, bool ROUTE, bool SPLIT>
-__global__ __launch_bounds__(kGateWaves * 64) void gate_scores_kernel(float *__restrict__ scores,
+__global__ __launch_bounds__(SPLIT ? EPL * 64 : kGateWaves * 64) void gate_scores_kernel(float *__restrict__ scores,
                                                                       const float *__restrict__ partial, int T,
                                                                       int E, int n_seg, int scoring,
                                                                       uint32_t *__restrict__ out_idx,
@@ -468,38 +472,44 @@ __global__ __launch_bounds__(kGateWaves * 64) void gate_scores_kernel(float *__r
                                                                       const float *__restrict__ bias,
                                                                       const uint8_t *__restrict__ resident, int K,
                                                                       int normalize, float route_scale) {
+    __shared__ float shared_v[SPLIT ? EPL * 64 : 1];
     const int lane = (int)threadIdx.x & 63;
-    const int t = (int)blockIdx.x * kGateWaves + ((int)threadIdx.x >> 6);
+    const int t = SPLIT ? (int)blockIdx.x : (int)blockIdx.x * kGateWaves + ((int)threadIdx.x >> 6);
     if (t >= T) return;
+    auto score = [&](float x) { // (softmax: below)
+        if (scoring == DMOE_SCORE_SIGMOID) return 1.0f / (1.0f + det_expf(-x));
+        if (scoring == DMOE_SCORE_SQRTSOFTPLUS) return sqrtf(det_logf(1.0f + det_expf(x))); // the reference's literal form (:575-583)
+        return sqrtf(det_softplusf(x));
+    };
     float v[EPL];
     float mx = -__builtin_inff();
-    // SPLIT (the matmul kernel stored every segment's sum): the segment sums of all of the lane's experts are requested
-    // 64 at a time (one memory round trip per batch, not one per expert and eight segments) and added per expert in
-    // segment order. Otherwise there is one sum per expert (n_seg == 1).
-    constexpr int SB = SPLIT ? 64 / EPL : 1;
     const float *const p = partial + (size_t)t * n_seg * E;
+    if (SPLIT) {
+        constexpr int SB = 32; // sums requested at a time: all of them up to 4096 hidden
+        const int e = (int)threadIdx.x, ec = e < E ? e : E - 1;
+        float x = 0.0f;
+        for (int s0 = 0; s0 < n_seg; s0 += SB) {
+            float q[SB];
 #pragma unroll
-    for (int i = 0; i < EPL; ++i) v[i] = 0.0f;
-    for (int s0 = 0; s0 < n_seg; s0 += SB) {
-        float q[EPL][SB];
-#pragma unroll
-        for (int i = 0; i < EPL; ++i) {
-            const int e = lane + 64 * i;
-            const int ec = e < E ? e : E - 1;
-#pragma unroll
-            for (int j = 0; j < SB; ++j) q[i][j] = s0 + j < n_seg ? p[(size_t)(s0 + j) * E + ec] : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < EPL; ++i)
+            for (int j = 0; j < SB; ++j) q[j] = p[(size_t)(s0 + j < n_seg ? s0 + j : n_seg - 1) * E + ec];
 #pragma unroll
             for (int j = 0; j < SB; ++j)
-                if (s0 + j < n_seg) v[i] = v[i] + q[i][j];
+                if (s0 + j < n_seg) x = x + q[j];
+        }
+        x = bf16_bits_to_f32(f32_to_bf16_bits(x));
+        shared_v[e] = scoring == DMOE_SCORE_SOFTMAX ? x : score(x);
+        __syncthreads();
+        if (e >= 64) return;
+    }
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) { // loads unconditional, ahead of everything else
+        const int ec = lane + 64 * i < E ? lane + 64 * i : E - 1;
+        v[i] = SPLIT ? shared_v[ec] : 0.0f + p[ec];
     }
 #pragma unroll
     for (int i = 0; i < EPL; ++i) {
-        const int e = lane + 64 * i;
-        if (e < E) {
-            v[i] = bf16_bits_to_f32(f32_to_bf16_bits(v[i]));
+        if (lane + 64 * i < E) {
+            if (!SPLIT) v[i] = bf16_bits_to_f32(f32_to_bf16_bits(v[i]));
             mx = v[i] > mx ? v[i] : mx;
         } else {
             v[i] = 0.0f;
@@ -524,14 +534,10 @@ __global__ __launch_bounds__(kGateWaves * 64) void gate_scores_kernel(float *__r
 #pragma unroll
         for (int i = 0; i < EPL; ++i)
             if (lane + 64 * i < E) v[i] = v[i] / sum;
-    } else {
+    } else if (!SPLIT) {
 #pragma unroll
-        for (int i = 0; i < EPL; ++i) {
-            if (lane + 64 * i >= E) continue;
-            if (scoring == DMOE_SCORE_SIGMOID) v[i] = 1.0f / (1.0f + det_expf(-v[i]));
-            else if (scoring == DMOE_SCORE_SQRTSOFTPLUS) v[i] = sqrtf(det_logf(1.0f + det_expf(v[i]))); // the reference's literal form (:575-583)
-            else v[i] = sqrtf(det_softplusf(v[i]));
-        }
+        for (int i = 0; i < EPL; ++i)
+            if (lane + 64 * i < E) v[i] = score(v[i]);
     }
     if (scores) {
 #pragma unroll
@@ -551,8 +557,8 @@ __global__ __launch_bounds__(kGateWaves * 64) void gate_scores_kernel(float *__r
 
 template <int EPL, bool ROUTE, typename... Args>
 static void launch_scores(bool split, dim3 grid, dim3 block, hipStream_t st, Args... args) {
-    if (split) hipLaunchKernelGGL((gate_scores_kernel<EPL, ROUTE, true>), grid, block, 0, st, args...);
-    else hipLaunchKernelGGL((gate_scores_kernel<EPL, ROUTE, false>), grid, block, 0, st, args...);
+    if (split) hipLaunchKernelGGL((gate_scores_kernel<EPL, ROUTE, true>), grid, block, 0, st, args...); // a workgroup per token
+    else hipLaunchKernelGGL((gate_scores_kernel<EPL, ROUTE, false>), grid, block, 0, st, args...);      // a wavefront per token
 }
 
 // Hash routing (deepseek_v4.zig:619-636, then :655-678): the experts of a token come from a table indexed by its
@@ -714,13 +720,13 @@ int dmoe_gate_forward(uint32_t *d_out_indices, float *d_out_weights, float *d_ou
     DMOE_LAUNCH_CHECK();
     // the reference renormalises for every scoring function except softmax (:663)
     const int normalize = G->scoring != DMOE_SCORE_SOFTMAX ? 1 : 0;
-    const dim3 sgrid((unsigned)ceil_div(T, kGateWaves));
+    const dim3 sgrid((unsigned)(split ? T : ceil_div(T, kGateWaves))), sblock(split ? ceil_div(G->E, 64) * 64 : kGateWaves * 64);
     if (hash) { // hash layer with token ids: the table replaces the top-k (:619-636)
         if (G->E <= 256)
-            launch_scores<4, false>(split, sgrid, block, st, scores, partial, T, G->E, n_out_seg, G->scoring, nullptr, nullptr,
+            launch_scores<4, false>(split, sgrid, sblock, st, scores, partial, T, G->E, n_out_seg, G->scoring, nullptr, nullptr,
                                     nullptr, nullptr, 0, 0, 1.0f);
         else
-            launch_scores<16, false>(split, sgrid, block, st, scores, partial, T, G->E, n_out_seg, G->scoring, nullptr, nullptr,
+            launch_scores<16, false>(split, sgrid, sblock, st, scores, partial, T, G->E, n_out_seg, G->scoring, nullptr, nullptr,
                                      nullptr, nullptr, 0, 0, 1.0f);
         DMOE_LAUNCH_CHECK();
         hipLaunchKernelGGL(gate_hash_route_kernel, dim3((unsigned)ceil_div(T, 256)), dim3(256), 0, st, d_out_indices,
@@ -731,10 +737,10 @@ int dmoe_gate_forward(uint32_t *d_out_indices, float *d_out_weights, float *d_ou
     // scoring and selection in one launch; the scores leave the registers only if the caller asked for them
     DMOE_REQUIRE(G->K >= 1 && G->K <= G->E && G->K <= 64, "gate_forward: K=%d must satisfy 1 <= K <= min(E,64)", G->K);
     if (G->E <= 256)
-        launch_scores<4, true>(split, sgrid, block, st, d_out_scores, partial, T, G->E, n_out_seg, G->scoring, d_out_indices,
+        launch_scores<4, true>(split, sgrid, sblock, st, d_out_scores, partial, T, G->E, n_out_seg, G->scoring, d_out_indices,
                                d_out_weights, G->bias, G->mask, G->K, normalize, G->route_scale);
     else
-        launch_scores<16, true>(split, sgrid, block, st, d_out_scores, partial, T, G->E, n_out_seg, G->scoring, d_out_indices,
+        launch_scores<16, true>(split, sgrid, sblock, st, d_out_scores, partial, T, G->E, n_out_seg, G->scoring, d_out_indices,
                                 d_out_weights, G->bias, G->mask, G->K, normalize, G->route_scale);
     DMOE_LAUNCH_CHECK();
     return DMOE_OK;
