@@ -432,7 +432,10 @@ struct ChunkStream {
     // still find each other's lines in L2
     __device__ __forceinline__ uint4 load_chunk_stream(int step) const {
         typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-        const u32x4_t v = __builtin_nontemporal_load((const u32x4_t *)(w + (size_t)step * (PACKED ? 1024 : 32) + wlane));
+        // (global, said aloud: what pin() has passed through is a pointer of unknown kind to the compiler, and the flat loads it
+        // made of it held up every wait for LDS data until memory had answered)
+        typedef const __attribute__((address_space(1))) u32x4_t *global_u32x4;
+        const u32x4_t v = __builtin_nontemporal_load((global_u32x4)(uintptr_t)(w + (size_t)step * (PACKED ? 1024 : 32) + wlane));
         return make_uint4(v.x, v.y, v.z, v.w);
     }
     __device__ __forceinline__ void load_meta(const QView &q, int step, uint32_t *sb) const {
