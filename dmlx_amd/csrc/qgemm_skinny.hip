@@ -78,19 +78,26 @@ struct SkinnyStage {
 // reach g.tile_done_target before it reads its activations (the other role's output), its weight ring already in flight.
 constexpr int kSkinnySyncNone = 0, kSkinnySyncSignal = 1, kSkinnySyncWait = 2;
 
-// LDS: [activation window][sums of x per step][GROUPED only: 4 KiB per wavefront for turning weight lines]
+// LDS: [activation window][sums of x per step][MBLK only: 4 KiB per wavefront for turning weight lines][zeros]
 __host__ __device__ constexpr size_t skinny_turn_offset(int cols, int kstep) {
     return (size_t)kSkinnyRowBlock * (size_t)cols * 2 + (size_t)kSkinnyTileM * 16 +
            (size_t)(cols / kstep) * kSkinnyRowBlock * sizeof(float) + 128;
 }
 constexpr size_t kSkinnyTurnBytes = (size_t)2 * kSkinnyWaves * 4 * 1024;
+// The matrix instruction covers 32 rows of activations, most tiles have a few. In the factored 4-bit form the lanes past a
+// tile's rows read zeros: the chip is power-limited under a decode step too, and multiplying zeros costs less of it than
+// multiplying row 0 again (steps of 64 / 509 tokens 244 / 813 -> 233 / 795 us). One round of the ring's worth of zeros serves
+// every step. The other formats gained 1 % on 64 tokens (MXFP4) and lost up to 5 % on a few (2 to 5 tokens).
+__host__ __device__ constexpr size_t skinny_zero_bytes(bool mblk) { return mblk ? 2048 : 1024; }
+constexpr size_t kSkinnyMaxLds = 151 * 1024;
+constexpr size_t kSkinnyMblkBytes = kSkinnyTurnBytes + skinny_zero_bytes(true) - skinny_zero_bytes(false); // on top, MBLK kernels
 // where a tile's outputs are gathered before they are stored: behind the exchange areas of the epilogue (16 KiB)
 constexpr size_t kSkinnyStageOffset = 16384, kSkinnyStageBytes = (size_t)kSkinnyTileM * 256 * 2;
 
 // MBLK (MLX layout only): the scale / bias entries of a row are not fetched one per step (32 cache lines touched per
 // load for 2 useful bytes each, again at every step: these loads, not the weights, bounded the MLX-layout path) but 16
 // bytes at a time - eight bf16 or sixteen E8M0 entries, the next block requested while the current one is in use.
-template <typename Fmt, bool FACTORED, bool PACKED, int RJT, bool MBLK, bool KSPLIT = false>
+template <typename Fmt, bool FACTORED, bool PACKED, int RJT, bool MBLK, bool KSPLIT = false, bool ZEROS = FACTORED>
 __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, uint8_t *skinny_lds, const bool gate_up,
                                             const int sync, const uint32_t slot) {
     using CS = ChunkStream<Fmt, PACKED>;
@@ -285,6 +292,9 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         }
     };
 
+    uint8_t *const zeros = skinny_lds + skinny_turn_offset(cols, KSTEP) + (MBLK ? kSkinnyTurnBytes : 0);
+    static_assert((size_t)ROUND * KSTEP * 2 <= skinny_zero_bytes(MBLK), "a round of zeros");
+    if (ZEROS && tid * 16 < (int)skinny_zero_bytes(MBLK)) *(uint4 *)(zeros + tid * 16) = make_uint4(0, 0, 0, 0);
     SkinnyStage<NM> ring[STAGES];
     if (MBLK) load_mblock(0); // taken over by step 0, which requests block 1
     if (sync == kSkinnySyncWait) {
@@ -329,9 +339,11 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         __syncthreads();
     }
 
-    // A-operand source of this lane: tile row ln, reduction half h. Lanes past the tile's rows read row 0 again:
-    // their operand rows only reach accumulator rows that are never stored.
-    const uint8_t *xlane = xs_lds + (ln < nrows ? ln : 0) * pitch + h * KV * 2;
+    // A-operand source of this lane: tile row ln, reduction half h, from step `xs` of the span on; lanes past the tile's rows
+    // stay on the zeros (else: read row 0 again; their operand rows only reach accumulator rows that are never stored).
+    const uint8_t *const xlane = (ln < nrows ? xs_lds + ln * pitch : ZEROS ? zeros : xs_lds) + h * KV * 2;
+    const uint32_t xmove = !ZEROS || ln < nrows ? 0xffffffffu : 0u;
+    auto x_from = [&](int xs) { return xlane + ((uint32_t)((xs + sb0) * KSTEP * 2) & xmove); };
     const uint32_t mask = vgpr_const32(0x000f000fu), magic = vgpr_const32(0x43004300u);
 
     // accumulator registers 4 j + r of a lane belong to tile row 8 j + 4 h + r (row block j)
@@ -348,9 +360,8 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
             for (int r = 0; r < 4 * RJT; ++r) facc[mi][r] = 0.0f;
 
         // One step: decode every projection's chunk first, then issue the matrix instructions of the projections
-        // alternately (independent accumulation chains), then apply the scales. `xs` = step within the span.
-        auto consume = [&](int gstep, int p8, int xs, const SkinnyStage<NM> &s) {
-            const uint8_t *xstep = xlane + (size_t)(xs + sb0) * KSTEP * 2;
+        // alternately (independent accumulation chains), then apply the scales. `xs` = step within the span, `xstep` its activations.
+        auto consume = [&](int gstep, int p8, int xs, const uint8_t *xstep, const SkinnyStage<NM> &s) {
             const float *gs_step = gs_lds + (xs + sb0) * rp + 4 * h;
             Meta meta[NM];
             if (MBLK) {
@@ -468,6 +479,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
                 x0 = s0;
                 next_span += span_steps;
             }
+            const uint8_t *const xround = x_from(s0 - x0);
 #pragma unroll
             for (int j = 0; j < ROUND; ++j) {
                 const int step = s0 + j, ahead = step + PRE;
@@ -480,15 +492,16 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
                             load_stage(ahead + LG + i < n_loc ? ahead + LG + i : n_loc - LG + i, ring[(j + LG) % STAGES + i], i);
                     }
                     turned.raw[0] = turned_raw[j % LG];
-                    consume(step, j & 7, step - x0, turned);
+                    consume(step, j & 7, step - x0, xround + j * KSTEP * 2, turned);
                     continue;
                 }
                 load_stage(LEAN_TAIL || ahead < n_loc ? ahead : n_loc - 1, ring[(j + PRE) % STAGES]);
-                consume(step, j & 7, step - x0, ring[j % STAGES]);
+                consume(step, j & 7, step - x0, xround + j * KSTEP * 2, ring[j % STAGES]);
             }
         }
 #pragma unroll 1
         for (int t0 = full; RJT == 1 && t0 < n_loc; t0 += ROUND) { // only tiles of one row block get here
+            const uint8_t *const xround = x_from(t0);
 #pragma unroll
             for (int j = 0; j < ROUND; ++j) {
                 const int step = t0 + j;
@@ -499,12 +512,12 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
                             if (step + LG < n_loc) turn_write((j + LG) % STAGES);
                         }
                         turned.raw[0] = turned_raw[j % LG];
-                        consume(step, j & 7, step, turned);
+                        consume(step, j & 7, step, xround + j * KSTEP * 2, turned);
                     }
                     continue;
                 }
                 if (step + PRE < n_loc) load_stage(step + PRE, ring[(j + PRE) % STAGES]);
-                if (step < n_loc) consume(step, j & 7, step, ring[j % STAGES]);
+                if (step < n_loc) consume(step, j & 7, step, xround + j * KSTEP * 2, ring[j % STAGES]);
             }
         }
 
@@ -603,7 +616,9 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
 // y < a.max_tiles are the gate/up tiles, the next a.max_tiles the down tiles of the same list. The hardware starts
 // workgroups in index order, so every producer of a tile is running or done by the time a consumer of it starts to
 // wait; the down workgroups that become resident while the last gate/up workgroups drain stream their weights meanwhile.
-template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false>
+// ONE: launches of a few workgroups (single launches of tiles of at most one row block). They are paced by each workgroup's own
+// chain, not by power, and read their code cold: no zeros, no copies for larger tiles (small layer, 16 tokens: 36.3 -> 34.7 us).
+template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool ONE = false>
 __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(GemmArgs a, GemmArgs b, int paired) {
     extern __shared__ __attribute__((aligned(16))) uint8_t skinny_lds[];
     const bool second = paired && blockIdx.y >= (uint32_t)a.max_tiles; // workgroup-uniform
@@ -633,8 +648,8 @@ __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(Gem
         uint32_t left = (uint32_t)g.dense_rows - t.row0;
         t.nrows = left < (uint32_t)g.tile_m ? left : (uint32_t)g.tile_m;
     }
-    if (KSPLIT) { // the launcher builds no tile above one row block for this kernel
-        skinny_tile<Fmt, FACTORED, PACKED, 1, MBLK, KSPLIT>(g, t, skinny_lds, g.gate_up, sync, slot);
+    if (KSPLIT || ONE) { // the launcher builds no tile above one row block for these kernels
+        skinny_tile<Fmt, FACTORED, PACKED, 1, MBLK, KSPLIT, false>(g, t, skinny_lds, g.gate_up, sync, slot);
         return;
     }
     if (__builtin_amdgcn_readfirstlane((int)t.nrows) <= kSkinnyRowBlock)
@@ -654,7 +669,7 @@ static size_t skinny_lds_bytes(const QView &b) {
     // At least 32 KiB: once the main loop is done the wavefronts exchange their sums through the start of the window
     // (gate/up pairs: 4 KiB per row block of the tile, up to 16 KiB; split reduction: bytes 4096 .. 8191) and gather
     // the tile's outputs behind that (up to 32 rows of 256 columns), which a short reduction dimension would not cover.
-    return std::max(skinny_turn_offset(b.cols, 2 * skinny_vals(b)), kSkinnyStageOffset + kSkinnyStageBytes);
+    return std::max(skinny_turn_offset(b.cols, 2 * skinny_vals(b)) + skinny_zero_bytes(false), kSkinnyStageOffset + kSkinnyStageBytes);
 }
 
 // Rows per tile to build tile lists with for this weight shape: a tile of 2 (4) row blocks splits the reduction
@@ -669,7 +684,7 @@ int qgemm_skinny_tile_m(const QView &b) {
 bool qgemm_skinny_supports(const QView &b) {
     // unquantized weights: resident (re-ordered) stacks only, whole 32-row blocks
     if (b.mode == DMOE_QUANT_NONE && !(b.packed && b.rows % 32 == 0 && ((uintptr_t)b.w % 16) == 0)) return false;
-    return b.cols % (2 * skinny_vals(b)) == 0 && skinny_lds_bytes(b) <= 150 * 1024;
+    return b.cols % (2 * skinny_vals(b)) == 0 && skinny_lds_bytes(b) <= kSkinnyMaxLds;
 }
 
 // GemmArgs::ksplit needs the packed layout, two halves of the reduction that are whole ring rounds and start on a
@@ -689,17 +704,17 @@ static bool mlx_meta_blocks(const QView &b) {
     // a block of entries must span exactly eight reduction steps (affine 4-bit: groups of 64; MXFP4: 32; 8-bit: 32)
     const int kstep = b.bits == 4 ? 64 : 32;
     if ((int)(16 / esz) * b.group != 8 * kstep) return false;
-    if (skinny_lds_bytes(b) + kSkinnyTurnBytes > 150 * 1024 || b.w_row % 128 != 0 || ((uintptr_t)b.w % 16) != 0 || b.w_mat % 16 != 0 ||
+    if (skinny_lds_bytes(b) + kSkinnyMblkBytes > kSkinnyMaxLds + 1024 || b.w_row % 128 != 0 || ((uintptr_t)b.w % 16) != 0 || b.w_mat % 16 != 0 ||
         (uint64_t)b.rows * (uint64_t)b.w_row >= (1ull << 32))
         return false; // the line-wise weight loads of the small tiles: LDS to turn them in, whole lines per group
     return row >= 16 && row % 16 == 0 && b.s_row % 16 == 0 && b.s_mat % 16 == 0 && ((uintptr_t)b.scales % 16) == 0 &&
            (!b.biases || ((uintptr_t)b.biases % 16) == 0);
 }
 
-template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK, bool KSPLIT = false>
+template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK, bool KSPLIT = false, bool ONE = false>
 static int skinny_raise_limit() {
     static LdsLimit limit; // per instantiation
-    return raise_lds_limit(limit, (const void *)qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT>, 150 * 1024);
+    return raise_lds_limit(limit, (const void *)qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, ONE>, (int)kSkinnyMaxLds + 1024);
 }
 // the instantiations SkinnyLaunch can pick for one format
 template <typename Fmt>
@@ -709,6 +724,7 @@ static int skinny_prepare_format() {
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, true, false>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, true, false>()));
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, true, false, true>()));
+    DMOE_TRY((skinny_raise_limit<Fmt, can_factor, true, false, false, can_factor>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, true, false, true>()));
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, false, has_entries>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, false, has_entries>()));
@@ -728,14 +744,15 @@ struct SkinnyLaunch {
     const GemmArgs &g;
     hipStream_t st;
     const GemmArgs *second = nullptr; // paired launch: the down projection behind the gate/up GEMM `g`
-    template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false>
+    template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool ONE = false>
     int go() {
-        if constexpr (PACKED && !MBLK && !KSPLIT) {
+        if constexpr (PACKED && !MBLK && !KSPLIT && !ONE) {
             if (g.ksplit) return go<Fmt, FACTORED, PACKED, MBLK, true>(); // validated by the launch functions
+            if (FACTORED && !second && std::min(g.tile_m, g.max_rows) <= kSkinnyRowBlock) return go<Fmt, FACTORED, PACKED, MBLK, false, FACTORED>();
         }
-        auto kern = qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT>;
-        const size_t lds = skinny_lds_bytes(g.b0) + (MBLK ? kSkinnyTurnBytes : 0);
-        DMOE_TRY((skinny_raise_limit<Fmt, FACTORED, PACKED, MBLK, KSPLIT>())); // done by dmoe_init for its device; a flag test otherwise
+        auto kern = qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, ONE>;
+        const size_t lds = skinny_lds_bytes(g.b0) + (MBLK ? kSkinnyMblkBytes : 0);
+        DMOE_TRY((skinny_raise_limit<Fmt, FACTORED, PACKED, MBLK, KSPLIT, ONE>())); // done by dmoe_init for its device; a flag test otherwise
         // 8 wavefronts per workgroup: 128 output columns of gate AND up, or 256 of a single projection
         auto blocks_x = [](const GemmArgs &a) { return ceil_div((a.ksplit ? 2 : 1) * a.b0.rows, (a.gate_up ? 1 : 2) * kSkinnyWaves * 32); };
         dim3 block(2 * kSkinnyWaves * 64);
@@ -743,7 +760,7 @@ struct SkinnyLaunch {
             GemmArgs a = g, b = *second;
             a.tile_done_target = b.tile_done_target = (uint32_t)blocks_x(g);
             b.tile_done = a.tile_done;
-            const size_t lds2 = std::max(lds, skinny_lds_bytes(second->b0) + (MBLK ? kSkinnyTurnBytes : 0));
+            const size_t lds2 = std::max(lds, skinny_lds_bytes(second->b0) + (MBLK ? kSkinnyMblkBytes : 0));
             dim3 grid((unsigned)std::max(blocks_x(a), blocks_x(b)), (unsigned)(2 * g.max_tiles));
             hipLaunchKernelGGL(kern, grid, block, lds2, st, a, b, 1);
         } else {
