@@ -156,28 +156,68 @@ __device__ __forceinline__ void place_row(const PackOut &o, uint32_t pos, uint32
     if (o.sorted_e) o.sorted_e[pos] = e;
 }
 
-// ---- one launch, n <= 1024 * GROUPS --------------------------------------------------------------------------
-// One workgroup; wavefront w packs the `groups` (<= GROUPS) groups of 64 rows from row w * groups * 64 on, with the ids in
+// ---- one launch, n <= 1024 ---------------------------------------------------------------------------------
+// `e` = this thread's expert id (row i = tid), `pack_sm` = hist[kPackWaves][E] in LDS
+__device__ __forceinline__ void pack_fused_body(const PackOut &o, uint32_t e, bool active, uint32_t n, int K, int E,
+                                                int tile_m, uint32_t *pack_sm, uint32_t *scan_sm) {
+    const int tid = (int)threadIdx.x, lane = lane_id(), wave = tid >> 6;
+    for (int i = tid; i < kPackWaves * E; i += kPackThreads) pack_sm[i] = 0;
+    __syncthreads();
+    if (active && e >= (uint32_t)E) { // a corrupt id: stay in bounds, and tell the host
+        if (o.bad_ids) atomicAdd(o.bad_ids, 1u);
+        e = (uint32_t)E - 1;
+    }
+    if (active) atomicAdd(&pack_sm[wave * E + e], 1u);
+    __syncthreads();
+    uint32_t count = 0;
+    if (tid < E) {
+        for (int w = 0; w < kPackWaves; ++w) {
+            uint32_t c = pack_sm[w * E + tid];
+            pack_sm[w * E + tid] = count;
+            count += c;
+        }
+    }
+    uint32_t off = emit_segments(count, tid, E, n, tile_m, o, scan_sm);
+    if (tid < E)
+        for (int w = 0; w < kPackWaves; ++w) pack_sm[w * E + tid] += off;
+    __syncthreads();
+    uint64_t peers = match_expert(e, active, log2_ceil(E));
+    if (active) {
+        uint32_t rank = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
+        place_row(o, pack_sm[wave * E + e] + rank, (uint32_t)tid, e, K);
+    }
+}
+
+__global__ __launch_bounds__(kPackThreads) void pack_fused_kernel(PackOut o, const uint32_t *__restrict__ idx,
+                                                                  uint32_t n, int K, int E, int tile_m) {
+    extern __shared__ uint32_t pack_sm[]; // hist[kPackWaves][E]
+    __shared__ uint32_t scan_sm[4 * kPackWaves];
+    const bool active = threadIdx.x < n;
+    const uint32_t e = active ? packed_id(o, idx[threadIdx.x]) : 0u;
+    pack_fused_body(o, e, active, n, K, E, tile_m, pack_sm, scan_sm);
+}
+
+// ---- one launch, n <= 1024 * kPackGroups --------------------------------------------------------------------------
+// One workgroup; wavefront w packs the `groups` (<= kPackGroups) groups of 64 rows from row w * groups * 64 on, with the ids in
 // registers in between. One compute unit does all of it, so the time grows with the rows (us in a layer step, this kernel | the three
 // launches below, which also have two boundaries between them): 3054 rows 11.7 | 20.2, 9186 rows 24.4 | 20.2.
-template <int GROUPS>
-__global__ __launch_bounds__(kPackThreads) void pack_fused_kernel(PackOut o, const uint32_t *__restrict__ idx,
-                                                                  uint32_t n, int K, int E, int tile_m, int groups_) {
+// (Also for one group it would do, but takes 0.3 us longer than the kernel above.)
+__global__ __launch_bounds__(kPackThreads) void pack_groups_kernel(PackOut o, const uint32_t *__restrict__ idx,
+                                                                   uint32_t n, int K, int E, int tile_m, int groups) {
     extern __shared__ uint32_t pack_sm[]; // hist[kPackWaves][E]
     __shared__ uint32_t scan_sm[4 * kPackWaves];
     const int tid = (int)threadIdx.x, lane = lane_id(), wave = tid >> 6;
-    const int groups = GROUPS == 1 ? 1 : groups_;
     const uint32_t row0 = (uint32_t)(wave * groups * 64 + lane);
-    uint32_t ids[GROUPS];
+    uint32_t ids[kPackGroups];
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
+    for (int g = 0; g < kPackGroups; ++g) {
         const uint32_t i = row0 + 64u * (uint32_t)g;
         ids[g] = g < groups && i < n ? packed_id(o, idx[i]) : 0u;
     }
     for (int i = tid; i < kPackWaves * E; i += kPackThreads) pack_sm[i] = 0;
     __syncthreads();
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
+    for (int g = 0; g < kPackGroups; ++g) {
         if (g >= groups || row0 + 64u * (uint32_t)g >= n) continue;
         if (ids[g] >= (uint32_t)E) { // a corrupt id: stay in bounds, and tell the host
             if (o.bad_ids) atomicAdd(o.bad_ids, 1u);
@@ -200,7 +240,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_fused_kernel(PackOut o, con
     __syncthreads();
     const int nbits = log2_ceil(E);
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
+    for (int g = 0; g < kPackGroups; ++g) {
         if (g >= groups) continue; // uniform
         const uint32_t i = row0 + 64u * (uint32_t)g;
         const bool active = i < n;
@@ -211,7 +251,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_fused_kernel(PackOut o, con
         const uint32_t pos = *next + rank;
         place_row(o, pos, i, ids[g], K);
         // the next group starts behind this one: the wavefront's own counters, whose operations complete in order
-        if (GROUPS > 1 && (peers >> lane) <= 1ull) *next = pos + 1u;
+        if ((peers >> lane) <= 1ull) *next = pos + 1u;
     }
 }
 
@@ -449,8 +489,10 @@ int launch_pack(const PackOut &o, const uint32_t *d_idx, size_t n, int K, int E,
     if (n <= (size_t)kPackThreads * kPackGroups) {
         const size_t lds = sizeof(uint32_t) * (size_t)kPackWaves * E;
         const int groups = (int)((n + kPackThreads - 1) / kPackThreads);
-        auto kern = groups == 1 ? pack_fused_kernel<1> : pack_fused_kernel<kPackGroups>;
-        hipLaunchKernelGGL(kern, dim3(1), dim3(kPackThreads), lds, st, o, d_idx, (uint32_t)n, K, E, tile_m, groups);
+        if (groups == 1)
+            hipLaunchKernelGGL(pack_fused_kernel, dim3(1), dim3(kPackThreads), lds, st, o, d_idx, (uint32_t)n, K, E, tile_m);
+        else
+            hipLaunchKernelGGL(pack_groups_kernel, dim3(1), dim3(kPackThreads), lds, st, o, d_idx, (uint32_t)n, K, E, tile_m, groups);
         DMOE_LAUNCH_CHECK();
         return DMOE_OK;
     }
