@@ -257,6 +257,8 @@ struct GemmArgs {
 };
 // tile_m the kernels were built for
 constexpr int kSkinnyTileM = 32;          // most rows a skinny tile can hold (see qgemm_skinny_tile_m)
+// Workgroups of the weight-streaming kernel up to which a launch leaves the chip half empty (one per compute unit, where two fit)
+constexpr int kSkinnyFewGroups = 256;
 constexpr int kSkinnyDenseTileM = 8;      // dense (one matrix) launches: small tiles, many workgroups per row block
 constexpr int kMfmaTileM = 128;
 constexpr int kMfmaWideTileM = 128;

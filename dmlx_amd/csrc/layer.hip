@@ -180,12 +180,11 @@ __global__ void combine_kernel(uint16_t *__restrict__ out, const uint16_t *__res
 // the weight-streaming kernel gives 4.1 / 4.0 against the matrix-core kernel's 3.5 / 3.6 (4-bit affine), 4.5 / 4.3 against
 // 4.4 / 4.3 (MXFP4), 5.3 / 5.3 against 5.2 / 5.2 (8-bit); at 24 and 32 rows the matrix-core kernel is level or ahead.
 constexpr int kSkinnyAvgRows = 16;
-// Workgroups of the weight-streaming kernel up to which a launch leaves the chip half empty (one per compute unit, where two
-// fit). It is then bound by each workgroup's own chain of memory round trips, not by bandwidth: tiles are cut to one row
-// block (no restaging of the activations on the way; an expert's second tile finds the weights in L2; the sums, and so the
-// bits, are the same). 8 experts top-2, hidden 1024, ffn 2048, 4-bit: 16 / 32 tokens 39.9 / 42.1 -> 32.3 / 34.3 us per step;
-// hidden 4096: 32 tokens 62.2 -> 53.3 us; one projection [8, 1408, 2048] on 64 rows, 4-bit / MXFP4: 24.5 / 21.9 -> 19.1 / 17.7.
-constexpr int kSkinnyFewGroups = 256;
+// A launch of at most kSkinnyFewGroups workgroups is bound by each workgroup's own chain of memory round trips, not by
+// bandwidth: tiles are cut to one row block (no restaging of the activations on the way; an expert's second tile finds the
+// weights in L2; the sums, and so the bits, are the same). 8 experts top-2, hidden 1024, ffn 2048, 4-bit: 16 / 32 tokens 39.9 /
+// 42.1 -> 32.3 / 34.3 us per step; hidden 4096: 32 tokens 62.2 -> 53.3 us; one projection [8, 1408, 2048] on 64 rows, 4-bit /
+// MXFP4: 24.5 / 21.9 -> 19.1 / 17.7.
 // Sorted rows up to which each tile's reduction is also split over two workgroups (GemmArgs::ksplit). The split adds two
 // halves where the other kernels sum left to right, so it stays with single tokens: a token's bits above this line do not
 // depend on the batch it is in. (Up to 64 rows it would save 2 us of 32 on the small layer and 10 of 50 at hidden 4096.)

@@ -97,7 +97,7 @@ constexpr size_t kSkinnyStageOffset = 16384, kSkinnyStageBytes = (size_t)kSkinny
 // MBLK (MLX layout only): the scale / bias entries of a row are not fetched one per step (32 cache lines touched per
 // load for 2 useful bytes each, again at every step: these loads, not the weights, bounded the MLX-layout path) but 16
 // bytes at a time - eight bf16 or sixteen E8M0 entries, the next block requested while the current one is in use.
-template <typename Fmt, bool FACTORED, bool PACKED, int RJT, bool MBLK, bool KSPLIT = false, bool ZEROS = FACTORED>
+template <typename Fmt, bool FACTORED, bool PACKED, int RJT, bool MBLK, bool KSPLIT = false, bool FEW = false>
 __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, uint8_t *skinny_lds, const bool gate_up,
                                             const int sync, const uint32_t slot) {
     using CS = ChunkStream<Fmt, PACKED>;
@@ -128,6 +128,14 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     constexpr int ROUND = MBLK && STAGES < 8 ? 8 : STAGES;  // steps per unrolled round (MBLK: whole blocks of entries)
     static_assert(ROUND % STAGES == 0 && (!MBLK || ROUND % 8 == 0), "rounds are whole turns of the ring");
     constexpr int NM = 1;                           // projections per wavefront
+    constexpr bool ZEROS = FACTORED && !KSPLIT && !FEW; // see skinny_zero_bytes
+    // Launches of a few workgroups are paced by each wavefront's own chain of steps, and the look-ahead has to be in the machine
+    // code: left alone, the scheduler gathers the loads of a round behind its fourth step and waits for nearly all of them at
+    // the next one's start, where in the round depending on what surrounds it. Each step's loads are pinned to its head (small
+    // layer, 16 tokens 34.5 -> 33.0 us; hidden 4096, 1 / 2 tokens: 4-bit 34.8 / 49.2 -> 32.9 / 47.6, MXFP4 34.0 / 47.2 -> 31.3 / 44.1,
+    // 8-bit 45.6 / 78.3 -> 44.7 / 69.9). Not where the launch fills the chip: there a wavefront's gathered loads are no loss (24 to
+    // 64 tokens, 4-bit: pinned 0 to 2 % slower), and not on unquantized weights (32 instructions per round, level).
+    constexpr bool PIN = (KSPLIT || FEW) && KV > 8;
     constexpr int WAVES = 2 * kSkinnyWaves;         // eight wavefronts share one staging of the tile's activations
     const int cg = gate_up ? kSkinnyWaves : WAVES;  // 32-row blocks of weight rows per workgroup
     const int tid = (int)threadIdx.x, lane = tid & 63, ln = lane & 31, h = lane >> 5;
@@ -496,6 +504,10 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
                     continue;
                 }
                 load_stage(LEAN_TAIL || ahead < n_loc ? ahead : n_loc - 1, ring[(j + PRE) % STAGES]);
+                if (PIN) {
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 consume(step, j & 7, step - x0, xround + j * KSTEP * 2, ring[j % STAGES]);
             }
         }
@@ -616,9 +628,9 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
 // y < a.max_tiles are the gate/up tiles, the next a.max_tiles the down tiles of the same list. The hardware starts
 // workgroups in index order, so every producer of a tile is running or done by the time a consumer of it starts to
 // wait; the down workgroups that become resident while the last gate/up workgroups drain stream their weights meanwhile.
-// ONE: launches of a few workgroups (single launches of tiles of at most one row block). They are paced by each workgroup's own
-// chain, not by power, and read their code cold: no zeros, no copies for larger tiles (small layer, 16 tokens: 36.3 -> 34.7 us).
-template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool ONE = false>
+// FEW: a single launch of at most kSkinnyFewGroups workgroups and of tiles of one row block. It is paced by each workgroup's own
+// chain, not by bandwidth or power: the ring's loads are pinned (see PIN), no zeros, no copies for larger tiles.
+template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool FEW = false>
 __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(GemmArgs a, GemmArgs b, int paired) {
     extern __shared__ __attribute__((aligned(16))) uint8_t skinny_lds[];
     const bool second = paired && blockIdx.y >= (uint32_t)a.max_tiles; // workgroup-uniform
@@ -648,8 +660,8 @@ __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(Gem
         uint32_t left = (uint32_t)g.dense_rows - t.row0;
         t.nrows = left < (uint32_t)g.tile_m ? left : (uint32_t)g.tile_m;
     }
-    if (KSPLIT || ONE) { // the launcher builds no tile above one row block for these kernels
-        skinny_tile<Fmt, FACTORED, PACKED, 1, MBLK, KSPLIT, false>(g, t, skinny_lds, g.gate_up, sync, slot);
+    if (KSPLIT || FEW) { // the launcher builds no tile above one row block for these kernels
+        skinny_tile<Fmt, FACTORED, PACKED, 1, MBLK, KSPLIT, FEW>(g, t, skinny_lds, g.gate_up, sync, slot);
         return;
     }
     if (__builtin_amdgcn_readfirstlane((int)t.nrows) <= kSkinnyRowBlock)
@@ -711,10 +723,10 @@ static bool mlx_meta_blocks(const QView &b) {
            (!b.biases || ((uintptr_t)b.biases % 16) == 0);
 }
 
-template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK, bool KSPLIT = false, bool ONE = false>
+template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK, bool KSPLIT = false, bool FEW = false>
 static int skinny_raise_limit() {
     static LdsLimit limit; // per instantiation
-    return raise_lds_limit(limit, (const void *)qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, ONE>, (int)kSkinnyMaxLds + 1024);
+    return raise_lds_limit(limit, (const void *)qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>, (int)kSkinnyMaxLds + 1024);
 }
 // the instantiations SkinnyLaunch can pick for one format
 template <typename Fmt>
@@ -724,7 +736,8 @@ static int skinny_prepare_format() {
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, true, false>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, true, false>()));
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, true, false, true>()));
-    DMOE_TRY((skinny_raise_limit<Fmt, can_factor, true, false, false, can_factor>()));
+    DMOE_TRY((skinny_raise_limit<Fmt, can_factor, true, false, false, true>()));
+    DMOE_TRY((skinny_raise_limit<Fmt, false, true, false, false, true>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, true, false, true>()));
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, false, has_entries>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, false, has_entries>()));
@@ -744,17 +757,20 @@ struct SkinnyLaunch {
     const GemmArgs &g;
     hipStream_t st;
     const GemmArgs *second = nullptr; // paired launch: the down projection behind the gate/up GEMM `g`
-    template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool ONE = false>
+    template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool FEW = false>
     int go() {
-        if constexpr (PACKED && !MBLK && !KSPLIT && !ONE) {
-            if (g.ksplit) return go<Fmt, FACTORED, PACKED, MBLK, true>(); // validated by the launch functions
-            if (FACTORED && !second && std::min(g.tile_m, g.max_rows) <= kSkinnyRowBlock) return go<Fmt, FACTORED, PACKED, MBLK, false, FACTORED>();
-        }
-        auto kern = qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, ONE>;
-        const size_t lds = skinny_lds_bytes(g.b0) + (MBLK ? kSkinnyMblkBytes : 0);
-        DMOE_TRY((skinny_raise_limit<Fmt, FACTORED, PACKED, MBLK, KSPLIT, ONE>())); // done by dmoe_init for its device; a flag test otherwise
         // 8 wavefronts per workgroup: 128 output columns of gate AND up, or 256 of a single projection
         auto blocks_x = [](const GemmArgs &a) { return ceil_div((a.ksplit ? 2 : 1) * a.b0.rows, (a.gate_up ? 1 : 2) * kSkinnyWaves * 32); };
+        if constexpr (PACKED && !MBLK && !KSPLIT && !FEW) {
+            if (g.ksplit) return go<Fmt, FACTORED, PACKED, MBLK, true>(); // validated by the launch functions
+            if constexpr (Fmt::kVals > 8) // (unquantized weights: nothing to pin, see PIN)
+                if (!second && std::min(g.tile_m, g.max_rows) <= kSkinnyRowBlock &&
+                    (size_t)blocks_x(g) * (size_t)g.max_tiles <= (size_t)kSkinnyFewGroups)
+                    return go<Fmt, FACTORED, PACKED, MBLK, false, true>();
+        }
+        auto kern = qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>;
+        const size_t lds = skinny_lds_bytes(g.b0) + (MBLK ? kSkinnyMblkBytes : 0);
+        DMOE_TRY((skinny_raise_limit<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>())); // done by dmoe_init for its device; a flag test otherwise
         dim3 block(2 * kSkinnyWaves * 64);
         if (second) {
             GemmArgs a = g, b = *second;
