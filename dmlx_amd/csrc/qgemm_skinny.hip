@@ -78,7 +78,7 @@ struct SkinnyStage {
 // reach g.tile_done_target before it reads its activations (the other role's output), its weight ring already in flight.
 constexpr int kSkinnySyncNone = 0, kSkinnySyncSignal = 1, kSkinnySyncWait = 2;
 
-// LDS: [activation window][sums of x per step][MBLK only: 4 KiB per wavefront for turning weight lines][zeros]
+// LDS: [activation window][sums of x per step][MBLK only: 4 KiB per wavefront for turning weight lines][zeros, where read]
 __host__ __device__ constexpr size_t skinny_turn_offset(int cols, int kstep) {
     return (size_t)kSkinnyRowBlock * (size_t)cols * 2 + (size_t)kSkinnyTileM * 16 +
            (size_t)(cols / kstep) * kSkinnyRowBlock * sizeof(float) + 128;
@@ -88,11 +88,24 @@ constexpr size_t kSkinnyTurnBytes = (size_t)2 * kSkinnyWaves * 4 * 1024;
 // tile's rows read zeros: the chip is power-limited under a decode step too, and multiplying zeros costs less of it than
 // multiplying row 0 again (steps of 64 / 509 tokens 244 / 813 -> 233 / 795 us). One round of the ring's worth of zeros serves
 // every step. The other formats gained 1 % on 64 tokens (MXFP4) and lost up to 5 % on a few (2 to 5 tokens).
+__host__ __device__ constexpr bool skinny_reads_zeros(bool factored, bool ksplit, bool few) { return factored && !ksplit && !few; }
 __host__ __device__ constexpr size_t skinny_zero_bytes(bool mblk) { return mblk ? 2048 : 1024; }
-constexpr size_t kSkinnyMaxLds = 151 * 1024;
-constexpr size_t kSkinnyMblkBytes = kSkinnyTurnBytes + skinny_zero_bytes(true) - skinny_zero_bytes(false); // on top, MBLK kernels
+constexpr size_t kSkinnyMaxLds = 150 * 1024; // without the zeros
 // where a tile's outputs are gathered before they are stored: behind the exchange areas of the epilogue (16 KiB)
 constexpr size_t kSkinnyStageOffset = 16384, kSkinnyStageBytes = (size_t)kSkinnyTileM * 256 * 2;
+// LDS of a launch, `zeros` = bytes of zeros its kernel reads. A two-row-block tile reads (and ignores) up to 24 floats past its
+// last step's sums: the 128 bytes in the offset. At least 32 KiB: once the main loop is done the wavefronts exchange their sums
+// through the start of the window (gate/up pairs: 4 KiB per row block of the tile, up to 16 KiB; split reduction: bytes 4096 ..
+// 8191) and gather the tile's outputs behind that (up to 32 rows of 256 columns), which a short reduction would not cover.
+constexpr size_t skinny_lds_bytes(int cols, int kstep, bool mblk, size_t zeros) {
+    const size_t window = skinny_turn_offset(cols, kstep) + (mblk ? 0 : zeros), least = kSkinnyStageOffset + kSkinnyStageBytes;
+    return (window > least ? window : least) + (mblk ? kSkinnyTurnBytes + zeros : 0);
+}
+// A kernel without zeros pays nothing for them: 8-bit reductions of 3072 keep three workgroups on a compute unit (160 KiB,
+// handed out in pieces of 1280 bytes) and those of 4768 two.
+constexpr size_t skinny_lds_share(size_t bytes) { return (bytes + 1279) / 1280 * 1280; }
+static_assert(3 * skinny_lds_share(skinny_lds_bytes(3072, 32, false, 0)) <= 160 * 1024 &&
+              2 * skinny_lds_share(skinny_lds_bytes(4768, 32, false, 0)) <= 160 * 1024, "workgroups per compute unit");
 
 // MBLK (MLX layout only): the scale / bias entries of a row are not fetched one per step (32 cache lines touched per
 // load for 2 useful bytes each, again at every step: these loads, not the weights, bounded the MLX-layout path) but 16
@@ -128,7 +141,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     constexpr int ROUND = MBLK && STAGES < 8 ? 8 : STAGES;  // steps per unrolled round (MBLK: whole blocks of entries)
     static_assert(ROUND % STAGES == 0 && (!MBLK || ROUND % 8 == 0), "rounds are whole turns of the ring");
     constexpr int NM = 1;                           // projections per wavefront
-    constexpr bool ZEROS = FACTORED && !KSPLIT && !FEW; // see skinny_zero_bytes
+    constexpr bool ZEROS = skinny_reads_zeros(FACTORED, KSPLIT, FEW);
     // Launches of a few workgroups are paced by each wavefront's own chain of steps, and the look-ahead has to be in the machine
     // code: left alone, the scheduler gathers the loads of a round behind its fourth step and waits for nearly all of them at
     // the next one's start, where in the round depending on what surrounds it. Each step's loads are pinned to its head (small
@@ -676,12 +689,8 @@ static int skinny_vals(const QView &b) {
     if (b.mode == DMOE_QUANT_NONE) return 8;
     return (b.mode == DMOE_QUANT_AFFINE && b.bits == 4) || b.mode == DMOE_QUANT_MXFP4 ? 32 : 16;
 }
-static size_t skinny_lds_bytes(const QView &b) {
-    // a two-row-block tile reads (and ignores) up to 24 floats past its last step's sums: the 128 bytes in the offset.
-    // At least 32 KiB: once the main loop is done the wavefronts exchange their sums through the start of the window
-    // (gate/up pairs: 4 KiB per row block of the tile, up to 16 KiB; split reduction: bytes 4096 .. 8191) and gather
-    // the tile's outputs behind that (up to 32 rows of 256 columns), which a short reduction dimension would not cover.
-    return std::max(skinny_turn_offset(b.cols, 2 * skinny_vals(b)) + skinny_zero_bytes(false), kSkinnyStageOffset + kSkinnyStageBytes);
+static size_t skinny_lds_bytes(const QView &b, bool mblk = false, size_t zeros = 0) {
+    return skinny_lds_bytes(b.cols, 2 * skinny_vals(b), mblk, zeros);
 }
 
 // Rows per tile to build tile lists with for this weight shape: a tile of 2 (4) row blocks splits the reduction
@@ -716,7 +725,7 @@ static bool mlx_meta_blocks(const QView &b) {
     // a block of entries must span exactly eight reduction steps (affine 4-bit: groups of 64; MXFP4: 32; 8-bit: 32)
     const int kstep = b.bits == 4 ? 64 : 32;
     if ((int)(16 / esz) * b.group != 8 * kstep) return false;
-    if (skinny_lds_bytes(b) + kSkinnyMblkBytes > kSkinnyMaxLds + 1024 || b.w_row % 128 != 0 || ((uintptr_t)b.w % 16) != 0 || b.w_mat % 16 != 0 ||
+    if (skinny_lds_bytes(b, true) > kSkinnyMaxLds || b.w_row % 128 != 0 || ((uintptr_t)b.w % 16) != 0 || b.w_mat % 16 != 0 ||
         (uint64_t)b.rows * (uint64_t)b.w_row >= (1ull << 32))
         return false; // the line-wise weight loads of the small tiles: LDS to turn them in, whole lines per group
     return row >= 16 && row % 16 == 0 && b.s_row % 16 == 0 && b.s_mat % 16 == 0 && ((uintptr_t)b.scales % 16) == 0 &&
@@ -726,7 +735,7 @@ static bool mlx_meta_blocks(const QView &b) {
 template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK, bool KSPLIT = false, bool FEW = false>
 static int skinny_raise_limit() {
     static LdsLimit limit; // per instantiation
-    return raise_lds_limit(limit, (const void *)qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>, (int)kSkinnyMaxLds + 1024);
+    return raise_lds_limit(limit, (const void *)qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>, (int)(kSkinnyMaxLds + skinny_zero_bytes(true)));
 }
 // the instantiations SkinnyLaunch can pick for one format
 template <typename Fmt>
@@ -769,14 +778,15 @@ struct SkinnyLaunch {
                     return go<Fmt, FACTORED, PACKED, MBLK, false, true>();
         }
         auto kern = qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>;
-        const size_t lds = skinny_lds_bytes(g.b0) + (MBLK ? kSkinnyMblkBytes : 0);
+        constexpr size_t zeros = skinny_reads_zeros(FACTORED, KSPLIT, FEW) ? skinny_zero_bytes(MBLK) : 0;
+        const size_t lds = skinny_lds_bytes(g.b0, MBLK, zeros);
         DMOE_TRY((skinny_raise_limit<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>())); // done by dmoe_init for its device; a flag test otherwise
         dim3 block(2 * kSkinnyWaves * 64);
         if (second) {
             GemmArgs a = g, b = *second;
             a.tile_done_target = b.tile_done_target = (uint32_t)blocks_x(g);
             b.tile_done = a.tile_done;
-            const size_t lds2 = std::max(lds, skinny_lds_bytes(second->b0) + (MBLK ? kSkinnyMblkBytes : 0));
+            const size_t lds2 = std::max(lds, skinny_lds_bytes(second->b0, MBLK, zeros));
             dim3 grid((unsigned)std::max(blocks_x(a), blocks_x(b)), (unsigned)(2 * g.max_tiles));
             hipLaunchKernelGGL(kern, grid, block, lds2, st, a, b, 1);
         } else {
