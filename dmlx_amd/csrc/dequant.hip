@@ -98,7 +98,14 @@ __global__ void dequant_kernel(uint16_t *__restrict__ out, QView q, int mat) {
 }
 
 // The same matrix through the decoder that the matrix-core kernels run in registers (pair_meta / decode_pair), for
-// tests that compare it bit for bit with decode().
+// tests that compare it bit for bit with decode(). It takes its scale in two forms, from the entries of the checkpoint layout
+// (qgemm_ring.hip) and from the words of the packed one (qgemm_wide.hip), and both are run: a value on which they disagree
+// comes out as kFormsDisagree, unless both are NaN.
+constexpr uint32_t kFormsDisagree = 0x0badu;
+__device__ __forceinline__ uint32_t agreed_bf16(uint32_t a, uint32_t b) {
+    const bool both_nan = (a & 0x7fffu) > 0x7f80u && (b & 0x7fffu) > 0x7f80u;
+    return a == b || both_nan ? a : kFormsDisagree;
+}
 template <typename Fmt>
 __global__ void dequant_fused_kernel(uint16_t *__restrict__ out, QView q, int mat) {
     const int chunks_per_row = q.cols / Fmt::kVals;
@@ -112,12 +119,18 @@ __global__ void dequant_fused_kernel(uint16_t *__restrict__ out, QView q, int ma
     uint4 raw = *(const uint4 *)(wrow + (size_t)c * 16);
     uint32_t sb[2];
     Fmt::load_meta_raw(q, srow, brow, k0, sb);
+    const Meta m = Fmt::pair_meta(Fmt::meta_from_raw(sb));
     if (Fmt::kMetaEntryBytes == 2) sb[0] |= sb[1] << 16; // the word of the packed layout
-    const Meta m = Fmt::pair_meta(Fmt::meta_from_packed(sb));
-    uint32_t pairs[Fmt::kVals / 2], st[Fmt::kPairState] = {};
+    const Meta mp = Fmt::pair_meta(Fmt::meta_from_packed(sb));
+    uint32_t pairs[Fmt::kVals / 2], packed[Fmt::kVals / 2], st[Fmt::kPairState] = {}, stp[Fmt::kPairState] = {};
     Fmt::pair_state(st);
+    Fmt::pair_state(stp);
 #pragma unroll
-    for (int p = 0; p < Fmt::kVals / 2; ++p) Fmt::decode_pair(raw, m, p, pairs, st);
+    for (int p = 0; p < Fmt::kVals / 2; ++p) {
+        Fmt::decode_pair(raw, m, p, pairs, st);
+        Fmt::decode_pair(raw, mp, p, packed, stp);
+        pairs[p] = agreed_bf16(pairs[p] & 0xffffu, packed[p] & 0xffffu) | agreed_bf16(pairs[p] >> 16, packed[p] >> 16) << 16;
+    }
     if (Fmt::kRowScale) {
         float rs = *(const float *)srow;
 #pragma unroll

@@ -462,7 +462,8 @@ int dmoe_debug_last_activations(uint16_t *d_out, dmoe_layer layer, int T, dmoe_w
 
 /* dmoe_dequantize through the decoder that the prefill kernels run in registers between their matrix instructions
  * (same arguments, same result layout). For parity tests: the fused decode must give the bits of dmoe_dequantize,
- * i.e. of mlx_dequantize as called at deepseek_v4_loader.zig:129, for every scale and bias. */
+ * i.e. of mlx_dequantize as called at deepseek_v4_loader.zig:129, for every scale and bias. Decodes with the scales in the
+ * form of the checkpoint layout and in that of the packed one; a value on which the two differ comes out as 0x0bad. */
 int dmoe_debug_dequantize_fused(uint16_t *d_out, const dmoe_qweight *qw, int mat_index, dmoe_stream s);
 
 /* Calibration for the benchmark (no counterpart in the reference): ONE launch of a loop of bf16 matrix instructions
