@@ -254,6 +254,7 @@ struct GemmArgs {
     uint32_t row_scale_rows = 0xffffffffu; // row_scale applies to sorted rows below this
     const uint32_t *n_live = nullptr; // nullable: experts with rows, for the wide kernel's choice of a tile map
     int stream_weights = 0;           // wide kernel, set by its launcher: see kWideStreamBytes
+    int dense_tiles = 0;              // of the tile list: the always-on expert's, which n_live does not count
 };
 // tile_m the kernels were built for
 constexpr int kSkinnyTileM = 32;          // most rows a skinny tile can hold (see qgemm_skinny_tile_m)

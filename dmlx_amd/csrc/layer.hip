@@ -405,6 +405,7 @@ static int routed_forward(const Layer *L, Workspace *w, const FwdLayout &f, cons
     gu.tiles = po.tiles;
     gu.n_tiles = po.n_tiles;
     gu.n_live = po.n_live;
+    gu.dense_tiles = f.fold ? ceil_div(T, f.tile_m) : 0;
     gu.max_tiles = f.max_tiles;
     gu.tile_m = f.tile_m;
     gu.ksplit = f.ksplit ? 1 : 0;
@@ -424,6 +425,7 @@ static int routed_forward(const Layer *L, Workspace *w, const FwdLayout &f, cons
     dn.tiles = po.tiles;
     dn.n_tiles = po.n_tiles;
     dn.n_live = po.n_live;
+    dn.dense_tiles = gu.dense_tiles;
     dn.max_tiles = f.max_tiles;
     dn.tile_m = f.tile_m;
     dn.ksplit = f.ksplit ? 1 : 0;

@@ -348,6 +348,14 @@ __host__ __device__ constexpr uint32_t wide_run() {
     return Fmt::kVals == 8 ? 4u : 1u;
 }
 
+// Experts of several tiles: an eighth more tiles than live experts. The dense tiles of a shared expert in the list count on
+// neither side, so that the choice is the routing's alone.
+__host__ __device__ constexpr bool wide_several_tiles(uint32_t tiles, uint32_t dense_tiles, uint32_t live) {
+    return 8u * (tiles - dense_tiles) >= 9u * live;
+}
+static_assert(!wide_several_tiles(64, 0, 64) && !wide_several_tiles(64 + 8, 8, 64) && wide_several_tiles(72, 0, 64) && wide_several_tiles(72 + 64, 64, 64),
+              "the same choice with and without a shared expert in the list");
+
 template <typename Fmt, bool GATE_UP>
 __global__ __launch_bounds__(kWideWaves * 64, 2) void qgemm_wide_kernel(GemmArgs g) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t wide_lds[]; // [slots][rows of the tile][128 bytes], swizzled
@@ -367,7 +375,7 @@ __global__ __launch_bounds__(kWideWaves * 64, 2) void qgemm_wide_kernel(GemmArgs
     if (g.tiles) {
         n_slots = *g.n_tiles;
         if (g.n_live) {
-            const bool shared = 8u * n_slots >= 9u * *g.n_live; // experts of several tiles
+            const bool shared = wide_several_tiles(n_slots, (uint32_t)g.dense_tiles, *g.n_live);
             run = shared ? RUN : 1u;
             stream = g.stream_weights && !shared;
         }
