@@ -886,7 +886,7 @@ static int gather_qmm_view(uint16_t *d_out, const uint16_t *d_x, const QView &v,
     const int max_tiles = pack_max_tiles((size_t)R, v.n_mats, tile_m);
     Bump b;
     size_t o_order = b.take((size_t)R * 4), o_arows = b.take((size_t)R * 4);
-    size_t o_tiles = b.take((size_t)max_tiles * sizeof(Tile)), o_nt = b.take(4), o_nl = b.take(4);
+    size_t o_tiles = b.take((size_t)max_tiles * sizeof(Tile)), o_nt = b.take(8), o_nl = o_nt + 4;
     size_t o_scr = b.take(pack_scratch_bytes((size_t)R, v.n_mats));
     Workspace *w = nullptr;
     DMOE_TRY(workspace_reserve(ws, b.off, &w));
