@@ -107,10 +107,10 @@ def test_decode_step_reports_a_wait_that_gave_up(dmoe, ws):
 
 def test_pack_reports_expert_ids_out_of_range(dmoe, ws):
     """An expert id >= E is packed under the last expert (every access stays in bounds) and the workspace check
-    reports it once, for the one-launch and the three-launch packing kernels."""
+    reports it once, for the one-launch kernels (one and several groups of rows per wavefront) and the three launches."""
     from dmlx_amd.capi import DmoeError
     E, K = 16, 2
-    for T in (64, 2000):
+    for T in (64, 2000, 3000):
         idx = torch.randint(0, E, (T, K), dtype=torch.int32, device="cuda")
         dmoe.pack(idx, E, ws)
         ws.check()
