@@ -70,6 +70,7 @@ struct Workspace {
     hipEvent_t fork = nullptr, join = nullptr;
     hipEvent_t packed = nullptr, small_done = nullptr; // prefill: the small tiles' GEMMs run on the side stream
     bool last_with_shared = true; // layout of the last forward on this workspace (for dmoe_debug_last_activations)
+    bool last_ordered = false;    // its gate/up outputs are in code order (GemmArgs::out_sums)
     // Device words that outlive workspace growth, read and cleared by dmoe_workspace_check: [0] counts waits inside a
     // paired GEMM launch that gave up (see GemmArgs::wait_expired), [1] counts expert ids outside [0, E) met by the
     // pack kernels (see PackOut::bad_ids).
@@ -169,6 +170,12 @@ struct PackOut {
     // table maps to slot 0 like an expert that is not loaded)
     const int32_t *remap = nullptr;
     uint32_t n_remap = 0;
+    // Optional: the activations in code order with their sums (see GemmArgs::a_sums), made by further workgroups of the same
+    // launch while the first one packs. rows_pieces = 16-byte pieces of `rows_in`, a multiple of 8 (rows of whole 64s).
+    const uint4 *rows_in = nullptr;
+    uint4 *rows_out = nullptr;
+    float *rows_sums = nullptr;
+    uint32_t rows_pieces = 0;
 };
 
 inline int pack_max_tiles(size_t n, int E, int tile_m) {
@@ -255,6 +262,11 @@ struct GemmArgs {
     const uint32_t *n_live = nullptr; // nullable: experts with rows, for the wide kernel's choice of a tile map
     int stream_weights = 0;           // wide kernel, set by its launcher: see kWideStreamBytes
     int dense_tiles = 0;              // of the tile list: the always-on expert's, which n_live does not count
+    // Weight-streaming kernel, factored 4-bit form (see skinny_factored). `a_sums` set: the rows of `a` are in code order (the
+    // 16-byte piece x0..x7 as x0,x4,x1,x5,x2,x6,x3,x7), and a_sums[row][cols / 64] holds the sum of each 64 of their values.
+    // `out_sums` set (gate/up role): the outputs leave in that form, the sums here.
+    const float *a_sums = nullptr;
+    float *out_sums = nullptr;
 };
 // tile_m the kernels were built for
 constexpr int kSkinnyTileM = 32;          // most rows a skinny tile can hold (see qgemm_skinny_tile_m)
@@ -266,6 +278,7 @@ constexpr int kMfmaWideTileM = 128;
 int launch_qgemm_skinny(const GemmArgs &g, hipStream_t st);
 // gate/up + down of one tile list in one launch (down waits per tile for gate/up); gu.tile_done must be zeroed
 bool qgemm_skinny_pair_supports(const GemmArgs &gu, const GemmArgs &dn);
+bool qgemm_skinny_factored(const QView &b); // 4-bit affine, groups of 64 and more: the form that reads GemmArgs::a_sums
 int launch_qgemm_skinny_pair(const GemmArgs &gu, const GemmArgs &dn, hipStream_t st);
 int launch_qgemm_mfma(const GemmArgs &g, hipStream_t st); // picks the wide kernel when the format allows it
 int launch_qgemm_wide(const GemmArgs &g, hipStream_t st);
@@ -312,6 +325,33 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
 __device__ __forceinline__ float round_bf16(float f) { return bf16_bits_to_f32(f32_to_bf16_bits(f)); }
 
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63u); }
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float x) {
+    const int v = __float_as_int(x);
+    return __int_as_float(__builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false));
+}
+// Code order of a 16-byte piece of eight bf16 (x0..x7): x0,x4,x1,x5,x2,x6,x3,x7, the order in which the factored 4-bit form
+// leaves a word's codes. The sum of 64 values has one order of additions wherever it is formed: pairs, left to right within a
+// piece, then a tree over the eight pieces (eight neighbouring lanes; every one of them ends up with the sum).
+__device__ __forceinline__ uint4 to_code_order(const uint4 &v) {
+    return make_uint4((v.x & 0xffffu) | (v.z << 16), (v.x >> 16) | (v.z & 0xffff0000u), (v.y & 0xffffu) | (v.w << 16),
+                      (v.y >> 16) | (v.w & 0xffff0000u));
+}
+__device__ __forceinline__ uint4 from_code_order(const uint4 &v) {
+    return make_uint4((v.x & 0xffffu) | (v.y << 16), (v.z & 0xffffu) | (v.w << 16), (v.x >> 16) | (v.y & 0xffff0000u),
+                      (v.z >> 16) | (v.w & 0xffff0000u));
+}
+__device__ __forceinline__ float sum64_of_code_order(const uint4 &v) {
+    float sum = (bf16_bits_to_f32(v.x & 0xffffu) + bf16_bits_to_f32(v.y & 0xffffu)) +
+                (bf16_bits_to_f32(v.z & 0xffffu) + bf16_bits_to_f32(v.w & 0xffffu)) +
+                (bf16_bits_to_f32(v.x >> 16) + bf16_bits_to_f32(v.y >> 16)) +
+                (bf16_bits_to_f32(v.z >> 16) + bf16_bits_to_f32(v.w >> 16));
+    sum += dpp_f32<0xB1>(sum);  // lane ^ 1 (quad_perm 1,0,3,2)
+    sum += dpp_f32<0x4E>(sum);  // lane ^ 2 (quad_perm 2,3,0,1)
+    sum += dpp_f32<0x141>(sum); // the other quad of the eight lanes (row_half_mirror)
+    return sum;
+}
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -128,13 +128,13 @@ __global__ void compose_rows_kernel(uint32_t *__restrict__ out, const uint32_t *
     if (i < n) out[i] = lhs[order[i]];
 }
 
-// out[dst[p], :] = in[p, :], 16 bytes per thread
+// out[dst[p], :] = in[p, :], 16 bytes per thread; `code_order`: the pieces of `in` are, those of `out` are not
 __global__ void scatter_rows_kernel(uint4 *__restrict__ out, const uint4 *__restrict__ in,
-                                    const uint32_t *__restrict__ dst, size_t row_vecs, size_t total) {
+                                    const uint32_t *__restrict__ dst, size_t row_vecs, size_t total, int code_order) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= total) return;
     size_t p = i / row_vecs, c = i - p * row_vecs;
-    out[(size_t)dst[p] * row_vecs + c] = in[i];
+    out[(size_t)dst[p] * row_vecs + c] = code_order ? from_code_order(in[i]) : in[i];
 }
 
 // out[t, :] = sum_k (w ? w[t,k] : 1) * y[t*K+k, :] + (shared ? shared[t, :] : 0); 8 columns per thread
@@ -193,6 +193,7 @@ constexpr int kSplitTileM = 8;
 #define DMOE_PAIR_MIN_ROWS 64
 #endif
 constexpr int kPairMinRows = DMOE_PAIR_MIN_ROWS; // decode steps above this many sorted rows run gate/up and down in one launch
+constexpr int kOrderedAvgRows = 4; // rows per expert from which a paired launch's rows go through code order (FwdLayout::ordered)
 constexpr int kSharedSkinnyRows = 64;
 
 static bool few_rows(size_t rows, int n_experts) { return rows <= (size_t)kSkinnyAvgRows * (size_t)n_experts; }
@@ -228,9 +229,17 @@ static bool layer_small_path(const Layer *L, size_t rows) {
 
 struct FwdLayout {
     size_t order, inv, token, sorted_e, counts, offsets, live, n_live, tiles, n_tiles, tile_done, scratch;
-    size_t h, y, sh_h, sh_y, total;
+    size_t h, y, sh_h, sh_y, xo, xs, hs, total;
     int max_tiles, tile_m;
     bool small;
+    // Paired launch of 4-bit affine weights whose scales are factored out: the rows of both roles come in code order with their
+    // sums (GemmArgs::a_sums), x from the packing launch's idle compute units (`xo`, `xs`), h from the gate/up role (`hs`).
+    // Otherwise every workgroup re-orders the rows in its LDS (a token's x 96 times over, with 16 strips and 6 experts): a pass of
+    // 40 vector instructions per 16 bytes, which the larger tiles pay for at every span. 256 experts, us per step re-ordered in
+    // LDS | in code order: 509 tokens 811 | 792, 600 at hidden 3072 640 | 624, 200 tokens (4.7 rows per expert) 372 | 369; but 64
+    // tokens (1.5 rows) 256 | 258, hence kOrderedAvgRows. gather_qmm, where a row of x serves one projection only, stays with
+    // LDS: 200 / 600 tokens on checkpoint arrays 211.5 / 367.6 | 213.0 / 365.0.
+    bool ordered;
     bool ksplit; // at most kSplitTileM sorted rows: the weight-streaming kernel splits each tile's reduction in two
     bool fold; // the shared expert rides in the routed launches: T more sorted rows behind the T*K routed ones
 };
@@ -283,7 +292,7 @@ static bool fold_prefill(const Layer *L, int T) {
     return routed + (size_t)ceil_div(T, kMfmaTileM) * strips <= 256 || (bf16 && routed >= 1024);
 }
 
-static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean) {
+static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean, bool fixed) {
     FwdLayout f;
     Bump b;
     size_t n = (size_t)T * L->K;
@@ -324,6 +333,11 @@ static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean)
     f.y = b.take(rows * (size_t)L->D * 2);
     f.sh_h = b.take(L->has_shared && !f.fold ? (size_t)T * L->Fs * 2 : 0);
     f.sh_y = b.take(L->has_shared && !f.fold ? (size_t)T * L->D * 2 : 0);
+    f.ordered = f.small && !fixed && rows > (size_t)kPairMinRows && n >= (size_t)kOrderedAvgRows * (size_t)L->E && qgemm_skinny_factored(L->gate.view) && qgemm_skinny_factored(L->down.view) &&
+                L->D % 64 == 0 && L->F % 64 == 0;
+    f.xo = b.take(f.ordered ? (size_t)T * L->D * 2 : 0);
+    f.xs = b.take(f.ordered ? (size_t)T * (L->D / 64) * 4 : 0);
+    f.hs = b.take(f.ordered ? rows * (size_t)(L->F / 64) * 4 : 0);
     f.total = b.off;
     return f;
 }
@@ -339,8 +353,8 @@ static size_t static_need(const Layer *L, int T, const FwdLayout &f) {
 // `fixed`: scratch is the static array. Small tiles and a folded shared expert lengthen the lists by a few bytes per token;
 // the largest batches that fit without them are planned without them, so that they still fit.
 static FwdLayout forward_layout(const Layer *L, int T, bool with_shared = true, bool fixed = false) {
-    const FwdLayout f = plan_layout(L, T, with_shared, false);
-    if (fixed && static_need(L, T, f) > kStaticScratchBytes - kStaticFlagBytes) return plan_layout(L, T, with_shared, true);
+    const FwdLayout f = plan_layout(L, T, with_shared, false, fixed);
+    if (fixed && static_need(L, T, f) > kStaticScratchBytes - kStaticFlagBytes) return plan_layout(L, T, with_shared, true, fixed);
     return f;
 }
 
@@ -390,9 +404,6 @@ static int routed_forward(const Layer *L, Workspace *w, const FwdLayout &f, cons
         po.remap = L->remap;
         po.n_remap = (uint32_t)L->n_total;
     }
-    if (route) DMOE_TRY(launch_route_pack_tiny(po, *route, L->E, f.tile_m, st)); // the selection has not run yet: one launch for both
-    else DMOE_TRY(launch_pack(po, d_ids, n, L->K, L->E, f.tile_m, at<void>(w, f.scratch), st));
-    DMOE_TRY(stage_end(w, DMOE_STAGE_PACK, st));
 
     GemmArgs gu;
     gu.b0 = L->gate.view;
@@ -438,7 +449,22 @@ static int routed_forward(const Layer *L, Workspace *w, const FwdLayout &f, cons
     // (Up to kPairMinRows sorted rows the two projections run as two launches: with so few tiles nearly every gate/up
     // workgroup is resident from the start, no down workgroup can begin before they end, and what the single launch
     // adds is the hand-over through memory - stores acknowledged, counter, poll - of 6-8 us per step.)
-    if (f.small && w->paired && n + (f.fold ? (size_t)T : 0) > (size_t)kPairMinRows && qgemm_skinny_pair_supports(gu, dn)) {
+    const bool pair = f.small && w->paired && n + (f.fold ? (size_t)T : 0) > (size_t)kPairMinRows && qgemm_skinny_pair_supports(gu, dn);
+    w->last_ordered = pair && f.ordered;
+    if (w->last_ordered) {
+        po.rows_in = (const uint4 *)d_x;
+        po.rows_out = at<uint4>(w, f.xo);
+        po.rows_sums = at<float>(w, f.xs);
+        po.rows_pieces = (uint32_t)((size_t)T * L->D / 8);
+        gu.a = at<uint16_t>(w, f.xo);
+        gu.a_sums = po.rows_sums;
+        gu.out_sums = at<float>(w, f.hs);
+        dn.a_sums = gu.out_sums;
+    }
+    if (route) DMOE_TRY(launch_route_pack_tiny(po, *route, L->E, f.tile_m, st)); // the selection has not run yet: one launch for both
+    else DMOE_TRY(launch_pack(po, d_ids, n, L->K, L->E, f.tile_m, at<void>(w, f.scratch), st));
+    DMOE_TRY(stage_end(w, DMOE_STAGE_PACK, st));
+    if (pair) {
         DMOE_TRY(stage_begin(w, DMOE_STAGE_GATE_UP, st));
         DMOE_TRY(launch_qgemm_skinny_pair(gu, dn, st));
         DMOE_TRY(stage_end(w, DMOE_STAGE_GATE_UP, st));
@@ -866,7 +892,7 @@ int dmoe_debug_last_activations(uint16_t *d_out, dmoe_layer layer, int T, dmoe_w
     size_t n = (size_t)T * L->K, rv = (size_t)L->F / 8, total = n * rv;
     if (total == 0) return DMOE_OK;
     hipLaunchKernelGGL(scatter_rows_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, to_hip(s),
-                       (uint4 *)d_out, (const uint4 *)at<uint16_t>(w, f.h), at<uint32_t>(w, f.order), rv, total);
+                       (uint4 *)d_out, (const uint4 *)at<uint16_t>(w, f.h), at<uint32_t>(w, f.order), rv, total, w->last_ordered ? 1 : 0);
     DMOE_LAUNCH_CHECK();
     return DMOE_OK;
 }

@@ -8,6 +8,8 @@
 // of one expert keep ascending flat index. No global atomics; the result is deterministic.
 //
 // Up to 4096 rows everything runs in ONE launch (16 wavefronts x 1 to 4 groups of 64 rows); above that in three.
+#include <algorithm>
+
 #include "common.h"
 #include "route_device.h"
 
@@ -156,6 +158,20 @@ __device__ __forceinline__ void place_row(const PackOut &o, uint32_t pos, uint32
     if (o.sorted_e) o.sorted_e[pos] = e;
 }
 
+// The launch's further workgroups put the activations in code order for the weight-streaming kernel (PackOut::rows_in), on
+// compute units that the packing leaves idle. A thread takes a 16-byte piece.
+__device__ __forceinline__ void order_rows(const PackOut &o, uint32_t block, uint32_t n_blocks) {
+    for (uint32_t i = block * blockDim.x + threadIdx.x; i < o.rows_pieces; i += n_blocks * blockDim.x) { // whole eights of lanes
+        const uint4 v = to_code_order(o.rows_in[i]);
+        o.rows_out[i] = v;
+        const float sum = sum64_of_code_order(v);
+        if ((i & 7u) == 0) o.rows_sums[i >> 3] = sum;
+    }
+}
+static uint32_t order_rows_blocks(const PackOut &o, int threads) {
+    return std::min<uint32_t>((o.rows_pieces + (uint32_t)threads - 1) / (uint32_t)threads, 512u);
+}
+
 // ---- one launch, n <= 1024 ---------------------------------------------------------------------------------
 // `e` = this thread's expert id (row i = tid), `pack_sm` = hist[kPackWaves][E] in LDS
 __device__ __forceinline__ void pack_fused_body(const PackOut &o, uint32_t e, bool active, uint32_t n, int K, int E,
@@ -192,6 +208,10 @@ __global__ __launch_bounds__(kPackThreads) void pack_fused_kernel(PackOut o, con
                                                                   uint32_t n, int K, int E, int tile_m) {
     extern __shared__ uint32_t pack_sm[]; // hist[kPackWaves][E]
     __shared__ uint32_t scan_sm[4 * kPackWaves];
+    if (blockIdx.x > 0) {
+        order_rows(o, blockIdx.x - 1, gridDim.x - 1);
+        return;
+    }
     const bool active = threadIdx.x < n;
     const uint32_t e = active ? packed_id(o, idx[threadIdx.x]) : 0u;
     pack_fused_body(o, e, active, n, K, E, tile_m, pack_sm, scan_sm);
@@ -207,6 +227,10 @@ __global__ __launch_bounds__(kPackThreads) void pack_groups_kernel(PackOut o, co
                                                                    uint32_t n, int K, int E, int tile_m, int groups) {
     extern __shared__ uint32_t pack_sm[]; // hist[kPackWaves][E]
     __shared__ uint32_t scan_sm[4 * kPackWaves];
+    if (blockIdx.x > 0) {
+        order_rows(o, blockIdx.x - 1, gridDim.x - 1);
+        return;
+    }
     const int tid = (int)threadIdx.x, lane = lane_id(), wave = tid >> 6;
     const uint32_t row0 = (uint32_t)(wave * groups * 64 + lane);
     uint32_t ids[kPackGroups];
@@ -392,6 +416,11 @@ __global__ __launch_bounds__(kScatterWaves * 64) void pack_hist_kernel(PackOut o
                                                                        const uint32_t *__restrict__ idx,
                                                                        size_t n, int E, int n_sub) {
     extern __shared__ uint32_t pack_sm[]; // hist[kScatterWaves][E]
+    const uint32_t hist_blocks = (uint32_t)((n_sub + kScatterWaves - 1) / kScatterWaves);
+    if (blockIdx.x >= hist_blocks) {
+        order_rows(o, blockIdx.x - hist_blocks, gridDim.x - hist_blocks);
+        return;
+    }
     const int tid = (int)threadIdx.x, lane = lane_id(), wave = tid >> 6;
     for (int i = tid; i < kScatterWaves * E; i += kScatterWaves * 64) pack_sm[i] = 0;
     __syncthreads();
@@ -482,6 +511,8 @@ int launch_pack(const PackOut &o, const uint32_t *d_idx, size_t n, int K, int E,
     DMOE_REQUIRE(K >= 1, "pack: K=%d", K);
     DMOE_REQUIRE(n < (1ull << 31), "pack: too many rows");
     DMOE_REQUIRE(n == 0 || (o.order != nullptr && d_idx != nullptr), "pack: null pointer");
+    DMOE_REQUIRE(o.rows_pieces == 0 || (n > (size_t)kPackWaveRows && o.rows_pieces % 8 == 0 && o.rows_in && o.rows_out && o.rows_sums),
+                 "pack: %u pieces of rows to put in code order", o.rows_pieces);
     if (n <= (size_t)kPackWaveRows) { // also covers n == 0: counts / offsets / n_tiles / n_live are still written (all zero)
         hipLaunchKernelGGL(pack_wave_kernel, dim3(1), dim3(64), 0, st, o, d_idx, (uint32_t)n, K, E, tile_m);
         DMOE_LAUNCH_CHECK();
@@ -491,9 +522,9 @@ int launch_pack(const PackOut &o, const uint32_t *d_idx, size_t n, int K, int E,
         const size_t lds = sizeof(uint32_t) * (size_t)kPackWaves * E;
         const int groups = (int)((n + kPackThreads - 1) / kPackThreads);
         if (groups == 1)
-            hipLaunchKernelGGL(pack_fused_kernel, dim3(1), dim3(kPackThreads), lds, st, o, d_idx, (uint32_t)n, K, E, tile_m);
+            hipLaunchKernelGGL(pack_fused_kernel, dim3(1 + order_rows_blocks(o, kPackThreads)), dim3(kPackThreads), lds, st, o, d_idx, (uint32_t)n, K, E, tile_m);
         else
-            hipLaunchKernelGGL(pack_groups_kernel, dim3(1), dim3(kPackThreads), lds, st, o, d_idx, (uint32_t)n, K, E, tile_m, groups);
+            hipLaunchKernelGGL(pack_groups_kernel, dim3(1 + order_rows_blocks(o, kPackThreads)), dim3(kPackThreads), lds, st, o, d_idx, (uint32_t)n, K, E, tile_m, groups);
         DMOE_LAUNCH_CHECK();
         return DMOE_OK;
     }
@@ -502,7 +533,7 @@ int launch_pack(const PackOut &o, const uint32_t *d_idx, size_t n, int K, int E,
     int n_sub = (int)((n + kSubRows - 1) / kSubRows);
     dim3 grid((unsigned)ceil_div(n_sub, kScatterWaves)), block(kScatterWaves * 64);
     size_t lds = sizeof(uint32_t) * (size_t)kScatterWaves * E;
-    hipLaunchKernelGGL(pack_hist_kernel, grid, block, lds, st, o, cnt, d_idx, n, E, n_sub);
+    hipLaunchKernelGGL(pack_hist_kernel, dim3(grid.x + order_rows_blocks(o, kScatterWaves * 64)), block, lds, st, o, cnt, d_idx, n, E, n_sub);
     DMOE_LAUNCH_CHECK();
     hipLaunchKernelGGL(pack_scan_kernel, dim3(1), dim3(kPackThreads), 0, st, o, cnt, n, E, n_sub, tile_m);
     DMOE_LAUNCH_CHECK();

@@ -52,11 +52,8 @@ __device__ __forceinline__ void codes_to_bf16(uint32_t w, uint32_t mask, uint32_
 // s_waitcnt immediate for "at most n vector-memory loads outstanding" (gfx9: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14])
 constexpr int skinny_wait_vmcnt(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
 
-template <int CTRL>
-__device__ __forceinline__ float skinny_dpp(float x) {
-    const int v = __float_as_int(x);
-    return __int_as_float(__builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false));
-}
+// the factored 4-bit form on activations that come in code order, with the sums beside them (GemmArgs::a_sums)
+struct FmtAffine4Ordered : FmtAffine4 {};
 
 template <int NM>
 struct SkinnyStage {
@@ -141,6 +138,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     constexpr int ROUND = MBLK && STAGES < 8 ? 8 : STAGES;  // steps per unrolled round (MBLK: whole blocks of entries)
     static_assert(ROUND % STAGES == 0 && (!MBLK || ROUND % 8 == 0), "rounds are whole turns of the ring");
     constexpr int NM = 1;                           // projections per wavefront
+    constexpr bool ORDERED = std::is_same<Fmt, FmtAffine4Ordered>::value;
     constexpr bool ZEROS = skinny_reads_zeros(FACTORED, KSPLIT, FEW);
     // Launches of a few workgroups are paced by each wavefront's own chain of steps, and the look-ahead has to be in the machine
     // code: left alone, the scheduler gathers the loads of a round behind its fourth step and waits for nearly all of them at
@@ -295,21 +293,44 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         for (int idx = tid; idx < nrows * pieces; idx += WAVES * 64) {
             const int r = idx / pieces, pc = idx - r * pieces;
             uint4 *px = (uint4 *)(xs_lds + r * pitch + pc * 16);
-            const uint4 v = *px;
-            float sum = (bf16_bits_to_f32(v.x & 0xffffu) + bf16_bits_to_f32(v.x >> 16)) +
-                        (bf16_bits_to_f32(v.y & 0xffffu) + bf16_bits_to_f32(v.y >> 16)) +
-                        (bf16_bits_to_f32(v.z & 0xffffu) + bf16_bits_to_f32(v.z >> 16)) +
-                        (bf16_bits_to_f32(v.w & 0xffffu) + bf16_bits_to_f32(v.w >> 16));
-            uint4 o;
-            o.x = (v.x & 0xffffu) | (v.z << 16);
-            o.y = (v.x >> 16) | (v.z & 0xffff0000u);
-            o.z = (v.y & 0xffffu) | (v.w << 16);
-            o.w = (v.y >> 16) | (v.w & 0xffff0000u);
-            *px = o;
-            sum += skinny_dpp<0xB1>(sum);  // lane ^ 1 (quad_perm 1,0,3,2)
-            sum += skinny_dpp<0x4E>(sum);  // lane ^ 2 (quad_perm 2,3,0,1)
-            sum += skinny_dpp<0x141>(sum); // the other quad of the eight lanes (row_half_mirror)
+            const uint4 v = to_code_order(*px);
+            *px = v;
+            const float sum = sum64_of_code_order(v);
             if ((pc & 7) == 0) gs_lds[(pc >> 3) * rp + r] = sum;
+        }
+    };
+    // ORDERED: the rows come in code order (g.a_sums) and need no pass over LDS; the sums are fetched beside them. Wavefront w takes rows
+    // w, w + 8, ..., a lane a step; requested ahead of the rows, so that whoever waits for those has these too.
+    constexpr int SUM_CHUNKS = RJT == 1 ? 3 : RJT == 2 ? 2 : 1; // 64 steps each: spans of the longest reduction LDS can hold
+    static_assert((kSkinnyMaxLds / (kSkinnyRowBlock * 2) / 64 + RJT - 1) / RJT <= SUM_CHUNKS * 64, "steps of a span");
+    float sums[RJT * SUM_CHUNKS];
+    auto load_sums = [&](int span) {
+#pragma unroll
+        for (int i = 0; i < RJT; ++i) {
+            const int r = wave + WAVES * i;
+            if (r >= nrows) continue; // uniform
+            const float *row = g.a_sums + (size_t)(uint32_t)__builtin_amdgcn_readlane((int)src_of_lane, r) * (size_t)n_steps + span * span_steps;
+#pragma unroll
+            for (int c = 0; c < SUM_CHUNKS; ++c) {
+                const int s = c * 64 + lane;
+                if (s >= span_steps) continue;
+                if (sync == kSkinnySyncWait) // (written by this launch's gate/up workgroups, like the rows)
+                    sums[i * SUM_CHUNKS + c] = __hip_atomic_load(row + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else
+                    sums[i * SUM_CHUNKS + c] = row[s];
+            }
+        }
+    };
+    auto place_sums = [&]() {
+#pragma unroll
+        for (int i = 0; i < RJT; ++i) {
+            const int r = wave + WAVES * i;
+            if (r >= nrows) continue;
+#pragma unroll
+            for (int c = 0; c < SUM_CHUNKS; ++c) {
+                const int s = c * 64 + lane;
+                if (s < span_steps) gs_lds[s * rp + r] = sums[i * SUM_CHUNKS + c];
+            }
         }
     };
 
@@ -339,11 +360,13 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         __syncthreads();
 #pragma unroll
         for (int mi = 0; mi < NM; ++mi) cs[mi].pin();
+        if (ORDERED) load_sums(0);
         issue_x(0);
         __builtin_amdgcn_s_waitcnt(skinny_wait_vmcnt(0));
     } else {
         // Loads return in issue order: the first span is requested ahead of the first stages of the weight ring, and
         // the wait below lets the ring stay in flight.
+        if (ORDERED) load_sums(0);
         issue_x(0);
 #pragma unroll
         for (int mi = 0; mi < NM; ++mi) cs[mi].pin(); // keeps the weight loads behind the requests above
@@ -354,8 +377,9 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         if (n_loc >= PRE) __builtin_amdgcn_s_waitcnt(skinny_wait_vmcnt(PRE * NM));
         else __builtin_amdgcn_s_waitcnt(skinny_wait_vmcnt(0));
     }
+    if (ORDERED) place_sums();
     __syncthreads();
-    if (FACTORED) {
+    if (FACTORED && !ORDERED) {
         fix_x();
         __syncthreads();
     }
@@ -490,10 +514,12 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
                 // the next span of the activations replaces the one in LDS (the weight ring stays in flight; its
                 // loads are older than these requests, so the wait covers nothing that was not due anyway)
                 __syncthreads();
+                if (ORDERED) load_sums(s0 / span_steps);
                 issue_x(s0 / span_steps);
                 __builtin_amdgcn_s_waitcnt(skinny_wait_vmcnt(0));
+                if (ORDERED) place_sums();
                 __syncthreads();
-                if (FACTORED) {
+                if (FACTORED && !ORDERED) {
                     fix_x();
                     __syncthreads();
                 }
@@ -592,6 +618,8 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         const int cw_shift = (gate_up ? 7 : 8) - (ks ? 1 : 0); // log2 of the workgroup's output columns
         uint16_t *const stage = (uint16_t *)(skinny_lds + kSkinnyStageOffset); // [tile rows][columns of the workgroup]
         if (wide_out && !gate_up && !ks) __syncthreads(); // (the other roles have met at a barrier since the main loop)
+        const bool order_out = ORDERED && g.out_sums != nullptr; // whole 64s of columns, see the launch functions
+        const int out_ln = order_out ? (ln & 24) + ((ln & 3) << 1) + ((ln >> 2) & 1) : ln;
 #pragma unroll
         for (int j = 0; j < RJT; ++j) {
 #pragma unroll
@@ -602,7 +630,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
                 float val = gate_up ? limited_swiglu(v[0][4 * j + r], v[1][4 * j + r], swiglu_limit) : v[0][4 * j + r];
                 if (g.row_scale && p < g.row_scale_rows) val *= g.row_scale[g.row_scale_idx ? g.row_scale_idx[p] : p];
                 if (wide_out) {
-                    stage[(i << cw_shift) + (gate_up ? wq >> 1 : wq) * 32 + ln] = f32_to_bf16_bits(val);
+                    stage[(i << cw_shift) + (gate_up ? wq >> 1 : wq) * 32 + out_ln] = f32_to_bf16_bits(val);
                     continue;
                 }
                 const size_t dst = g.out_rows ? g.out_rows[p] : p;
@@ -614,7 +642,23 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
                     g.out[dst * (size_t)g.ldo + n] = f32_to_bf16_bits(val);
             }
         }
-        if (wide_out) {
+        if (order_out) { // gate/up role: 16 pieces of 8 columns per row, eight neighbouring lanes have a sum's 64
+            __syncthreads();
+            const int strip0 = (int)blockIdx.x << cw_shift;
+            for (int idx = tid; idx < (nrows << 4); idx += WAVES * 64) {
+                const int r = idx >> 4, c = (idx & 15) * 8;
+                if (strip0 + c >= n_out) continue;
+                const size_t p = t.row0 + (uint32_t)r;
+                const uint4 d = *(const uint4 *)(stage + (r << cw_shift) + c);
+                const float sum = sum64_of_code_order(d);
+                uint64_t *o = (uint64_t *)(g.out + p * (size_t)g.ldo + strip0 + c);
+                float *so = g.out_sums + p * (size_t)(n_out >> 6) + ((strip0 + c) >> 6);
+                const uint64_t lo = (uint64_t)d.y << 32 | d.x, hi = (uint64_t)d.w << 32 | d.z;
+                __hip_atomic_store(o, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(o + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((lane & 7) == 0) __hip_atomic_store(so, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        } else if (wide_out) {
             __syncthreads();
             const int pp_shift = cw_shift - 2;                     // 4-column pieces per row
             const int strip0 = (int)blockIdx.x << cw_shift;        // the workgroup's first output column
@@ -751,6 +795,7 @@ static int skinny_prepare_format() {
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, false, has_entries>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, false, has_entries>()));
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, false, false>()));
+    if constexpr (can_factor) DMOE_TRY((skinny_raise_limit<FmtAffine4Ordered, true, true, false>()));
     return skinny_raise_limit<Fmt, false, false, false>();
 }
 int qgemm_skinny_prepare() {
@@ -770,7 +815,10 @@ struct SkinnyLaunch {
     int go() {
         // 8 wavefronts per workgroup: 128 output columns of gate AND up, or 256 of a single projection
         auto blocks_x = [](const GemmArgs &a) { return ceil_div((a.ksplit ? 2 : 1) * a.b0.rows, (a.gate_up ? 1 : 2) * kSkinnyWaves * 32); };
-        if constexpr (PACKED && !MBLK && !KSPLIT && !FEW) {
+        if constexpr (FACTORED && PACKED && !KSPLIT && !FEW && !std::is_same<Fmt, FmtAffine4Ordered>::value) {
+            if (g.a_sums) return go<FmtAffine4Ordered, true, true>(); // validated by the launch functions
+        }
+        if constexpr (PACKED && !MBLK && !KSPLIT && !FEW && !std::is_same<Fmt, FmtAffine4Ordered>::value) {
             if (g.ksplit) return go<Fmt, FACTORED, PACKED, MBLK, true>(); // validated by the launch functions
             if constexpr (Fmt::kVals > 8) // (unquantized weights: nothing to pin, see PIN)
                 if (!second && std::min(g.tile_m, g.max_rows) <= kSkinnyRowBlock &&
@@ -800,7 +848,7 @@ struct SkinnyLaunch {
     int operator()() {
         // the scale can be factored out of the matrix product when both halves of a step share a group
         constexpr bool can_factor = std::is_same<Fmt, FmtAffine4>::value;
-        const bool factor = can_factor && g.b0.group >= 64;
+        const bool factor = can_factor && qgemm_skinny_factored(g.b0);
         if (g.b0.packed) return factor ? go<Fmt, can_factor, true>() : go<Fmt, false, true>();
         // MLX layout: scale / bias entries in 16-byte blocks when every row of them is a whole number of blocks
         constexpr bool has_entries = Fmt::kMetaEntryBytes != 0;
@@ -810,13 +858,13 @@ struct SkinnyLaunch {
     }
 };
 
-static bool skinny_factored(const QView &b) { return b.mode == DMOE_QUANT_AFFINE && b.bits == 4 && b.group >= 64; }
+bool qgemm_skinny_factored(const QView &b) { return b.mode == DMOE_QUANT_AFFINE && b.bits == 4 && b.group >= 64; }
 
 bool qgemm_skinny_pair_supports(const GemmArgs &gu, const GemmArgs &dn) {
     const QView &a = gu.b0, &b = dn.b0;
     return gu.gate_up && !dn.gate_up && gu.tiles && gu.tiles == dn.tiles && gu.n_tiles == dn.n_tiles &&
            gu.max_tiles == dn.max_tiles && gu.max_tiles > 0 && 2 * (long)gu.max_tiles <= 65535 &&
-           a.packed == b.packed && a.mode == b.mode && a.bits == b.bits && skinny_factored(a) == skinny_factored(b) &&
+           a.packed == b.packed && a.mode == b.mode && a.bits == b.bits && qgemm_skinny_factored(a) == qgemm_skinny_factored(b) &&
            qgemm_skinny_supports(a) && qgemm_skinny_supports(b) && std::min(gu.tile_m, gu.max_rows) <= qgemm_skinny_tile_m(a) &&
            std::min(dn.tile_m, dn.max_rows) <= qgemm_skinny_tile_m(b) && gu.max_rows == dn.max_rows &&
            gu.tile_done != nullptr && dn.a == gu.out;
@@ -824,6 +872,11 @@ bool qgemm_skinny_pair_supports(const GemmArgs &gu, const GemmArgs &dn) {
 
 int launch_qgemm_skinny_pair(const GemmArgs &gu, const GemmArgs &dn, hipStream_t st) {
     DMOE_REQUIRE(qgemm_skinny_pair_supports(gu, dn), "skinny GEMM pair: arguments do not form a gate/up + down pair");
+    DMOE_REQUIRE((!gu.a_sums && !gu.out_sums && !dn.a_sums) ||
+                     (qgemm_skinny_factored(gu.b0) && gu.b0.packed && gu.a_sums && gu.out_sums && dn.a_sums == gu.out_sums && !gu.out_rows && gu.b0.rows % 64 == 0 && gu.ldo % 8 == 0 &&
+                      ((uintptr_t)gu.out % 16) == 0),
+                 "skinny GEMM pair: rows in code order need the factored 4-bit form in both roles");
+    DMOE_REQUIRE(!dn.out_sums, "skinny GEMM pair: the down projection's outputs have no code order");
     DMOE_REQUIRE(!gu.ksplit && !dn.ksplit, "skinny GEMM pair: the split reduction is for single launches (steps of a few rows run as two)");
     DMOE_REQUIRE(gu.a && gu.out && dn.out && ((uintptr_t)gu.a % 16) == 0 && ((uintptr_t)dn.a % 16) == 0, "skinny GEMM pair: bad pointer");
     DMOE_REQUIRE(gu.b1.rows == gu.b0.rows && gu.b1.cols == gu.b0.cols && gu.b1.mode == gu.b0.mode && gu.b1.bits == gu.b0.bits &&
@@ -847,6 +900,7 @@ int launch_qgemm_skinny(const GemmArgs &g, hipStream_t st) {
                      "skinny GEMM: gate and up projections differ in shape or format");
     DMOE_REQUIRE(!g.ksplit || (g.tile_m <= kSkinnyRowBlock && qgemm_skinny_ksplit_ok(g.b0) && (!g.gate_up || qgemm_skinny_ksplit_ok(g.b1))),
                  "skinny GEMM: a split reduction needs packed weights and tiles of at most %d rows", kSkinnyRowBlock);
+    DMOE_REQUIRE(!g.out_sums && !g.a_sums, "skinny GEMM: rows in code order are for the paired launch");
     if (g.max_tiles == 0) return DMOE_OK;
     if (g.b0.mode == DMOE_QUANT_NONE) return SkinnyLaunch{g, st}.template go<FmtBf16, false, true>();
     return dispatch_format(g.b0, SkinnyLaunch{g, st});
