@@ -267,6 +267,13 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     // source rows of the tile: one load for all of them (lane r holds row r's), then uniform reads
     uint32_t src_of_lane = __builtin_amdgcn_readfirstlane(t.row0) + (uint32_t)(lane < nrows ? lane : 0);
     if (g.a_rows) src_of_lane = g.a_rows[src_of_lane];
+    // Pinned rows: known before the loop over the requests below, whose first use of them would otherwise make every turn wait
+    // for the turn before it to come back from memory (a span of 16 rows of 4 KiB: eight turns of a wavefront, at
+    // every restaging). us per step before | now: 509 tokens 4-bit 792 | 761, MXFP4 686 | 675, 64 tokens MXFP4 132 | 128, 200 tokens
+    // 4-bit 361 | 354, 600 at hidden 3072 604 | 588. Not for small tiles of the factored form on a full chip, where the spread-out
+    // requests are no loss (64 tokens 256.5 | 258.4, 200 tokens 354.7 | 356.3).
+    constexpr bool PIN_ROWS = RJT > 1 || !FACTORED || KSPLIT || FEW;
+    if (PIN_ROWS) asm volatile("" : "+v"(src_of_lane));
     // requests span `span` of every row straight into LDS (no registers); completion is the caller's wait
     auto issue_x = [&](int span) {
         const int cpr = (span_bytes + 1023) >> 10; // 1 KiB operations per row
