@@ -481,6 +481,8 @@ __global__ __launch_bounds__(SPLIT ? EPL * 64 : kGateWaves * 64) void gate_score
         if (scoring == DMOE_SCORE_SQRTSOFTPLUS) return sqrtf(det_logf(1.0f + det_expf(x))); // the reference's literal form (:575-583)
         return sqrtf(det_softplusf(x));
     };
+    RouteBias<EPL> sel; // (requested ahead of the sums)
+    if (ROUTE) sel.load(bias, resident, E, lane);
     float v[EPL];
     float mx = -__builtin_inff();
     const float *const p = partial + (size_t)t * n_seg * E;
@@ -547,7 +549,7 @@ __global__ __launch_bounds__(SPLIT ? EPL * 64 : kGateWaves * 64) void gate_score
     if (ROUTE) {
         uint32_t my_idx;
         float w;
-        route_from_registers<EPL>(v, bias, resident, E, K, normalize, 1, route_scale, lane, my_idx, w);
+        route_from_registers<EPL>(v, sel, E, K, normalize, 1, route_scale, lane, my_idx, w);
         if (lane < K) {
             out_idx[(size_t)t * K + lane] = my_idx;
             out_w[(size_t)t * K + lane] = w;

@@ -158,6 +158,24 @@ __device__ __forceinline__ void place_row(const PackOut &o, uint32_t pos, uint32
     if (o.sorted_e) o.sorted_e[pos] = e;
 }
 
+// Phase 2 of the one-launch kernels: hist[kPackWaves][E] -> the wavefronts' first positions. The counts of an expert are read in
+// one go and their places written in one go (one after the other, each of 32 passes would wait for the LDS).
+__device__ __forceinline__ void pack_offsets(uint32_t *pack_sm, int tid, int E, uint32_t n, int tile_m, const PackOut &o, uint32_t *scan_sm) {
+    uint32_t c[kPackWaves], count = 0;
+#pragma unroll
+    for (int w = 0; w < kPackWaves; ++w) c[w] = tid < E ? pack_sm[w * E + tid] : 0u;
+#pragma unroll
+    for (int w = 0; w < kPackWaves; ++w) {
+        const uint32_t v = c[w];
+        c[w] = count;
+        count += v;
+    }
+    const uint32_t off = emit_segments(count, tid, E, n, tile_m, o, scan_sm);
+    if (tid < E)
+#pragma unroll
+        for (int w = 0; w < kPackWaves; ++w) pack_sm[w * E + tid] = off + c[w];
+}
+
 // The launch's further workgroups put the activations in code order for the weight-streaming kernel (PackOut::rows_in), on
 // compute units that the packing leaves idle. A thread takes a 16-byte piece.
 __device__ __forceinline__ void order_rows(const PackOut &o, uint32_t block, uint32_t n_blocks) {
@@ -185,17 +203,7 @@ __device__ __forceinline__ void pack_fused_body(const PackOut &o, uint32_t e, bo
     }
     if (active) atomicAdd(&pack_sm[wave * E + e], 1u);
     __syncthreads();
-    uint32_t count = 0;
-    if (tid < E) {
-        for (int w = 0; w < kPackWaves; ++w) {
-            uint32_t c = pack_sm[w * E + tid];
-            pack_sm[w * E + tid] = count;
-            count += c;
-        }
-    }
-    uint32_t off = emit_segments(count, tid, E, n, tile_m, o, scan_sm);
-    if (tid < E)
-        for (int w = 0; w < kPackWaves; ++w) pack_sm[w * E + tid] += off;
+    pack_offsets(pack_sm, tid, E, n, tile_m, o, scan_sm);
     __syncthreads();
     uint64_t peers = match_expert(e, active, log2_ceil(E));
     if (active) {
@@ -251,17 +259,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_groups_kernel(PackOut o, co
         atomicAdd(&pack_sm[wave * E + ids[g]], 1u);
     }
     __syncthreads();
-    uint32_t count = 0;
-    if (tid < E) {
-        for (int w = 0; w < kPackWaves; ++w) {
-            uint32_t c = pack_sm[w * E + tid];
-            pack_sm[w * E + tid] = count;
-            count += c;
-        }
-    }
-    uint32_t off = emit_segments(count, tid, E, n, tile_m, o, scan_sm);
-    if (tid < E)
-        for (int w = 0; w < kPackWaves; ++w) pack_sm[w * E + tid] += off;
+    pack_offsets(pack_sm, tid, E, n, tile_m, o, scan_sm);
     __syncthreads();
     const int nbits = log2_ceil(E);
 #pragma unroll
@@ -379,15 +377,14 @@ __global__ __launch_bounds__(kPackWaveRows * 64) void route_pack_tiny_kernel(Pac
     __shared__ uint32_t ids[kPackWaveRows];
     const int lane = lane_id(), t = (int)(threadIdx.x >> 6);
     {
-        const float *const rows[1] = {r.scores + (size_t)t * r.E};
-        uint32_t my_idx[1];
-        float w[1];
-        route_tokens<1, 4>(rows, r.bias, r.resident, r.E, r.K, r.normalize, r.apply_scale, r.route_scale, lane, my_idx, w);
+        uint32_t my_idx;
+        float w;
+        route_token<4>(r.scores + (size_t)t * r.E, r.bias, r.resident, r.E, r.K, r.normalize, r.apply_scale, r.route_scale, lane, my_idx, w);
         if (lane < r.K) {
             const size_t at = (size_t)t * r.K + lane;
-            r.out_idx[at] = my_idx[0];
-            r.out_w[at] = w[0];
-            ids[at] = my_idx[0];
+            r.out_idx[at] = my_idx;
+            r.out_w[at] = w;
+            ids[at] = my_idx;
         }
     }
     __syncthreads();

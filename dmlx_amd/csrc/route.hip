@@ -10,7 +10,7 @@ namespace dmoe {
 
 constexpr int kRouteWaves = 4;
 
-// One wavefront per token (route_tokens); EPL = experts per lane
+// One wavefront per token (route_token); EPL = experts per lane
 template <int EPL>
 __global__ __launch_bounds__(kRouteWaves * 64) void route_kernel(
     uint32_t *__restrict__ out_idx, float *__restrict__ out_w, const float *__restrict__ scores,
@@ -19,13 +19,12 @@ __global__ __launch_bounds__(kRouteWaves * 64) void route_kernel(
     const int wave = (int)(threadIdx.x >> 6), lane = lane_id();
     const int t = (int)blockIdx.x * kRouteWaves + wave;
     if (t >= T) return;
-    const float *const rows[1] = {scores + (size_t)t * E};
-    uint32_t my_idx[1];
-    float w[1];
-    route_tokens<1, EPL>(rows, bias, resident, E, K, normalize, apply_scale, route_scale, lane, my_idx, w);
+    uint32_t my_idx;
+    float w;
+    route_token<EPL>(scores + (size_t)t * E, bias, resident, E, K, normalize, apply_scale, route_scale, lane, my_idx, w);
     if (lane < K) {
-        out_idx[(size_t)t * K + lane] = my_idx[0];
-        out_w[(size_t)t * K + lane] = w[0];
+        out_idx[(size_t)t * K + lane] = my_idx;
+        out_w[(size_t)t * K + lane] = w;
     }
 }
 
