@@ -442,6 +442,32 @@ struct ChunkStream {
         if (PACKED) Fmt::load_meta_at(mbase + Fmt::packed_meta_step(q, step) + mlane, sb);
         else Fmt::load_meta_raw(q, srow, brow, (step * 2 + h) * Fmt::kVals, sb);
     }
+    // The same loads of the packed layout with a scalar base and the lane's 32-bit offset. Base and offset go through an empty asm
+    // statement, or the compiler keeps their 64-bit sum in vector registers and adds the step to it, a vector addition per load
+    // and two registers of address. Prefill kernel, us per step: 8192 tokens 4-bit 2480 -> 2432, bf16 3079 -> 3028, 1531 tokens MXFP4
+    // 903 -> 894.
+    template <typename T, bool STREAM>
+    __device__ static __forceinline__ T load_at(const uint8_t *uniform, uint32_t lane_offset) {
+        static_assert(PACKED, "the packed layout only");
+        uint64_t base = (uint64_t)(uintptr_t)uniform;
+        asm("" : "+s"(base), "+v"(lane_offset));
+        typedef const __attribute__((address_space(1))) uint8_t *global_u8;
+        typedef const __attribute__((address_space(1))) T *global_t;
+        const global_t p = (global_t)((global_u8)base + lane_offset);
+        return STREAM ? __builtin_nontemporal_load(p) : *p;
+    }
+    template <bool STREAM>
+    __device__ __forceinline__ uint4 load_chunk_scalar(int step) const {
+        typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+        const u32x4_t v = load_at<u32x4_t, STREAM>(w + (size_t)step * 1024, wlane);
+        return make_uint4(v.x, v.y, v.z, v.w);
+    }
+    __device__ __forceinline__ void load_meta_scalar(const QView &q, int step, uint32_t *sb) const {
+        const uint8_t *const m = mbase + Fmt::packed_meta_step(q, step);
+        if (Fmt::kMetaEntryBytes == 2) sb[0] = load_at<uint32_t, false>(m, mlane); // affine: scale | bias << 16
+        else if (Fmt::kMetaEntryBytes == 1) sb[0] = load_at<uint8_t, false>(m, mlane);
+        else sb[0] = 0u;
+    }
     __device__ static __forceinline__ Meta meta(const uint32_t *sb) {
         return PACKED ? Fmt::meta_from_packed(sb) : Fmt::meta_from_raw(sb);
     }

@@ -140,6 +140,11 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     constexpr int NM = 1;                           // projections per wavefront
     constexpr bool ORDERED = std::is_same<Fmt, FmtAffine4Ordered>::value;
     constexpr bool ZEROS = skinny_reads_zeros(FACTORED, KSPLIT, FEW);
+    // Weight loads with a scalar base (ChunkStream::load_at) where the launch fills the chip: 509 tokens on MXFP4 675 -> 666 us, 64
+    // tokens on MXFP4 129 -> 126.5, on 8-bit 479 -> 473; not for the scales of the factored form's small tiles (64 tokens 255.4 ->
+    // 252.3 with the chunks alone, 257.0 with both), nor in launches of a few workgroups (8 tokens, 64 experts 49.2 -> 50.7; one
+    // token 45.1 -> 45.7; the small layer 32.6 -> 32.0).
+    constexpr bool SCALAR = PACKED && !KSPLIT && !FEW, SCALAR_META = SCALAR && !(FACTORED && RJT == 1);
     // Launches of a few workgroups are paced by each wavefront's own chain of steps, and the look-ahead has to be in the machine
     // code: left alone, the scheduler gathers the loads of a round behind its fourth step and waits for nearly all of them at
     // the next one's start, where in the round depending on what surrounds it. Each step's loads are pinned to its head (small
@@ -203,8 +208,10 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         }
 #pragma unroll
         for (int mi = 0; mi < NM; ++mi) {
-            s.raw[mi] = cs[mi].load_chunk_stream(step + sb0);
-            if (!MBLK) cs[mi].load_meta(qv, step + sb0, s.sb[mi]);
+            if constexpr (SCALAR) s.raw[mi] = cs[mi].template load_chunk_scalar<true>(step + sb0);
+            else s.raw[mi] = cs[mi].load_chunk_stream(step + sb0);
+            if constexpr (SCALAR_META) cs[mi].load_meta_scalar(qv, step + sb0, s.sb[mi]);
+            else if (!MBLK) cs[mi].load_meta(qv, step + sb0, s.sb[mi]);
         }
     };
     // ---- blocks of scale / bias entries (MBLK) -------------------------------------------------------------

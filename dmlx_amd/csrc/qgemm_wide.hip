@@ -123,8 +123,8 @@ __device__ __forceinline__ void wide_tile(const GemmArgs &g, const Tile &t, uint
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             const QView &b = (GATE_UP && nt == 1) ? g.b1 : g.b0;
-            ring_raw[slot_][nt] = STREAM ? cs[nt].load_chunk_stream(cstep) : cs[nt].load_chunk(cstep);
-            cs[nt].load_meta(b, cstep, ring_sb[slot_][nt]);
+            ring_raw[slot_][nt] = cs[nt].template load_chunk_scalar<STREAM>(cstep);
+            cs[nt].load_meta_scalar(b, cstep, ring_sb[slot_][nt]);
         }
     };
 
