@@ -267,7 +267,21 @@ struct GemmArgs {
     // `out_sums` set (gate/up role): the outputs leave in that form, the sums here.
     const float *a_sums = nullptr;
     float *out_sums = nullptr;
+    // Weight-streaming kernel, launches of a few workgroups (qgemm_skinny_takes_ids): instead of a tile list from a packing launch,
+    // the expert ids of at most kInlineRows rows. Every workgroup orders them for itself, stably by expert, into tiles of at most
+    // 8 rows; dense_rows further rows of matrix dense_expert are the tiles in front. max_tiles bounds the number of tiles.
+    const uint32_t *ids = nullptr;
+    uint32_t n_ids = 0;
+    int ids_experts = 0;            // ids at or past it count as the last one, and in *bad_ids (null: not counted here)
+    const int32_t *ids_remap = nullptr; // optional map of every id, n_remap entries (an id outside it maps to 0)
+    uint32_t n_remap = 0, dense_expert = 0;
+    int ids_k = 0;                  // source row of row i: i / ids_k, of dense row j: j (0: the sorted row itself)
+    const uint32_t *ids_lhs = nullptr; // optional map of the source rows
+    bool ids_scatter = false;       // outputs and row_scale go by the original row, else outputs stay sorted
+    uint32_t *order_out = nullptr;  // optional: the original row of every sorted row
+    uint32_t *bad_ids = nullptr;
 };
+constexpr uint32_t kInlineRows = 64;
 // tile_m the kernels were built for
 constexpr int kSkinnyTileM = 32;          // most rows a skinny tile can hold (see qgemm_skinny_tile_m)
 // Workgroups of the weight-streaming kernel up to which a launch leaves the chip half empty (one per compute unit, where two fit)
@@ -278,6 +292,7 @@ constexpr int kMfmaWideTileM = 128;
 int launch_qgemm_skinny(const GemmArgs &g, hipStream_t st);
 // gate/up + down of one tile list in one launch (down waits per tile for gate/up); gu.tile_done must be zeroed
 bool qgemm_skinny_pair_supports(const GemmArgs &gu, const GemmArgs &dn);
+bool qgemm_skinny_takes_ids(const GemmArgs &g); // may this launch take GemmArgs::ids?
 bool qgemm_skinny_factored(const QView &b); // 4-bit affine, groups of 64 and more: the form that reads GemmArgs::a_sums
 int launch_qgemm_skinny_pair(const GemmArgs &gu, const GemmArgs &dn, hipStream_t st);
 int launch_qgemm_mfma(const GemmArgs &g, hipStream_t st); // picks the wide kernel when the format allows it

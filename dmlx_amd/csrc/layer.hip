@@ -212,6 +212,16 @@ constexpr int kPairMinRows = DMOE_PAIR_MIN_ROWS; // decode steps above this many
 constexpr int kOrderedAvgRows = 4; // rows per expert from which a paired launch's rows go through code order (FwdLayout::ordered)
 constexpr int kSharedSkinnyRows = 64;
 
+// Steps of so few rows run as launches of one-row-block tiles whose workgroups order the rows for themselves (GemmArgs::ids), also
+// where that is more than kSkinnyFewGroups workgroups. us per step, packing launch and tile list | this: 256 experts top-6, hidden
+// 4096, 4-bit blocks of 4 / 8 tokens 86.4 / 123.7 | 80.5 / 120.2, 10 tokens 116.7 | 114.0, MXFP4 8 / 10 tokens 118 / 137 | 110 / 133;
+// 64 experts, hidden 2048, 8 tokens 50.0 | 46.4. 8-bit 5 / 6 / 7 tokens 142 / 196 / 201 | 137 / 184 / 192, but 9 tokens (54 rows) 237 |
+// 242, 4-bit in groups of 32 at 60 rows 211 | 212: those fill the chip, where the pinned ring of such launches is no gain.
+static size_t inline_rows(const QView &b) {
+    if (!b.packed || b.mode == DMOE_QUANT_NONE) return 0;
+    return b.mode == DMOE_QUANT_MXFP4 || qgemm_skinny_factored(b) ? kInlineRows : kInlineRows * 3 / 4;
+}
+
 static bool few_rows(size_t rows, int n_experts) { return rows <= (size_t)kSkinnyAvgRows * (size_t)n_experts; }
 static bool use_small_path(size_t rows, int n_experts, const QView &b) {
     return qgemm_skinny_supports(b) && few_rows(rows, n_experts);
@@ -257,6 +267,7 @@ struct FwdLayout {
     // LDS: 200 / 600 tokens on checkpoint arrays 211.5 / 367.6 | 213.0 / 365.0.
     bool ordered;
     bool ksplit; // at most kSplitTileM sorted rows: the weight-streaming kernel splits each tile's reduction in two
+    bool few;    // gate/up and down as two launches of tiles of one row block (few workgroups, or few rows)
     bool fold; // the shared expert rides in the routed launches: T more sorted rows behind the T*K routed ones
 };
 
@@ -320,17 +331,17 @@ static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean,
     const size_t prefill_tiles = n / (size_t)f.tile_m + (size_t)L->E + (size_t)ceil_div(T, f.tile_m);
     f.fold = with_shared && L->shared_folded && (f.small || (!lean && fold_prefill(L, T) && 2 * prefill_tiles <= 65535));
     const size_t rows = n + (f.fold ? (size_t)T : 0); // sorted rows of the GEMMs
-    f.ksplit = false;
+    f.ksplit = f.few = false;
     if (f.small) {
         // (the widest launch decides: gate/up takes 128 output columns per workgroup, down 256)
         const size_t strips = (size_t)std::max(ceil_div(L->F, 128), ceil_div(L->D, 256));
         const size_t tiles = (size_t)pack_max_tiles(n, L->E, kSplitTileM) + (f.fold ? (size_t)ceil_div(T, kSplitTileM) : 0);
-        const bool few = !lean && tiles * strips <= (size_t)kSkinnyFewGroups;
+        f.few = !lean && (tiles * strips <= (size_t)kSkinnyFewGroups || rows <= std::min(inline_rows(L->gate.view), inline_rows(L->down.view)));
         f.ksplit = rows <= (size_t)kSplitTileM &&
                    qgemm_skinny_ksplit_ok(L->gate.view) && qgemm_skinny_ksplit_ok(L->up.view) && qgemm_skinny_ksplit_ok(L->down.view) &&
                    (!f.fold || (qgemm_skinny_ksplit_ok(L->sgate.view) && qgemm_skinny_ksplit_ok(L->sup.view) &&
                                 qgemm_skinny_ksplit_ok(L->sdown.view)));
-        if (few || f.ksplit) f.tile_m = std::min(f.tile_m, kSplitTileM);
+        if (f.few || f.ksplit) f.tile_m = std::min(f.tile_m, kSplitTileM);
     }
     f.max_tiles = pack_max_tiles(n, L->E, f.tile_m) + (f.fold ? ceil_div(T, f.tile_m) : 0);
     f.order = b.take(rows * 4);
@@ -477,7 +488,27 @@ static int routed_forward(const Layer *L, Workspace *w, const FwdLayout &f, cons
         gu.out_sums = at<float>(w, f.hs);
         dn.a_sums = gu.out_sums;
     }
-    if (route) DMOE_TRY(launch_route_pack_tiny(po, *route, L->E, f.tile_m, st)); // the selection has not run yet: one launch for both
+    // A few rows: every workgroup orders the expert ids for itself, without a packing launch and without the wait for its lists
+    // (see inline_rows; small layer, 16 tokens 32.5 -> 29.3 us per step, one / two tokens 33.8 -> 32.5, 59.6 -> 54.6).
+    const bool ids = (f.few || f.ksplit) && !pair && n + (f.fold ? (size_t)T : 0) <= (size_t)kInlineRows && qgemm_skinny_takes_ids(gu) && qgemm_skinny_takes_ids(dn);
+    if (ids) {
+        for (GemmArgs *a : {&gu, &dn}) {
+            a->ids = d_ids;
+            a->n_ids = (uint32_t)n;
+            a->ids_experts = L->E;
+            a->ids_remap = po.remap;
+            a->n_remap = po.n_remap;
+            a->dense_rows = (int)po.dense_rows;
+            a->dense_expert = po.dense_expert;
+            a->tiles = nullptr;
+            a->a_rows = a->out_rows = nullptr;
+        }
+        gu.ids_k = L->K;
+        gu.order_out = po.order; // (for dmoe_debug_last_activations)
+        gu.bad_ids = po.bad_ids;
+        dn.ids_scatter = true;
+        if (route) DMOE_TRY(launch_route(*route, st));
+    } else if (route) DMOE_TRY(launch_route_pack_tiny(po, *route, L->E, f.tile_m, st)); // the selection has not run yet: one launch for both
     else DMOE_TRY(launch_pack(po, d_ids, n, L->K, L->E, f.tile_m, at<void>(w, f.scratch), st));
     DMOE_TRY(stage_end(w, DMOE_STAGE_PACK, st));
     if (pair) {
@@ -923,7 +954,8 @@ static int gather_qmm_view(uint16_t *d_out, const uint16_t *d_x, const QView &v,
     const bool small = use_small_path((size_t)R, v.n_mats, v);
     DMOE_REQUIRE(small || qgemm_mfma_supports(v) || gemm_bf16_supports(v), "gather_qmm: unsupported weight shape rows=%d cols=%d", v.rows, v.cols);
     int tile_m = small ? qgemm_skinny_tile_m(v) : qgemm_mfma_tile_m(v);
-    if (small && (size_t)pack_max_tiles((size_t)R, v.n_mats, kSplitTileM) * (size_t)ceil_div(v.rows, 256) <= (size_t)kSkinnyFewGroups)
+    if (small && ((size_t)pack_max_tiles((size_t)R, v.n_mats, kSplitTileM) * (size_t)ceil_div(v.rows, 256) <= (size_t)kSkinnyFewGroups ||
+                  (size_t)R <= inline_rows(v)))
         tile_m = std::min(tile_m, kSplitTileM); // see kSkinnyFewGroups
     const int max_tiles = pack_max_tiles((size_t)R, v.n_mats, tile_m);
     Bump b;
@@ -932,6 +964,23 @@ static int gather_qmm_view(uint16_t *d_out, const uint16_t *d_x, const QView &v,
     size_t o_scr = b.take(pack_scratch_bytes((size_t)R, v.n_mats));
     Workspace *w = nullptr;
     DMOE_TRY(workspace_reserve(ws, b.off, &w));
+    GemmArgs g;
+    g.b0 = v;
+    g.a = d_x;
+    g.out = d_out;
+    g.ldo = v.rows;
+    g.max_tiles = max_tiles;
+    g.tile_m = tile_m;
+    if (small && R <= (int)kInlineRows && tile_m <= kSplitTileM && qgemm_skinny_takes_ids(g)) { // every workgroup orders the rows for itself
+        g.ids = d_rhs_indices;
+        g.n_ids = (uint32_t)R;
+        g.ids_experts = v.n_mats;
+        g.ids_k = 1;
+        g.ids_lhs = d_lhs_indices;
+        g.ids_scatter = true;
+        g.bad_ids = w->flags + 1;
+        return launch_qgemm_skinny(g, st);
+    }
     PackOut po;
     po.order = at<uint32_t>(w, o_order);
     po.tiles = at<Tile>(w, o_tiles);
@@ -947,18 +996,11 @@ static int gather_qmm_view(uint16_t *d_out, const uint16_t *d_x, const QView &v,
         DMOE_LAUNCH_CHECK();
         a_rows = ar;
     }
-    GemmArgs g;
-    g.b0 = v;
-    g.a = d_x;
     g.a_rows = a_rows;
-    g.out = d_out;
-    g.ldo = v.rows;
     g.out_rows = po.order;
     g.tiles = po.tiles;
     g.n_tiles = po.n_tiles;
     g.n_live = po.n_live;
-    g.max_tiles = max_tiles;
-    g.tile_m = tile_m;
     return run_gemm(g, small, st, small ? 0 : prefill_small_rows(v, v), few_rows((size_t)R, v.n_mats));
 }
 

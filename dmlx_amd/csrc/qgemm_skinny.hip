@@ -109,7 +109,7 @@ static_assert(3 * skinny_lds_share(skinny_lds_bytes(3072, 32, false, 0)) <= 160 
 // bytes at a time - eight bf16 or sixteen E8M0 entries, the next block requested while the current one is in use.
 template <typename Fmt, bool FACTORED, bool PACKED, int RJT, bool MBLK, bool KSPLIT = false, bool FEW = false>
 __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, uint8_t *skinny_lds, const bool gate_up,
-                                            const int sync, const uint32_t slot) {
+                                            const int sync, const uint32_t slot, const uint32_t *ord = nullptr) {
     using CS = ChunkStream<Fmt, PACKED>;
     constexpr int KV = Fmt::kVals;   // values per 16-byte chunk
     constexpr int KSTEP = 2 * KV;    // reduction elements per step (both lane halves)
@@ -273,7 +273,17 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     const uint32_t lds_addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)skinny_lds;
     // source rows of the tile: one load for all of them (lane r holds row r's), then uniform reads
     uint32_t src_of_lane = __builtin_amdgcn_readfirstlane(t.row0) + (uint32_t)(lane < nrows ? lane : 0);
-    if (g.a_rows) src_of_lane = g.a_rows[src_of_lane];
+    // (ord: the original row of every sorted row, where the workgroup has ordered the rows itself)
+    constexpr bool INLINE = KSPLIT || FEW;
+    auto original_row = [&](uint32_t p) { return p < g.n_ids ? ord[p] : p; };
+    if (INLINE && ord) {
+        if (g.ids_k > 0) {
+            src_of_lane = src_of_lane < g.n_ids ? ord[src_of_lane] / (uint32_t)g.ids_k : src_of_lane - g.n_ids;
+            if (g.ids_lhs) src_of_lane = g.ids_lhs[src_of_lane];
+        }
+    } else if (g.a_rows) {
+        src_of_lane = g.a_rows[src_of_lane];
+    }
     // Pinned rows: known before the loop over the requests below, whose first use of them would otherwise make every turn wait
     // for the turn before it to come back from memory (a span of 16 rows of 4 KiB: eight turns of a wavefront, at
     // every restaging). us per step before | now: 509 tokens 4-bit 792 | 761, MXFP4 686 | 675, 64 tokens MXFP4 132 | 128, 200 tokens
@@ -622,6 +632,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
                 }
             }
         }
+        auto out_row = [&](uint32_t p) -> size_t { return INLINE && ord ? (g.ids_scatter ? original_row(p) : p) : g.out_rows ? g.out_rows[p] : p; };
         const bool storer = store_on && proj == 0 && kh == 0;
         const float swiglu_limit = (t.flags & kTileDense) ? g.swiglu_limit_dense : g.swiglu_limit;
         // A lane holds ONE column of up to 16 rows: stored from here that is a 2-byte store per row and lane, and a
@@ -642,12 +653,12 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
                 if (proj != 0 || kh != 0 || i >= nrows || (!wide_out && !storer)) continue;
                 const uint32_t p = t.row0 + (uint32_t)i;
                 float val = gate_up ? limited_swiglu(v[0][4 * j + r], v[1][4 * j + r], swiglu_limit) : v[0][4 * j + r];
-                if (g.row_scale && p < g.row_scale_rows) val *= g.row_scale[g.row_scale_idx ? g.row_scale_idx[p] : p];
+                if (g.row_scale && p < g.row_scale_rows) val *= g.row_scale[INLINE && ord ? original_row(p) : g.row_scale_idx ? g.row_scale_idx[p] : p];
                 if (wide_out) {
                     stage[(i << cw_shift) + (gate_up ? wq >> 1 : wq) * 32 + out_ln] = f32_to_bf16_bits(val);
                     continue;
                 }
-                const size_t dst = g.out_rows ? g.out_rows[p] : p;
+                const size_t dst = out_row(p);
                 // a producer's rows are read by workgroups on other XCDs within the same launch: device-scope
                 // stores (written through this XCD's L2), so no cache-wide write-back is needed before the signal
                 if (sync == kSkinnySyncSignal)
@@ -679,8 +690,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
             for (int idx = tid; idx < (nrows << pp_shift); idx += WAVES * 64) {
                 const int r = idx >> pp_shift, c = (idx - (r << pp_shift)) * 4;
                 if (strip0 + c >= n_out) continue;                 // a strip that ends past the matrix
-                const uint32_t p = t.row0 + (uint32_t)r;
-                const size_t dst = g.out_rows ? g.out_rows[p] : p;
+                const size_t dst = out_row(t.row0 + (uint32_t)r);
                 const uint64_t d = *(const uint64_t *)(stage + (r << cw_shift) + c);
                 uint64_t *o = (uint64_t *)(g.out + dst * (size_t)g.ldo + strip0 + c);
                 if (sync == kSkinnySyncSignal) __hip_atomic_store(o, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -693,6 +703,61 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
             if (tid == 0) __hip_atomic_fetch_add(&g.tile_done[slot], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // ... before this
         }
     }
+}
+
+// The tile of launch slot `slot` from the expert ids themselves (GemmArgs::ids): lane i holds row i, and ballots over the bits of the
+// ids give every row the rows of smaller experts and the earlier rows of its own. Tiles of the ordered rows are numbered by their
+// first rows' places in the list, behind the dense ones. `ord`: 64 words of LDS; every wavefront writes the same and reads its own.
+__device__ __forceinline__ bool skinny_tile_of_ids(const GemmArgs &g, uint32_t slot, Tile &t, uint32_t *ord) {
+    const int lane = lane_id();
+    const bool active = (uint32_t)lane < g.n_ids;
+    uint32_t e = active ? g.ids[lane] : 0u;
+    if (g.ids_remap) {
+        const bool known = active && e < g.n_remap;
+        const uint32_t m = (uint32_t)g.ids_remap[known ? e : 0u];
+        e = known ? m : 0u;
+    }
+    const uint32_t last = (uint32_t)g.ids_experts - 1u;
+    const bool bad = active && e > last; // a corrupt id: stay in bounds, and tell the host
+    e = e > last ? last : e;
+    uint64_t same_mask = __ballot(active), below_mask = 0;
+    for (int b = 31 - __builtin_clz(last | 1u); b >= 0; --b) {
+        const bool bit = (e >> b) & 1u;
+        const uint64_t ones = __ballot(active && bit);
+        below_mask |= bit ? same_mask & ~ones : 0u;
+        same_mask &= bit ? ones : ~ones;
+    }
+    const uint64_t earlier = ((uint64_t)1 << lane) - 1u;
+    const uint32_t before = (uint32_t)__popcll(same_mask & earlier), same = (uint32_t)__popcll(same_mask);
+    const uint32_t rank = (uint32_t)__popcll(below_mask) + before;
+    if (active) ord[rank] = (uint32_t)lane;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64) { // once per launch
+        if (bad && g.bad_ids) atomicAdd(g.bad_ids, 1u);
+        if (g.order_out) {
+            if (active) g.order_out[rank] = (uint32_t)lane;
+            for (int i = lane; i < g.dense_rows; i += 64) g.order_out[g.n_ids + (uint32_t)i] = g.n_ids + (uint32_t)i;
+        }
+    }
+    t.flags = 0;
+    const uint32_t n_dense = ((uint32_t)g.dense_rows + kSkinnyRowBlock - 1) / kSkinnyRowBlock;
+    if (slot < n_dense) {
+        const uint32_t left = (uint32_t)g.dense_rows - slot * kSkinnyRowBlock;
+        t.expert = g.dense_expert;
+        t.row0 = g.n_ids + slot * kSkinnyRowBlock;
+        t.nrows = left < kSkinnyRowBlock ? left : kSkinnyRowBlock;
+        t.flags = kTileDense;
+        return true;
+    }
+    const bool first = active && before % kSkinnyRowBlock == 0;
+    const uint64_t firsts = __ballot(first);
+    const uint64_t mine = __ballot(first && (uint32_t)__popcll(firsts & earlier) == slot - n_dense);
+    if (mine == 0) return false; // uniform: a slot past the last tile
+    const int l = __builtin_ctzll(mine);
+    const uint32_t left = (uint32_t)__builtin_amdgcn_readlane((int)(same - before), l);
+    t.expert = (uint32_t)__builtin_amdgcn_readlane((int)e, l);
+    t.row0 = (uint32_t)__builtin_amdgcn_readlane((int)rank, l);
+    t.nrows = left < kSkinnyRowBlock ? left : kSkinnyRowBlock;
+    return true;
 }
 
 // `paired` = 0: one GEMM (`a`). `paired` = 1: gate/up (`a`) and down (`b`) of one tile list in one launch: workgroups
@@ -718,6 +783,14 @@ __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(Gem
     const int sync = !paired ? kSkinnySyncNone : second ? kSkinnySyncWait : kSkinnySyncSignal;
     if ((int)blockIdx.x * (g.gate_up ? 1 : 2) * kSkinnyWaves * 32 >= (KSPLIT ? 2 : 1) * g.b0.rows) return; // the grid is sized for the wider role
     Tile t;
+    if constexpr (KSPLIT || FEW) {
+        __shared__ uint32_t ord[kInlineRows];
+        if (g.ids) {
+            if (!skinny_tile_of_ids(g, slot, t, ord)) return;
+            skinny_tile<Fmt, FACTORED, PACKED, 1, MBLK, KSPLIT, FEW>(g, t, skinny_lds, g.gate_up, sync, slot, ord);
+            return;
+        }
+    }
     if (g.tiles) {
         const uint32_t n_tiles = *g.n_tiles; // both loads are issued before either is needed
         t = g.tiles[slot];                   // the list has room for every launched slot
@@ -821,23 +894,31 @@ int qgemm_skinny_prepare() {
     return skinny_prepare_format<FmtFp8Row>();
 }
 
+// 8 wavefronts per workgroup: 128 output columns of gate AND up, or 256 of a single projection
+static int skinny_blocks_x(const GemmArgs &a) { return ceil_div((a.ksplit ? 2 : 1) * a.b0.rows, (a.gate_up ? 1 : 2) * kSkinnyWaves * 32); }
+// a launch of a few workgroups (unquantized weights: nothing to pin, see PIN)
+static bool skinny_few(const GemmArgs &g) {
+    return g.b0.packed && g.b0.mode != DMOE_QUANT_NONE && !g.ksplit && std::min(g.tile_m, g.max_rows) <= kSkinnyRowBlock &&
+           (size_t)skinny_blocks_x(g) * (size_t)g.max_tiles <= (size_t)kSkinnyFewGroups;
+}
+bool qgemm_skinny_takes_ids(const GemmArgs &g) {
+    return g.b0.packed && (g.ksplit || (g.b0.mode != DMOE_QUANT_NONE && std::min(g.tile_m, g.max_rows) <= kSkinnyRowBlock));
+}
+
 struct SkinnyLaunch {
     const GemmArgs &g;
     hipStream_t st;
     const GemmArgs *second = nullptr; // paired launch: the down projection behind the gate/up GEMM `g`
     template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool FEW = false>
     int go() {
-        // 8 wavefronts per workgroup: 128 output columns of gate AND up, or 256 of a single projection
-        auto blocks_x = [](const GemmArgs &a) { return ceil_div((a.ksplit ? 2 : 1) * a.b0.rows, (a.gate_up ? 1 : 2) * kSkinnyWaves * 32); };
+        auto blocks_x = [](const GemmArgs &a) { return skinny_blocks_x(a); };
         if constexpr (FACTORED && PACKED && !KSPLIT && !FEW && !std::is_same<Fmt, FmtAffine4Ordered>::value) {
             if (g.a_sums) return go<FmtAffine4Ordered, true, true>(); // validated by the launch functions
         }
         if constexpr (PACKED && !MBLK && !KSPLIT && !FEW && !std::is_same<Fmt, FmtAffine4Ordered>::value) {
             if (g.ksplit) return go<Fmt, FACTORED, PACKED, MBLK, true>(); // validated by the launch functions
-            if constexpr (Fmt::kVals > 8) // (unquantized weights: nothing to pin, see PIN)
-                if (!second && std::min(g.tile_m, g.max_rows) <= kSkinnyRowBlock &&
-                    (size_t)blocks_x(g) * (size_t)g.max_tiles <= (size_t)kSkinnyFewGroups)
-                    return go<Fmt, FACTORED, PACKED, MBLK, false, true>();
+            if constexpr (Fmt::kVals > 8)
+                if (!second && (g.ids || skinny_few(g))) return go<Fmt, FACTORED, PACKED, MBLK, false, true>();
         }
         auto kern = qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>;
         constexpr size_t zeros = skinny_reads_zeros(FACTORED, KSPLIT, FEW) ? skinny_zero_bytes(MBLK) : 0;
@@ -914,6 +995,8 @@ int launch_qgemm_skinny(const GemmArgs &g, hipStream_t st) {
                      "skinny GEMM: gate and up projections differ in shape or format");
     DMOE_REQUIRE(!g.ksplit || (g.tile_m <= kSkinnyRowBlock && qgemm_skinny_ksplit_ok(g.b0) && (!g.gate_up || qgemm_skinny_ksplit_ok(g.b1))),
                  "skinny GEMM: a split reduction needs packed weights and tiles of at most %d rows", kSkinnyRowBlock);
+    DMOE_REQUIRE(!g.ids || (qgemm_skinny_takes_ids(g) && g.n_ids <= kInlineRows && g.ids_experts >= 1 && g.dense_rows >= 0 && !g.tiles),
+                 "skinny GEMM: %u expert ids in place of a tile list", g.n_ids);
     DMOE_REQUIRE(!g.out_sums && !g.a_sums, "skinny GEMM: rows in code order are for the paired launch");
     if (g.max_tiles == 0) return DMOE_OK;
     if (g.b0.mode == DMOE_QUANT_NONE) return SkinnyLaunch{g, st}.template go<FmtBf16, false, true>();
