@@ -54,6 +54,16 @@ constexpr int skinny_wait_vmcnt(int n) { return 0x0f70 | (n & 15) | ((n >> 4) <<
 
 // the factored 4-bit form on activations that come in code order, with the sums beside them (GemmArgs::a_sums)
 struct FmtAffine4Ordered : FmtAffine4 {};
+// launches of a few rows (GemmArgs::ids) on more workgroups than a few, factored 4-bit form: the loads of the ring go where the
+// scheduler puts them, and the rows past a tile's end read zeros, as in the other launches of that size (8 tokens over 64 experts
+// 51.7 -> 47.2 us, a block of 4 / 8 tokens over 256 84.0 / 123 -> 80.5 / 121; the other formats are faster pinned: 8 tokens MXFP4 122
+// -> 112, 6 tokens 8-bit 195 -> 181)
+template <typename Fmt>
+struct Loose : Fmt {};
+template <typename Fmt>
+struct IsLoose : std::false_type {};
+template <typename Fmt>
+struct IsLoose<Loose<Fmt>> : std::true_type {};
 
 template <int NM>
 struct SkinnyStage {
@@ -139,19 +149,19 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     static_assert(ROUND % STAGES == 0 && (!MBLK || ROUND % 8 == 0), "rounds are whole turns of the ring");
     constexpr int NM = 1;                           // projections per wavefront
     constexpr bool ORDERED = std::is_same<Fmt, FmtAffine4Ordered>::value;
-    constexpr bool ZEROS = skinny_reads_zeros(FACTORED, KSPLIT, FEW);
+    constexpr bool ZEROS = skinny_reads_zeros(FACTORED, KSPLIT, FEW && !IsLoose<Fmt>::value);
     // Weight loads with a scalar base (ChunkStream::load_at) where the launch fills the chip: 509 tokens on MXFP4 675 -> 666 us, 64
     // tokens on MXFP4 129 -> 126.5, on 8-bit 479 -> 473; not for the scales of the factored form's small tiles (64 tokens 255.4 ->
     // 252.3 with the chunks alone, 257.0 with both), nor in launches of a few workgroups (8 tokens, 64 experts 49.2 -> 50.7; one
     // token 45.1 -> 45.7; the small layer 32.6 -> 32.0).
-    constexpr bool SCALAR = PACKED && !KSPLIT && !FEW, SCALAR_META = SCALAR && !(FACTORED && RJT == 1);
+    constexpr bool SCALAR = PACKED && !KSPLIT && !(FEW && !IsLoose<Fmt>::value), SCALAR_META = SCALAR && !(FACTORED && RJT == 1);
     // Launches of a few workgroups are paced by each wavefront's own chain of steps, and the look-ahead has to be in the machine
     // code: left alone, the scheduler gathers the loads of a round behind its fourth step and waits for nearly all of them at
     // the next one's start, where in the round depending on what surrounds it. Each step's loads are pinned to its head (small
     // layer, 16 tokens 34.5 -> 33.0 us; hidden 4096, 1 / 2 tokens: 4-bit 34.8 / 49.2 -> 32.9 / 47.6, MXFP4 34.0 / 47.2 -> 31.3 / 44.1,
     // 8-bit 45.6 / 78.3 -> 44.7 / 69.9). Not where the launch fills the chip: there a wavefront's gathered loads are no loss (24 to
     // 64 tokens, 4-bit: pinned 0 to 2 % slower), and not on unquantized weights (32 instructions per round, level).
-    constexpr bool PIN = (KSPLIT || FEW) && KV > 8;
+    constexpr bool PIN = (KSPLIT || FEW) && KV > 8 && !IsLoose<Fmt>::value;
     constexpr int WAVES = 2 * kSkinnyWaves;         // eight wavefronts share one staging of the tile's activations
     const int cg = gate_up ? kSkinnyWaves : WAVES;  // 32-row blocks of weight rows per workgroup
     const int tid = (int)threadIdx.x, lane = tid & 63, ln = lane & 31, h = lane >> 5;
@@ -394,11 +404,13 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         issue_x(0);
 #pragma unroll
         for (int mi = 0; mi < NM; ++mi) cs[mi].pin(); // keeps the weight loads behind the requests above
+        // (PIN: past the last step that one again, never used: a request that may or may not have been made is one that the waits of
+        // the rounds below cannot count on, and the first step of each round then waits for all but a few loads)
 #pragma unroll
         for (int j = 0; j < PRE; ++j)
-            if (j < n_loc) load_stage(j, ring[j], j % LG);
+            if (PIN || j < n_loc) load_stage(PIN && j >= n_loc ? n_loc - 1 : j, ring[j], j % LG);
         // every ring stage holds at least NM loads younger than the activation requests
-        if (n_loc >= PRE) __builtin_amdgcn_s_waitcnt(skinny_wait_vmcnt(PRE * NM));
+        if (PIN || n_loc >= PRE) __builtin_amdgcn_s_waitcnt(skinny_wait_vmcnt(PRE * NM));
         else __builtin_amdgcn_s_waitcnt(skinny_wait_vmcnt(0));
     }
     if (ORDERED) place_sums();
@@ -769,7 +781,8 @@ __device__ __forceinline__ bool skinny_tile_of_ids(const GemmArgs &g, uint32_t s
 template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool FEW = false>
 __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(GemmArgs a, GemmArgs b, int paired) {
     extern __shared__ __attribute__((aligned(16))) uint8_t skinny_lds[];
-    const bool second = paired && blockIdx.y >= (uint32_t)a.max_tiles; // workgroup-uniform
+    constexpr bool SINGLE = KSPLIT || FEW; // kernels of single launches
+    const bool second = !SINGLE && paired && blockIdx.y >= (uint32_t)a.max_tiles; // workgroup-uniform
     // The role's arguments, read from the kernel-argument segment with a uniform index (`a` sits at offset 0 and `b`
     // right behind it): taking the address of `a` or `b` instead would move both structs to scratch memory.
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -780,18 +793,19 @@ __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(Gem
 #endif
     (void)b;
     const uint32_t slot = blockIdx.y - (second ? (uint32_t)a.max_tiles : 0u);
-    const int sync = !paired ? kSkinnySyncNone : second ? kSkinnySyncWait : kSkinnySyncSignal;
+    const int sync = SINGLE || !paired ? kSkinnySyncNone : second ? kSkinnySyncWait : kSkinnySyncSignal;
     if ((int)blockIdx.x * (g.gate_up ? 1 : 2) * kSkinnyWaves * 32 >= (KSPLIT ? 2 : 1) * g.b0.rows) return; // the grid is sized for the wider role
     Tile t;
+    const uint32_t *rows_of_ids = nullptr; // the workgroup's own order of the rows
     if constexpr (KSPLIT || FEW) {
         __shared__ uint32_t ord[kInlineRows];
         if (g.ids) {
             if (!skinny_tile_of_ids(g, slot, t, ord)) return;
-            skinny_tile<Fmt, FACTORED, PACKED, 1, MBLK, KSPLIT, FEW>(g, t, skinny_lds, g.gate_up, sync, slot, ord);
-            return;
+            rows_of_ids = ord;
         }
     }
-    if (g.tiles) {
+    if (rows_of_ids) {
+    } else if (g.tiles) {
         const uint32_t n_tiles = *g.n_tiles; // both loads are issued before either is needed
         t = g.tiles[slot];                   // the list has room for every launched slot
         if (slot >= n_tiles) return;
@@ -805,7 +819,7 @@ __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(Gem
         t.nrows = left < (uint32_t)g.tile_m ? left : (uint32_t)g.tile_m;
     }
     if (KSPLIT || FEW) { // the launcher builds no tile above one row block for these kernels
-        skinny_tile<Fmt, FACTORED, PACKED, 1, MBLK, KSPLIT, FEW>(g, t, skinny_lds, g.gate_up, sync, slot);
+        skinny_tile<Fmt, FACTORED, PACKED, 1, MBLK, KSPLIT, FEW>(g, t, skinny_lds, g.gate_up, sync, slot, rows_of_ids);
         return;
     }
     if (__builtin_amdgcn_readfirstlane((int)t.nrows) <= kSkinnyRowBlock)
@@ -878,6 +892,7 @@ static int skinny_prepare_format() {
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, true, false, true>()));
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, true, false, false, true>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, true, false, false, true>()));
+    if constexpr (can_factor) DMOE_TRY((skinny_raise_limit<Loose<Fmt>, true, true, false, false, true>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, true, false, true>()));
     DMOE_TRY((skinny_raise_limit<Fmt, can_factor, false, has_entries>()));
     DMOE_TRY((skinny_raise_limit<Fmt, false, false, has_entries>()));
@@ -918,10 +933,12 @@ struct SkinnyLaunch {
         if constexpr (PACKED && !MBLK && !KSPLIT && !FEW && !std::is_same<Fmt, FmtAffine4Ordered>::value) {
             if (g.ksplit) return go<Fmt, FACTORED, PACKED, MBLK, true>(); // validated by the launch functions
             if constexpr (Fmt::kVals > 8)
-                if (!second && (g.ids || skinny_few(g))) return go<Fmt, FACTORED, PACKED, MBLK, false, true>();
+                if (!second && skinny_few(g)) return go<Fmt, FACTORED, PACKED, MBLK, false, true>();
+            if constexpr (Fmt::kVals > 8)
+                if (g.ids) return go<typename std::conditional<FACTORED, Loose<Fmt>, Fmt>::type, FACTORED, PACKED, MBLK, false, true>();
         }
         auto kern = qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>;
-        constexpr size_t zeros = skinny_reads_zeros(FACTORED, KSPLIT, FEW) ? skinny_zero_bytes(MBLK) : 0;
+        constexpr size_t zeros = skinny_reads_zeros(FACTORED, KSPLIT, FEW && !IsLoose<Fmt>::value) ? skinny_zero_bytes(MBLK) : 0;
         const size_t lds = skinny_lds_bytes(g.b0, MBLK, zeros);
         DMOE_TRY((skinny_raise_limit<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>())); // done by dmoe_init for its device; a flag test otherwise
         dim3 block(2 * kSkinnyWaves * 64);
