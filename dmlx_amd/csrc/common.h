@@ -278,6 +278,7 @@ struct GemmArgs {
     int ids_k = 0;                  // source row of row i: i / ids_k, of dense row j: j (0: the sorted row itself)
     const uint32_t *ids_lhs = nullptr; // optional map of the source rows
     bool ids_scatter = false;       // outputs and row_scale go by the original row, else outputs stay sorted
+    int waves_log2 = 3;             // wavefronts of a workgroup of such a launch (set by its launcher)
     uint32_t *order_out = nullptr;  // optional: the original row of every sorted row
     uint32_t *bad_ids = nullptr;
 };

@@ -162,8 +162,14 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     // 8-bit 45.6 / 78.3 -> 44.7 / 69.9). Not where the launch fills the chip: there a wavefront's gathered loads are no loss (24 to
     // 64 tokens, 4-bit: pinned 0 to 2 % slower), and not on unquantized weights (32 instructions per round, level).
     constexpr bool PIN = (KSPLIT || FEW) && KV > 8 && !IsLoose<Fmt>::value;
-    constexpr int WAVES = 2 * kSkinnyWaves;         // eight wavefronts share one staging of the tile's activations
-    const int cg = gate_up ? kSkinnyWaves : WAVES;  // 32-row blocks of weight rows per workgroup
+    // Eight wavefronts share one staging of the tile's activations. A compute unit fetches no more than 40 GB/s, however many
+    // loads its wavefronts have in flight, so a launch of a few workgroups is spread over more of them: workgroups of four or two
+    // wavefronts as long as that makes at most kSkinnyFewGroups (us per step: small layer on MXFP4 25.5 -> 24.4, 4 tokens over 64
+    // experts, 4-bit in groups of 32 37.2 -> 30.7). Not the factored form, whose re-ordering pass over LDS a workgroup's threads share
+    // (small layer 33.1 -> 34.6).
+    const int wlog = FEW && !FACTORED ? g.waves_log2 : 3;
+    const int WAVES = 1 << wlog;
+    const int cg = gate_up ? WAVES >> 1 : WAVES;    // 32-row blocks of weight rows per workgroup
     const int tid = (int)threadIdx.x, lane = tid & 63, ln = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cols = g.b0.cols, n_out = g.b0.rows;
@@ -652,7 +658,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         // exchange areas) and leave as 8-byte pieces of a row, one or two per thread. Output rows that cannot be cut
         // into such pieces keep the direct stores.
         const bool wide_out = (n_out & 3) == 0 && (g.ldo & 3) == 0 && ((uintptr_t)g.out & 7) == 0;
-        const int cw_shift = (gate_up ? 7 : 8) - (ks ? 1 : 0); // log2 of the workgroup's output columns
+        const int cw_shift = 5 + wlog - (gate_up ? 1 : 0) - (ks ? 1 : 0); // log2 of the workgroup's output columns
         uint16_t *const stage = (uint16_t *)(skinny_lds + kSkinnyStageOffset); // [tile rows][columns of the workgroup]
         if (wide_out && !gate_up && !ks) __syncthreads(); // (the other roles have met at a barrier since the main loop)
         const bool order_out = ORDERED && g.out_sums != nullptr; // whole 64s of columns, see the launch functions
@@ -794,7 +800,8 @@ __global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(Gem
     (void)b;
     const uint32_t slot = blockIdx.y - (second ? (uint32_t)a.max_tiles : 0u);
     const int sync = SINGLE || !paired ? kSkinnySyncNone : second ? kSkinnySyncWait : kSkinnySyncSignal;
-    if ((int)blockIdx.x * (g.gate_up ? 1 : 2) * kSkinnyWaves * 32 >= (KSPLIT ? 2 : 1) * g.b0.rows) return; // the grid is sized for the wider role
+    // the grid is sized for the wider role
+    if ((int)blockIdx.x * (((g.gate_up ? 1 : 2) * kSkinnyWaves * 32) >> (FEW && !FACTORED ? 3 - g.waves_log2 : 0)) >= (KSPLIT ? 2 : 1) * g.b0.rows) return;
     Tile t;
     const uint32_t *rows_of_ids = nullptr; // the workgroup's own order of the rows
     if constexpr (KSPLIT || FEW) {
@@ -941,6 +948,14 @@ struct SkinnyLaunch {
         constexpr size_t zeros = skinny_reads_zeros(FACTORED, KSPLIT, FEW && !IsLoose<Fmt>::value) ? skinny_zero_bytes(MBLK) : 0;
         const size_t lds = skinny_lds_bytes(g.b0, MBLK, zeros);
         DMOE_TRY((skinny_raise_limit<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>())); // done by dmoe_init for its device; a flag test otherwise
+        if constexpr (FEW && !FACTORED) {
+            GemmArgs a = g;
+            while (a.waves_log2 > 1 && ((size_t)blocks_x(g) * (size_t)g.max_tiles << (4 - a.waves_log2)) <= (size_t)kSkinnyFewGroups) --a.waves_log2;
+            const int cols = ((g.gate_up ? 1 : 2) * kSkinnyWaves * 32) >> (3 - a.waves_log2);
+            hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(g.b0.rows, cols), (unsigned)g.max_tiles), dim3(64u << a.waves_log2), lds, st, a, a, 0);
+            DMOE_LAUNCH_CHECK();
+            return DMOE_OK;
+        }
         dim3 block(2 * kSkinnyWaves * 64);
         if (second) {
             GemmArgs a = g, b = *second;
