@@ -255,7 +255,7 @@ static bool layer_small_path(const Layer *L, size_t rows) {
 
 struct FwdLayout {
     size_t order, inv, token, sorted_e, counts, offsets, live, n_live, tiles, n_tiles, tile_done, scratch;
-    size_t h, y, sh_h, sh_y, xo, xs, hs, total;
+    size_t h, y, sh_h, sh_y, idx, wts, xo, xs, hs, plain, total;
     int max_tiles, tile_m;
     bool small;
     // Paired launch of 4-bit affine weights whose scales are factored out: the rows of both roles come in code order with their
@@ -319,7 +319,7 @@ static bool fold_prefill(const Layer *L, int T) {
     return routed + (size_t)ceil_div(T, kMfmaTileM) * strips <= 256 || (bf16 && routed >= 1024);
 }
 
-static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean, bool fixed) {
+static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean, bool fixed, bool routing) {
     FwdLayout f;
     Bump b;
     size_t n = (size_t)T * L->K;
@@ -360,6 +360,9 @@ static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean,
     f.y = b.take(rows * (size_t)L->D * 2);
     f.sh_h = b.take(L->has_shared && !f.fold ? (size_t)T * L->Fs * 2 : 0);
     f.sh_y = b.take(L->has_shared && !f.fold ? (size_t)T * L->D * 2 : 0);
+    f.idx = b.take(routing ? n * 4 : 0);
+    f.wts = b.take(routing ? n * 4 : 0);
+    f.plain = b.off; // what a call cannot do without: see fit_workspace
     f.ordered = f.small && !fixed && rows > (size_t)kPairMinRows && n >= (size_t)kOrderedAvgRows * (size_t)L->E && qgemm_skinny_factored(L->gate.view) && qgemm_skinny_factored(L->down.view) &&
                 L->D % 64 == 0 && L->F % 64 == 0;
     f.xo = b.take(f.ordered ? (size_t)T * L->D * 2 : 0);
@@ -372,17 +375,26 @@ static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean,
 constexpr size_t kStaticScratchBytes = (size_t)16 << 20;
 constexpr size_t kStaticFlagBytes = 256; // the workspace's flag words sit in front of the bump area
 
-// scratch of a whole call on the static array: the forward's buffers, then the routing outputs
-static size_t static_need(const Layer *L, int T, const FwdLayout &f) {
-    return f.total + 2 * (((size_t)T * L->K * 4 + 255) & ~(size_t)255);
-}
-
 // `fixed`: scratch is the static array. Small tiles and a folded shared expert lengthen the lists by a few bytes per token;
 // the largest batches that fit without them are planned without them, so that they still fit.
-static FwdLayout forward_layout(const Layer *L, int T, bool with_shared = true, bool fixed = false) {
-    const FwdLayout f = plan_layout(L, T, with_shared, false, fixed);
-    if (fixed && static_need(L, T, f) > kStaticScratchBytes - kStaticFlagBytes) return plan_layout(L, T, with_shared, true, fixed);
+// `routing`: the call's routing outputs are part of the layout (a call on the static array always has them).
+static FwdLayout forward_layout(const Layer *L, int T, bool with_shared, bool fixed, bool routing) {
+    const FwdLayout f = plan_layout(L, T, with_shared, false, fixed, routing);
+    if (fixed && f.total > kStaticScratchBytes - kStaticFlagBytes) return plan_layout(L, T, with_shared, true, fixed, routing);
     return f;
+}
+
+// The areas of the code order lie behind everything else and are taken only between 4 and 16 rows per expert, so a block that
+// was sized for the plain buffers, or by a larger batch, may be too short for them alone. It does not grow for their sake (growth
+// waits for the device, cannot be captured, and leaves graphs captured earlier with freed addresses): such a call runs
+// without them, with the same bits. A block that has to grow anyway takes them in.
+static int fit_workspace(dmoe_workspace ws, FwdLayout &f, Workspace **out) {
+    const Workspace *w = (const Workspace *)ws.ctx;
+    if (f.ordered && w && f.plain <= w->bytes && f.total > w->bytes) {
+        f.ordered = false;
+        f.total = f.plain;
+    }
+    return workspace_reserve(ws, f.total, out);
 }
 
 // `few` = few rows per expert (only read for unquantized weights; the quantized formats have `small`)
@@ -811,10 +823,10 @@ int dmoe_layer_destroy(dmoe_layer layer) {
 }
 
 // `route` (optional): the gate's selection has not run yet and is to share a launch with the packing; it fills
-// d_indices and d_scores (= route->out_idx, route->out_w) on the way.
+// d_indices and d_scores (= route->out_idx, route->out_w) on the way. `routing`: the caller's layout holds the routing outputs.
 static int forward_common(uint16_t *d_out, uint16_t *y_out, Layer *L, const uint16_t *d_x, const uint32_t *d_indices,
                           const float *d_scores, int T, bool apply_remap, bool with_shared, dmoe_workspace ws,
-                          dmoe_stream s, const RouteArgs *route = nullptr) {
+                          dmoe_stream s, bool routing = false, const RouteArgs *route = nullptr) {
     DMOE_REQUIRE(T >= 0, "forward: T=%d", T);
     if (T == 0) return DMOE_OK;
     DMOE_REQUIRE(d_x && d_indices, "forward: null pointer");
@@ -822,9 +834,9 @@ static int forward_common(uint16_t *d_out, uint16_t *y_out, Layer *L, const uint
     DMOE_REQUIRE(y_out || (d_out && ((uintptr_t)d_out % 16) == 0), "forward: out must be 16-byte aligned and non-null");
     hipStream_t st = to_hip(s);
     const bool fixed = ws.ctx && ((const Workspace *)ws.ctx)->fixed;
-    FwdLayout f = forward_layout(L, T, with_shared && !y_out, fixed);
+    FwdLayout f = forward_layout(L, T, with_shared && !y_out, fixed, routing);
     Workspace *w = nullptr;
-    DMOE_TRY(workspace_reserve(ws, f.total, &w));
+    DMOE_TRY(fit_workspace(ws, f, &w));
     w->last_with_shared = with_shared && !y_out;
     DMOE_TRY(stage_begin(w, DMOE_STAGE_PACK, st));
     const bool remap = apply_remap && L->remap;
@@ -887,25 +899,21 @@ int dmoe_moe_layer_forward(uint16_t *d_out, uint32_t *d_out_indices, float *d_ou
     if (L->remap) DMOE_REQUIRE(E_total == L->n_total, "moe_layer_forward: E_total %d != remap length %d", E_total, L->n_total);
     else DMOE_REQUIRE(E_total == L->E, "moe_layer_forward: E_total %d != resident experts %d", E_total, L->E);
     // routing outputs live in caller memory when given, else in a private tail of the workspace
-    FwdLayout f = forward_layout(L, T, true, ws.ctx && ((const Workspace *)ws.ctx)->fixed);
-    size_t n = (size_t)T * L->K;
-    Bump b;
-    b.off = f.total;
-    size_t o_idx = b.take(n * 4), o_w = b.take(n * 4);
+    FwdLayout f = forward_layout(L, T, true, ws.ctx && ((const Workspace *)ws.ctx)->fixed, true);
     Workspace *w = nullptr;
-    DMOE_TRY(workspace_reserve(ws, b.off, &w));
-    uint32_t *idx = d_out_indices ? d_out_indices : at<uint32_t>(w, o_idx);
-    float *wts = d_out_weights ? d_out_weights : at<float>(w, o_w);
+    DMOE_TRY(fit_workspace(ws, f, &w));
+    uint32_t *idx = d_out_indices ? d_out_indices : at<uint32_t>(w, f.idx);
+    float *wts = d_out_weights ? d_out_weights : at<float>(w, f.wts);
     RouteArgs r;
     r.out_idx = idx, r.out_w = wts, r.scores = d_scores, r.bias = d_bias, r.resident = d_resident_mask;
     r.T = T, r.E = E_total, r.K = L->K, r.normalize = renorm, r.apply_scale = 1, r.route_scale = route_scale;
     DMOE_REQUIRE(d_scores != nullptr, "moe_layer_forward: scores is null");
     // one or two sequences: the selection shares a launch with the packing (and is timed as the packing stage)
-    if (route_pack_tiny_supports(r)) return forward_common(d_out, nullptr, L, d_x, idx, wts, T, true, true, ws, s, &r);
+    if (route_pack_tiny_supports(r)) return forward_common(d_out, nullptr, L, d_x, idx, wts, T, true, true, ws, s, true, &r);
     DMOE_TRY(stage_begin(w, DMOE_STAGE_ROUTE, to_hip(s)));
     DMOE_TRY(launch_route(r, to_hip(s)));
     DMOE_TRY(stage_end(w, DMOE_STAGE_ROUTE, to_hip(s)));
-    return forward_common(d_out, nullptr, L, d_x, idx, wts, T, true, true, ws, s);
+    return forward_common(d_out, nullptr, L, d_x, idx, wts, T, true, true, ws, s, true);
 }
 
 int dmoe_moe_layer_forward_static(uint16_t *d_out, uint32_t *d_out_indices, float *d_out_weights, dmoe_layer layer,
@@ -920,7 +928,7 @@ int dmoe_moe_layer_forward_static(uint16_t *d_out, uint32_t *d_out_indices, floa
     DMOE_REQUIRE(L->device == w->device, "moe_layer_forward_static: the layer lives on device %d, the current device is %d",
                  L->device, w->device);
     // same layout as dmoe_moe_layer_forward
-    const size_t need = static_need(L, T, forward_layout(L, T, true, true));
+    const size_t need = forward_layout(L, T, true, true, true).total;
     DMOE_REQUIRE(need <= w->bytes,
                  "moe_layer_forward_static: T=%d tokens need %zu bytes of scratch memory, the static device scratch holds "
                  "%zu (use dmoe_moe_layer_forward with a workspace for larger batches)", T, need, w->bytes);
@@ -934,8 +942,8 @@ int dmoe_debug_last_activations(uint16_t *d_out, dmoe_layer layer, int T, dmoe_w
     DMOE_REQUIRE(layer.ctx && ws.ctx && d_out, "debug_last_activations: null argument");
     Layer *L = (Layer *)layer.ctx;
     Workspace *w = (Workspace *)ws.ctx;
-    FwdLayout f = forward_layout(L, T, w->last_with_shared);
-    DMOE_REQUIRE(w->bytes >= f.total, "debug_last_activations: no forward of this size has run on the workspace");
+    const FwdLayout f = forward_layout(L, T, w->last_with_shared, false, false);
+    DMOE_REQUIRE(w->bytes >= f.plain, "debug_last_activations: no forward of this size has run on the workspace");
     size_t n = (size_t)T * L->K, rv = (size_t)L->F / 8, total = n * rv;
     if (total == 0) return DMOE_OK;
     hipLaunchKernelGGL(scatter_rows_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, to_hip(s),
