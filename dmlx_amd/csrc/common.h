@@ -279,6 +279,7 @@ struct GemmArgs {
     const uint32_t *ids_lhs = nullptr; // optional map of the source rows
     bool ids_scatter = false;       // outputs and row_scale go by the original row, else outputs stay sorted
     int waves_log2 = 3;             // wavefronts of a workgroup of such a launch (set by its launcher)
+    bool third_group = false;       // paired launch, 8-bit affine: three workgroups per compute unit (see pair_third_group)
     uint32_t *order_out = nullptr;  // optional: the original row of every sorted row
     uint32_t *bad_ids = nullptr;
 };

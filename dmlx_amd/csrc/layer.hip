@@ -5,6 +5,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -253,6 +254,19 @@ static bool layer_small_path(const Layer *L, size_t rows) {
     return rows <= (size_t)(tile <= 16 ? 8 : 12) * (size_t)L->E;
 }
 
+// Workgroups per compute unit of a paired 8-bit launch, three or two. The third one pays only as a producer: with fewer gate/up
+// workgroups than three slots on each compute unit it is a down workgroup that waits from the start, its weight loads in
+// everyone's way. us per step, 8-bit affine, two | three: hidden 2048, ffn 1408, 64 experts top-6, 11 / 64 tokens 88 / 116 | 109 / 132, hidden
+// 1024, ffn 1024, 128 experts, 20 tokens 62.5 | 74.8, hidden 2048, ffn 3072, 64 experts top-4, 32 tokens 186 | 204. It gains where a tile's
+// strips are a multiple of 8, the XCDs, so that the down strips of every tile meet on the same ones, reductions up to 2048 that leave LDS for
+// it: hidden 1024, ffn 2048, 128 experts, 16 / 64 tokens 121 / 198 | 113 / 186, hidden 2048, 64 experts, 32 tokens 159 | 150.
+static bool pair_third_group(const Layer *L, size_t n) {
+    const int strips = std::max(ceil_div(L->F, 128), ceil_div(L->D, 256));
+    if (strips % 8 != 0 || L->D > 2048 || L->F > 2048) return false;
+    const double live = L->E * (1.0 - std::exp(-(double)n / L->E)); // experts with rows, if the routing is even
+    return live * ceil_div(L->F, 128) > 3 * 256;
+}
+
 struct FwdLayout {
     size_t order, inv, token, sorted_e, counts, offsets, live, n_live, tiles, n_tiles, tile_done, scratch;
     size_t h, y, sh_h, sh_y, idx, wts, xo, xs, hs, plain, total;
@@ -489,6 +503,7 @@ static int routed_forward(const Layer *L, Workspace *w, const FwdLayout &f, cons
     // workgroup is resident from the start, no down workgroup can begin before they end, and what the single launch
     // adds is the hand-over through memory - stores acknowledged, counter, poll - of 6-8 us per step.)
     const bool pair = f.small && w->paired && n + (f.fold ? (size_t)T : 0) > (size_t)kPairMinRows && qgemm_skinny_pair_supports(gu, dn);
+    gu.third_group = pair_third_group(L, n);
     w->last_ordered = pair && f.ordered;
     if (w->last_ordered) {
         po.rows_in = (const uint4 *)d_x;

@@ -108,11 +108,17 @@ constexpr size_t skinny_lds_bytes(int cols, int kstep, bool mblk, size_t zeros) 
     const size_t window = skinny_turn_offset(cols, kstep) + (mblk ? 0 : zeros), least = kSkinnyStageOffset + kSkinnyStageBytes;
     return (window > least ? window : least) + (mblk ? kSkinnyTurnBytes + zeros : 0);
 }
-// A kernel without zeros pays nothing for them: 8-bit reductions of 3072 keep three workgroups on a compute unit (160 KiB,
-// handed out in pieces of 1280 bytes) and those of 4768 two.
+// A kernel without zeros pays nothing for them: reductions of 3072 in 8 bits leave LDS for three workgroups on a compute unit
+// (160 KiB, handed out in pieces of 1280 bytes) and those of 4768 for two.
 constexpr size_t skinny_lds_share(size_t bytes) { return (bytes + 1279) / 1280 * 1280; }
 static_assert(3 * skinny_lds_share(skinny_lds_bytes(3072, 32, false, 0)) <= 160 * 1024 &&
               2 * skinny_lds_share(skinny_lds_bytes(4768, 32, false, 0)) <= 160 * 1024, "workgroups per compute unit");
+// Registers for three workgroups, six wavefronts per SIMD, on the 8-bit launches that fill the chip (the compiler left to itself takes
+// 81, one too many). Whether the third one is wanted is the launch's choice: what keeps it out is LDS asked for and not used.
+template <typename Fmt, bool PACKED, bool KSPLIT, bool FEW>
+constexpr bool skinny_counts_groups() { return std::is_same<Fmt, FmtAffine8>::value && PACKED && !KSPLIT && !FEW; }
+constexpr size_t kSkinnyTwoGroupsLds = 55040;
+static_assert(3 * skinny_lds_share(kSkinnyTwoGroupsLds) > 160 * 1024 && 2 * skinny_lds_share(kSkinnyTwoGroupsLds) <= 160 * 1024, "two workgroups");
 
 // MBLK (MLX layout only): the scale / bias entries of a row are not fetched one per step (32 cache lines touched per
 // load for 2 useful bytes each, again at every step: these loads, not the weights, bounded the MLX-layout path) but 16
@@ -785,7 +791,7 @@ __device__ __forceinline__ bool skinny_tile_of_ids(const GemmArgs &g, uint32_t s
 // FEW: a single launch of at most kSkinnyFewGroups workgroups and of tiles of one row block. It is paced by each workgroup's own
 // chain, not by bandwidth or power: the ring's loads are pinned (see PIN), no zeros, no copies for larger tiles.
 template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool FEW = false>
-__global__ __launch_bounds__(2 * kSkinnyWaves * 64) void qgemm_skinny_kernel(GemmArgs a, GemmArgs b, int paired) {
+__global__ __launch_bounds__(2 * kSkinnyWaves * 64, (skinny_counts_groups<Fmt, PACKED, KSPLIT, FEW>() ? 6 : 1)) void qgemm_skinny_kernel(GemmArgs a, GemmArgs b, int paired) {
     extern __shared__ __attribute__((aligned(16))) uint8_t skinny_lds[];
     constexpr bool SINGLE = KSPLIT || FEW; // kernels of single launches
     const bool second = !SINGLE && paired && blockIdx.y >= (uint32_t)a.max_tiles; // workgroup-uniform
@@ -957,16 +963,20 @@ struct SkinnyLaunch {
             return DMOE_OK;
         }
         dim3 block(2 * kSkinnyWaves * 64);
+        // (single launches, us for 8-bit [256, 1024, 512] 300 rows two | three groups 26.1 | 24.6, [128, 1024, 2048] 512 rows 54.1 | 54.0, but
+        // [128, 2048, 3072] 192 rows 117 | 123)
+        constexpr bool counts = skinny_counts_groups<Fmt, PACKED, KSPLIT, FEW>();
+        const size_t least = counts && !(second ? g.third_group : g.b0.cols <= 2048) ? kSkinnyTwoGroupsLds : 0;
         if (second) {
             GemmArgs a = g, b = *second;
             a.tile_done_target = b.tile_done_target = (uint32_t)blocks_x(g);
             b.tile_done = a.tile_done;
-            const size_t lds2 = std::max(lds, skinny_lds_bytes(second->b0, MBLK, zeros));
+            const size_t lds2 = std::max({lds, skinny_lds_bytes(second->b0, MBLK, zeros), least});
             dim3 grid((unsigned)std::max(blocks_x(a), blocks_x(b)), (unsigned)(2 * g.max_tiles));
             hipLaunchKernelGGL(kern, grid, block, lds2, st, a, b, 1);
         } else {
             dim3 grid((unsigned)blocks_x(g), (unsigned)g.max_tiles);
-            hipLaunchKernelGGL(kern, grid, block, lds, st, g, g, 0);
+            hipLaunchKernelGGL(kern, grid, block, std::max(lds, least), st, g, g, 0);
         }
         DMOE_LAUNCH_CHECK();
         return DMOE_OK;

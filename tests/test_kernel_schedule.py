@@ -2,6 +2,7 @@
 really there. A wavefront requests the weights of step s + 5 at the head of step s; the instruction scheduler, left alone, gathers
 the requests of a whole round at its end and waits for nearly all of them at once, which costs a launch of this kind up to 8 %
 and changes with unrelated edits. Compiles one file for the device (no GPU needed) and reads the main loops."""
+import functools
 import os
 import re
 import shutil
@@ -13,6 +14,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 STEPS = 6  # of a round: the ring's stages
 
 
+@functools.lru_cache(maxsize=None)
 def _device_asm(source):
     with open(os.path.join(CSRC, "Makefile")) as f:
         text = f.read().replace("\\\n", " ")
@@ -72,3 +74,17 @@ def test_few_workgroup_launches_keep_their_look_ahead():
         seen[m.groups()] = True
     # split reduction and few-workgroup launch of: 4-bit affine (scales factored out, and not), 8-bit affine, MXFP4, FP8 per row
     assert len(seen) == 10, sorted(seen)
+
+
+@pytest.mark.skipif(shutil.which(os.environ.get("HIPCC", "hipcc")) is None, reason="needs hipcc")
+def test_eight_bit_launches_leave_registers_for_three_workgroups():
+    """The packed 8-bit kernel of launches that fill the chip: six wavefronts per SIMD (512 registers, handed out by eight), three
+    workgroups of eight wavefronts on a compute unit, and nothing spilled for it. The LDS side is asserted in the source."""
+    seen = 0
+    for entry in _device_asm("qgemm_skinny.hip").split("  - .agpr_count:")[1:]:
+        if "qgemm_skinny_kernelINS_10FmtAffine8ELb0ELb1ELb0ELb0ELb0EEE" not in entry:
+            continue
+        get = lambda key: int(re.search(rf"\.{key}:\s*(\d+)", entry).group(1))
+        assert get("vgpr_count") <= 512 // 6 // 8 * 8 and get("vgpr_spill_count") == 0 and get("private_segment_fixed_size") == 0
+        seen += 1
+    assert seen == 1
