@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -222,6 +223,27 @@ static size_t inline_rows(const QView &b) {
     if (!b.packed || b.mode == DMOE_QUANT_NONE) return 0;
     return b.mode == DMOE_QUANT_MXFP4 || qgemm_skinny_factored(b) ? kInlineRows : kInlineRows * 3 / 4;
 }
+// Above kSkinnyFewGroups workgroups that only pays while the smaller tiles do not make the launches much longer: an expert of more
+// than 8 rows is read again for each further tile, and what counts is rounds of a workgroup per compute unit, each as long as its
+// reduction. Expected tiles of `n` rows over `E` experts: one each, or (n / 8 + E / 2: the last one half full) more. Rows of few, wide
+// experts, over 16 routings, time of the tile list over this: one projection [4, 14336, 4096], MXFP4 / 4-bit, 16 rows 1.08 / 1.12, 28
+// 0.73 / 0.85, 64 0.60 / 0.74; [8, 14336, 4096], 40 rows 1.07 / 1.09, 64 0.81 / 0.79; layers, hidden and ffn 4096, top-2, MXFP4: 6 experts, 12
+// tokens 1.22, 32 tokens 0.82, 8 experts 1.12 and 0.86; ffn 6144 and hidden 2048, 4 experts, 32 tokens 1.12. The 4-bit layers, whose
+// larger tiles are the slower ones, gain further (4096, 4 experts, 32 tokens 1.19). Over 860 such points the line costs 0.4 %
+// against the better side of each, always this 1.8 % (at most 40).
+struct LaunchShape {
+    int strips, cols;
+};
+static bool one_block_tiles_pay(size_t n, int E, size_t dense_tiles, size_t dense_tiles_of_list, std::initializer_list<LaunchShape> launches, size_t num,
+                                size_t den) {
+    const size_t live = std::min(n, (size_t)E), tiles = std::max(live, std::min(n, (n + 4 * (size_t)E + 7) / 8));
+    size_t cost = 0, list = 0;
+    for (const LaunchShape &l : launches) {
+        cost += ((tiles + dense_tiles) * (size_t)l.strips + kSkinnyFewGroups - 1) / kSkinnyFewGroups * (size_t)l.cols;
+        list += ((live + dense_tiles_of_list) * (size_t)l.strips + kSkinnyFewGroups - 1) / kSkinnyFewGroups * (size_t)l.cols;
+    }
+    return cost * den <= list * num;
+}
 
 static bool few_rows(size_t rows, int n_experts) { return rows <= (size_t)kSkinnyAvgRows * (size_t)n_experts; }
 static bool use_small_path(size_t rows, int n_experts, const QView &b) {
@@ -350,7 +372,11 @@ static FwdLayout plan_layout(const Layer *L, int T, bool with_shared, bool lean,
         // (the widest launch decides: gate/up takes 128 output columns per workgroup, down 256)
         const size_t strips = (size_t)std::max(ceil_div(L->F, 128), ceil_div(L->D, 256));
         const size_t tiles = (size_t)pack_max_tiles(n, L->E, kSplitTileM) + (f.fold ? (size_t)ceil_div(T, kSplitTileM) : 0);
-        f.few = !lean && (tiles * strips <= (size_t)kSkinnyFewGroups || rows <= std::min(inline_rows(L->gate.view), inline_rows(L->down.view)));
+        const bool factored = qgemm_skinny_factored(L->gate.view) && qgemm_skinny_factored(L->down.view);
+        f.few = !lean && (tiles * strips <= (size_t)kSkinnyFewGroups ||
+                          (rows <= std::min(inline_rows(L->gate.view), inline_rows(L->down.view)) &&
+                           one_block_tiles_pay(n, L->E, f.fold ? (size_t)ceil_div(T, kSplitTileM) : 0, f.fold ? (size_t)ceil_div(T, f.tile_m) : 0,
+                                               {{ceil_div(L->F, 128), L->D}, {ceil_div(L->D, 256), L->F}}, factored ? 3 : 7, factored ? 2 : 5)));
         f.ksplit = rows <= (size_t)kSplitTileM &&
                    qgemm_skinny_ksplit_ok(L->gate.view) && qgemm_skinny_ksplit_ok(L->up.view) && qgemm_skinny_ksplit_ok(L->down.view) &&
                    (!f.fold || (qgemm_skinny_ksplit_ok(L->sgate.view) && qgemm_skinny_ksplit_ok(L->sup.view) &&
@@ -978,7 +1004,7 @@ static int gather_qmm_view(uint16_t *d_out, const uint16_t *d_x, const QView &v,
     DMOE_REQUIRE(small || qgemm_mfma_supports(v) || gemm_bf16_supports(v), "gather_qmm: unsupported weight shape rows=%d cols=%d", v.rows, v.cols);
     int tile_m = small ? qgemm_skinny_tile_m(v) : qgemm_mfma_tile_m(v);
     if (small && ((size_t)pack_max_tiles((size_t)R, v.n_mats, kSplitTileM) * (size_t)ceil_div(v.rows, 256) <= (size_t)kSkinnyFewGroups ||
-                  (size_t)R <= inline_rows(v)))
+                  ((size_t)R <= inline_rows(v) && one_block_tiles_pay((size_t)R, v.n_mats, 0, 0, {{ceil_div(v.rows, 256), v.cols}}, 7, 5))))
         tile_m = std::min(tile_m, kSplitTileM); // see kSkinnyFewGroups
     const int max_tiles = pack_max_tiles((size_t)R, v.n_mats, tile_m);
     Bump b;
