@@ -86,8 +86,12 @@ struct SkinnyStage {
 constexpr int kSkinnySyncNone = 0, kSkinnySyncSignal = 1, kSkinnySyncWait = 2;
 
 // LDS: [activation window][sums of x per step][MBLK only: 4 KiB per wavefront for turning weight lines][zeros, where read]
-__host__ __device__ constexpr size_t skinny_turn_offset(int cols, int kstep) {
-    return (size_t)kSkinnyRowBlock * (size_t)cols * 2 + (size_t)kSkinnyTileM * 16 +
+// The window ends with 16 bytes per row of the largest tile. Kernels of single launches have tiles of one row block only, and keep the
+// order of their rows (kInlineRows words, static) in what that saves.
+constexpr size_t skinny_row_pads(bool one_block) { return (size_t)(one_block ? kSkinnyRowBlock : kSkinnyTileM) * 16; }
+static_assert(skinny_row_pads(true) + kInlineRows * sizeof(uint32_t) <= skinny_row_pads(false), "the order of the rows");
+__host__ __device__ constexpr size_t skinny_turn_offset(int cols, int kstep, bool one_block) {
+    return (size_t)kSkinnyRowBlock * (size_t)cols * 2 + skinny_row_pads(one_block) +
            (size_t)(cols / kstep) * kSkinnyRowBlock * sizeof(float) + 128;
 }
 constexpr size_t kSkinnyTurnBytes = (size_t)2 * kSkinnyWaves * 4 * 1024;
@@ -104,15 +108,17 @@ constexpr size_t kSkinnyStageOffset = 16384, kSkinnyStageBytes = (size_t)kSkinny
 // last step's sums: the 128 bytes in the offset. At least 32 KiB: once the main loop is done the wavefronts exchange their sums
 // through the start of the window (gate/up pairs: 4 KiB per row block of the tile, up to 16 KiB; split reduction: bytes 4096 ..
 // 8191) and gather the tile's outputs behind that (up to 32 rows of 256 columns), which a short reduction would not cover.
-constexpr size_t skinny_lds_bytes(int cols, int kstep, bool mblk, size_t zeros) {
-    const size_t window = skinny_turn_offset(cols, kstep) + (mblk ? 0 : zeros), least = kSkinnyStageOffset + kSkinnyStageBytes;
+constexpr size_t skinny_lds_bytes(int cols, int kstep, bool mblk, size_t zeros, bool one_block) {
+    const size_t window = skinny_turn_offset(cols, kstep, one_block) + (mblk ? 0 : zeros), least = kSkinnyStageOffset + kSkinnyStageBytes;
     return (window > least ? window : least) + (mblk ? kSkinnyTurnBytes + zeros : 0);
 }
 // A kernel without zeros pays nothing for them: reductions of 3072 in 8 bits leave LDS for three workgroups on a compute unit
 // (160 KiB, handed out in pieces of 1280 bytes) and those of 4768 for two.
 constexpr size_t skinny_lds_share(size_t bytes) { return (bytes + 1279) / 1280 * 1280; }
-static_assert(3 * skinny_lds_share(skinny_lds_bytes(3072, 32, false, 0)) <= 160 * 1024 &&
-              2 * skinny_lds_share(skinny_lds_bytes(4768, 32, false, 0)) <= 160 * 1024, "workgroups per compute unit");
+static_assert(3 * skinny_lds_share(skinny_lds_bytes(3072, 32, false, 0, false)) <= 160 * 1024 &&
+              2 * skinny_lds_share(skinny_lds_bytes(4768, 32, false, 0, false)) <= 160 * 1024 &&
+              2 * skinny_lds_share(skinny_lds_bytes(4768, 32, false, 0, true) + kInlineRows * sizeof(uint32_t)) <= 160 * 1024,
+              "workgroups per compute unit");
 // Registers for three workgroups, six wavefronts per SIMD, on the 8-bit launches that fill the chip (the compiler left to itself takes
 // 81, one too many). Whether the third one is wanted is the launch's choice: what keeps it out is LDS asked for and not used.
 template <typename Fmt, bool PACKED, bool KSPLIT, bool FEW>
@@ -291,7 +297,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     const int span_bytes = span_steps * KSTEP * 2;   // bytes of one row in one span
     const int pitch = span_bytes + 16;               // +16 keeps neighbouring rows on different banks
     uint8_t *xs_lds = skinny_lds;
-    float *gs_lds = (float *)(skinny_lds + kSkinnyRowBlock * cols * 2 + kSkinnyTileM * 16); // [span_steps][rp] sums of x
+    float *gs_lds = (float *)(skinny_lds + kSkinnyRowBlock * cols * 2 + (int)skinny_row_pads(KSPLIT || FEW)); // [span_steps][rp] sums of x
     const uint32_t lds_addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)skinny_lds;
     // source rows of the tile: one load for all of them (lane r holds row r's), then uniform reads
     uint32_t src_of_lane = __builtin_amdgcn_readfirstlane(t.row0) + (uint32_t)(lane < nrows ? lane : 0);
@@ -380,7 +386,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         }
     };
 
-    uint8_t *const zeros = skinny_lds + skinny_turn_offset(cols, KSTEP) + (MBLK ? kSkinnyTurnBytes : 0);
+    uint8_t *const zeros = skinny_lds + skinny_turn_offset(cols, KSTEP, KSPLIT || FEW) + (MBLK ? kSkinnyTurnBytes : 0);
     static_assert((size_t)ROUND * KSTEP * 2 <= skinny_zero_bytes(MBLK), "a round of zeros");
     if (ZEROS && tid * 16 < (int)skinny_zero_bytes(MBLK)) *(uint4 *)(zeros + tid * 16) = make_uint4(0, 0, 0, 0);
     SkinnyStage<NM> ring[STAGES];
@@ -526,7 +532,7 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
         };
 
         // GROUPED: ring stages j .. j+3 (one group as loaded) -> the chunks of its four steps in the operand layout
-        uint8_t *const turn_lds = skinny_lds + skinny_turn_offset(cols, KSTEP) + wave * (LG * 1024);
+        uint8_t *const turn_lds = skinny_lds + skinny_turn_offset(cols, KSTEP, KSPLIT || FEW) + wave * (LG * 1024);
         const uint8_t *const turn_rd = turn_lds + ln * 128;
         const int turn_sw = (ln >> 1) & 7;
         uint4 turned_raw[LG];
@@ -847,8 +853,8 @@ static int skinny_vals(const QView &b) {
     if (b.mode == DMOE_QUANT_NONE) return 8;
     return (b.mode == DMOE_QUANT_AFFINE && b.bits == 4) || b.mode == DMOE_QUANT_MXFP4 ? 32 : 16;
 }
-static size_t skinny_lds_bytes(const QView &b, bool mblk = false, size_t zeros = 0) {
-    return skinny_lds_bytes(b.cols, 2 * skinny_vals(b), mblk, zeros);
+static size_t skinny_lds_bytes(const QView &b, bool mblk = false, size_t zeros = 0, bool one_block = false) {
+    return skinny_lds_bytes(b.cols, 2 * skinny_vals(b), mblk, zeros, one_block);
 }
 
 // Rows per tile to build tile lists with for this weight shape: a tile of 2 (4) row blocks splits the reduction
@@ -952,7 +958,7 @@ struct SkinnyLaunch {
         }
         auto kern = qgemm_skinny_kernel<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>;
         constexpr size_t zeros = skinny_reads_zeros(FACTORED, KSPLIT, FEW && !IsLoose<Fmt>::value) ? skinny_zero_bytes(MBLK) : 0;
-        const size_t lds = skinny_lds_bytes(g.b0, MBLK, zeros);
+        const size_t lds = skinny_lds_bytes(g.b0, MBLK, zeros, KSPLIT || FEW);
         DMOE_TRY((skinny_raise_limit<Fmt, FACTORED, PACKED, MBLK, KSPLIT, FEW>())); // done by dmoe_init for its device; a flag test otherwise
         if constexpr (FEW && !FACTORED) {
             GemmArgs a = g;
