@@ -88,3 +88,15 @@ def test_eight_bit_launches_leave_registers_for_three_workgroups():
         assert get("vgpr_count") <= 512 // 6 // 8 * 8 and get("vgpr_spill_count") == 0 and get("private_segment_fixed_size") == 0
         seen += 1
     assert seen == 1
+
+
+@pytest.mark.skipif(shutil.which(os.environ.get("HIPCC", "hipcc")) is None, reason="needs hipcc")
+def test_checkpoint_layout_kernel_keeps_its_scalar_registers():
+    """The 4-bit kernels on the checkpoint's own arrays run out of scalar registers. What is spilled at their head is waited for load by
+    load (about 0.1 us each on calls of 20): no more of it than the 30 and 35 registers it was measured with."""
+    seen = {}
+    for entry in _device_asm("qgemm_skinny.hip").split("  - .agpr_count:")[1:]:
+        m = re.search(r"qgemm_skinny_kernelINS_10FmtAffine4ELb1ELb0ELb([01])ELb0ELb0EEE", entry)
+        if m:
+            seen[m.group(1)] = int(re.search(r"\.sgpr_spill_count:\s*(\d+)", entry).group(1))
+    assert set(seen) == {"0", "1"} and seen["1"] <= 30 and seen["0"] <= 35, seen
