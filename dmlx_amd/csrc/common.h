@@ -262,12 +262,12 @@ struct GemmArgs {
     const uint32_t *n_live = nullptr; // nullable: experts with rows, for the wide kernel's choice of a tile map
     int stream_weights = 0;           // wide kernel, set by its launcher: see kWideStreamBytes
     int dense_tiles = 0;              // of the tile list: the always-on expert's, which n_live does not count
-    // Weight-streaming kernel, factored 4-bit form (see skinny_factored). `a_sums` set: the rows of `a` are in code order (the
+    // Weight-streaming kernel, factored 4-bit form (see qgemm_skinny_factored). `a_sums` set: the rows of `a` are in code order (the
     // 16-byte piece x0..x7 as x0,x4,x1,x5,x2,x6,x3,x7), and a_sums[row][cols / 64] holds the sum of each 64 of their values.
     // `out_sums` set (gate/up role): the outputs leave in that form, the sums here.
     const float *a_sums = nullptr;
     float *out_sums = nullptr;
-    // Weight-streaming kernel, launches of a few workgroups (qgemm_skinny_takes_ids): instead of a tile list from a packing launch,
+    // Weight-streaming kernel, launches of a few rows (qgemm_skinny_takes_ids): instead of a tile list from a packing launch,
     // the expert ids of at most kInlineRows rows. Every workgroup orders them for itself, stably by expert, into tiles of at most
     // 8 rows; dense_rows further rows of matrix dense_expert are the tiles in front. max_tiles bounds the number of tiles.
     const uint32_t *ids = nullptr;

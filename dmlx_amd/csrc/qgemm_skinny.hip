@@ -174,8 +174,8 @@ __device__ __forceinline__ void skinny_tile(const GemmArgs &g, const Tile &t, ui
     // 8-bit 45.6 / 78.3 -> 44.7 / 69.9). Not where the launch fills the chip: there a wavefront's gathered loads are no loss (24 to
     // 64 tokens, 4-bit: pinned 0 to 2 % slower), and not on unquantized weights (32 instructions per round, level).
     constexpr bool PIN = (KSPLIT || FEW) && KV > 8 && !IsLoose<Fmt>::value;
-    // Eight wavefronts share one staging of the tile's activations. A compute unit fetches no more than 40 GB/s, however many
-    // loads its wavefronts have in flight, so a launch of a few workgroups is spread over more of them: workgroups of four or two
+    // Eight wavefronts share one staging of the tile's activations. A launch of a few workgroups leaves compute units idle that
+    // would fetch beside the others, so it is spread over more of them: workgroups of four or two
     // wavefronts as long as that makes at most kSkinnyFewGroups (us per step: small layer on MXFP4 25.5 -> 24.4, 4 tokens over 64
     // experts, 4-bit in groups of 32 37.2 -> 30.7). Not the factored form, whose re-ordering pass over LDS a workgroup's threads share
     // (small layer 33.1 -> 34.6).
@@ -794,8 +794,9 @@ __device__ __forceinline__ bool skinny_tile_of_ids(const GemmArgs &g, uint32_t s
 // y < a.max_tiles are the gate/up tiles, the next a.max_tiles the down tiles of the same list. The hardware starts
 // workgroups in index order, so every producer of a tile is running or done by the time a consumer of it starts to
 // wait; the down workgroups that become resident while the last gate/up workgroups drain stream their weights meanwhile.
-// FEW: a single launch of at most kSkinnyFewGroups workgroups and of tiles of one row block. It is paced by each workgroup's own
-// chain, not by bandwidth or power: the ring's loads are pinned (see PIN), no zeros, no copies for larger tiles.
+// FEW: a single launch of tiles of one row block only, no copies for larger tiles: of at most kSkinnyFewGroups workgroups, or of
+// any number that order a few rows by themselves (GemmArgs::ids). The former is paced by each workgroup's own chain, not by
+// bandwidth or power: the ring's loads are pinned (see PIN), no zeros. The latter is the same but for Loose (above).
 template <typename Fmt, bool FACTORED, bool PACKED, bool MBLK = false, bool KSPLIT = false, bool FEW = false>
 __global__ __launch_bounds__(2 * kSkinnyWaves * 64, (skinny_counts_groups<Fmt, PACKED, KSPLIT, FEW>() ? 6 : 1)) void qgemm_skinny_kernel(GemmArgs a, GemmArgs b, int paired) {
     extern __shared__ __attribute__((aligned(16))) uint8_t skinny_lds[];
